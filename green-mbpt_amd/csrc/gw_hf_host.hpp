@@ -120,7 +120,7 @@ void block_gemm(hipStream_t st, int n, int64_t nb, const double2* A, const doubl
   g.C = C; g.sCb = bs; g.sCm = ld; g.sCno = 0; g.sCni = 1;
   g.alpha = make_double2(alpha, 0.0);
   g.accumulate = acc ? 1 : 0;
-  zgemm_f64(g, true, false, st);
+  zgemm_f64(g, st);
 }
 }  // namespace
 
@@ -232,7 +232,7 @@ void gw_hip_kernel::hf_exchange_gemm(const double2* dm_s, int nblk) {
       y.B = orb_G_ + ro * nso + co; y.sBb = nso2; y.sBko = 0; y.sBki = nso; y.sBno = 0; y.sBni = 1;
       y.C = orb_W_; y.sCb = vq; y.sCm = nao; y.sCno = 0; y.sCni = 1;
       y.alpha = make_double2(1.0, 0.0);
-      zgemm_f64(y, true, false, stream_);
+      zgemm_f64(y, stream_);
       ZGemmArgs x{};
       x.M = (int)nao; x.N = (int)nao; x.K = (int)(NQ * nao); x.batch = (int)nk; x.kin = (int)nao; x.nin = (int)nao;
       x.A = orb_W_; x.sAb = vq; x.sAm = nao; x.sAko = nao2; x.sAki = 1;
@@ -240,7 +240,7 @@ void gw_hip_kernel::hf_exchange_gemm(const double2* dm_s, int nblk) {
       x.conjB = 1;
       x.C = hf_x_ + (bl * nk + q) * nk * nao2; x.sCb = nao2; x.sCm = nao; x.sCno = 0; x.sCni = 1;
       x.alpha = make_double2(1.0, 0.0);
-      zgemm_f64_splitk(x, ksplit, orb_part_, true, true, stream_);
+      zgemm_f64_splitk(x, ksplit, orb_part_, stream_);
     }
   }
 }

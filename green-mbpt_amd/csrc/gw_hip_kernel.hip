@@ -529,7 +529,8 @@ void gw_hip_kernel::p0_gemm(int64_t q, int64_t tc, double2* Pt0, int shape) {
   a.alpha = make_double2(-d_.prefactor / (double)nk, 0.0);
   a.accumulate = 0; a.conjA = 0; a.conjB = 1;
   a.upper = g_herm_ ? 1 : 0;
-  zgemm_f64(a, true, true, stream_, shape);
+  // partial products in the Dyson work buffer, which only stage_dyson uses
+  zgemm_f64_splitk(a, zgemm_auto_ksplit(a, qchunk_ * (int64_t)dyson_per_q()), Pw_, stream_, shape);
 }
 
 // R = P-tilde(t0 .. t0+tc) conj(V) into scratch_, FP64 (tile `shape`): Pt0 = P-tilde at t0
@@ -545,7 +546,7 @@ void gw_hip_kernel::sigma_gemm(const double2* Pt0, const double2* Vb, int64_t nk
   a.C = scratch_; a.sCb = nkb * NQ * nao2; a.sCm = nao2; a.sCno = NQ * nao2; a.sCni = 1;
   a.alpha = make_double2(1.0, 0.0);
   a.accumulate = 0; a.conjA = 0; a.conjB = 1;
-  zgemm_f64(a, true, false, stream_, shape);
+  zgemm_f64(a, stream_, shape);
 }
 
 // Split precision, P0: int8 slices of Z (rows (tau, Q), chunks k) into Zs_.
@@ -701,7 +702,7 @@ void gw_hip_kernel::block_inverse(double2* X, int64_t nmat) {
         a.B = P; a.sBb = sP; a.sBko = 0; a.sBki = n; a.sBno = 0; a.sBni = 1;
         a.C = Q; a.sCb = sP; a.sCm = n; a.sCno = 0; a.sCni = 1;
         a.alpha = make_double2(1.0, 0.0);
-        zgemm_f64(a, true, false, stream_);
+        zgemm_f64(a, stream_);
       }
       if (J0 > 0) {
         hipLaunchKernelGGL(hgj_negate_kernel, dim3((unsigned)ceil_div((int64_t)jb * J0, 256), (unsigned)mb), dim3(256),
@@ -717,7 +718,7 @@ void gw_hip_kernel::block_inverse(double2* X, int64_t nmat) {
         a.alpha = make_double2(-1.0, 0.0);
         a.accumulate = 1;
         a.upper = 1;
-        zgemm_f64(a, false, false, stream_);
+        zgemm_f64(a, stream_);
       }
       if (J0 > 0) {  // A[i][J] = -P^H D^-1 for the swept rows i < J0 (the rows below are not kept)
         ZGemmArgs a{};
@@ -726,7 +727,7 @@ void gw_hip_kernel::block_inverse(double2* X, int64_t nmat) {
         a.B = D; a.sBb = sD; a.sBko = 0; a.sBki = jb; a.sBno = 0; a.sBni = 1;
         a.C = A + J0; a.sCb = n2; a.sCm = n; a.sCno = 0; a.sCni = 1;
         a.alpha = make_double2(-1.0, 0.0);
-        zgemm_f64(a, false, false, stream_);
+        zgemm_f64(a, stream_);
       }
       hipLaunchKernelGGL(hgj_rows_kernel, dim3((unsigned)ceil_div((int64_t)jb * (n - J0), 256), (unsigned)mb), dim3(256),
                          0, stream_, A, (int)n, n2, J0, jb, Q, sP, D, sD);
@@ -760,7 +761,7 @@ void gw_hip_kernel::stage_dyson(int64_t nq, const int* q0_row) {
       a.B = P_ + q0 * nts * NQ2; a.sBb = nts * NQ2; a.sBko = 0; a.sBki = NQ2; a.sBno = 0; a.sBni = 1;
       a.C = W0; a.sCb = nwb * NQ2; a.sCm = NQ2; a.sCno = 0; a.sCni = 1;
       a.alpha = make_double2(1.0, 0.0);
-      zgemm_f64(a, true, false, stream_);
+      zgemm_f64(a, stream_);
     }
     mark(e1);
     const int64_t nmat = qc * nwb;
@@ -780,7 +781,7 @@ void gw_hip_kernel::stage_dyson(int64_t nq, const int* q0_row) {
       a.C = W2; a.sCb = NQ2; a.sCm = NQ; a.sCno = 0; a.sCni = 1;
       a.alpha = make_double2(1.0, 0.0);
       a.upper = 1;
-      zgemm_f64(a, true, false, stream_);
+      zgemm_f64(a, stream_);
     }
     mirror_upper(W2, (int)NQ, NQ2, nmat, stream_);
     GWHIP_CHECK(hipGetLastError());
@@ -797,7 +798,7 @@ void gw_hip_kernel::stage_dyson(int64_t nq, const int* q0_row) {
       a.B = W2; a.sBb = nwb * NQ2; a.sBko = 0; a.sBki = NQ2; a.sBno = 0; a.sBni = 1;
       a.C = P_ + q0 * nts * NQ2; a.sCb = nts * NQ2; a.sCm = NQ2; a.sCno = 0; a.sCni = 1;
       a.alpha = make_double2(1.0, 0.0);
-      zgemm_f64(a, true, false, stream_);
+      zgemm_f64(a, stream_);
     }
     mark(e3);
     if (timing_) {
@@ -993,7 +994,7 @@ void gw_hip_kernel::p0_prep_gemm(int64_t q, const double2* G, int64_t t0, int64_
       w.B = orb_G_ + a * nao * nso + b * nao; w.sBb = nso2; w.sBko = 0; w.sBki = nso; w.sBno = 0; w.sBni = 1;
       w.C = orb_W_; w.sCb = vq; w.sCm = nao; w.sCno = 0; w.sCni = 1;
       w.alpha = make_double2(1.0, 0.0);
-      zgemm_f64(w, true, false, stream_);
+      zgemm_f64(w, stream_);
       ZGemmArgs z{};
       z.M = (int)nao; z.N = (int)(NQ * nao); z.K = (int)nao; z.batch = (int)nk; z.kin = (int)nao; z.nin = (int)nao;
       z.A = G + (tt * d_.ns + is) * nk * nso2 + b * nao * nso + a * nao; z.sAb = nso2; z.sAm = nso; z.sAko = 0;
@@ -1002,7 +1003,7 @@ void gw_hip_kernel::p0_prep_gemm(int64_t q, const double2* G, int64_t t0, int64_
       z.C = scratch_ + t * nk * vq; z.sCb = vq; z.sCm = nao; z.sCno = nao2; z.sCni = 1;
       z.alpha = make_double2(1.0, 0.0);
       z.accumulate = s > 0 ? 1 : 0;
-      zgemm_f64(z, true, false, stream_);
+      zgemm_f64(z, stream_);
     }
   }
 }
@@ -1029,7 +1030,7 @@ void gw_hip_kernel::sigma_epi_gemm(const double2* G, double2* Sigma, const doubl
         x.B = Vb; x.sBb = vq; x.sBko = 0; x.sBki = 1; x.sBno = nao2; x.sBni = nao;
         x.C = orb_W_; x.sCb = vq; x.sCm = nao; x.sCno = nao2; x.sCni = 1;
         x.alpha = make_double2(1.0, 0.0);
-        zgemm_f64(x, false, false, stream_);
+        zgemm_f64(x, stream_);
         ZGemmArgs y{};
         y.M = (int)nao; y.N = (int)nao; y.K = (int)(NQ * nao); y.batch = (int)nkb; y.kin = (int)nao;
         y.nin = (int)nao;
@@ -1042,7 +1043,7 @@ void gw_hip_kernel::sigma_epi_gemm(const double2* G, double2* Sigma, const doubl
         // only nkb x (nao / 64)^2 output tiles, each over K = NQ nao: cut K so that ~1024 blocks run
         const int64_t tiles = nkb * ceil_div(nao, 64) * ceil_div(nao, 64);
         const int ksplit = (int)std::min<int64_t>(kOrbKsplit, std::max<int64_t>(1, ceil_div(1024, tiles)));
-        zgemm_f64_splitk(y, ksplit, orb_part_, false, false, stream_);
+        zgemm_f64_splitk(y, ksplit, orb_part_, stream_);
       }
     }
 }
@@ -1465,7 +1466,7 @@ void debug_zgemm(int M, int N, int K, const double2* A, const double2* B, double
   a.C = dC; a.sCm = N; a.sCni = 1;
   a.alpha = make_double2(1.0, 0.0);
   a.conjA = conjA; a.conjB = conjB;
-  zgemm_f64(a, true, false, nullptr, shape);
+  zgemm_f64(a, nullptr, shape);
   GWHIP_CHECK(hipDeviceSynchronize());
   GWHIP_CHECK(hipMemcpy(C, dC, (size_t)M * N * sizeof(double2), hipMemcpyDeviceToHost));
   (void)hipFree(dA);

@@ -261,7 +261,7 @@ const double2* gw_hip_kernel::star_rotate(int64_t iq, int64_t q) {
   a.C = T; a.sCb = NQ2; a.sCm = NQ; a.sCno = 0; a.sCni = 1;
   a.alpha = make_double2(1.0, 0.0);
   a.conjA = tr; a.conjB = tr;
-  zgemm_f64(a, true, false, stream_);
+  zgemm_f64(a, stream_);
   ZGemmArgs b{};
   b.M = (int)NQ; b.N = (int)NQ; b.K = (int)NQ; b.batch = (int)half; b.kin = (int)NQ; b.nin = (int)NQ;
   b.A = T; b.sAb = NQ2; b.sAm = NQ; b.sAko = 0; b.sAki = 1;
@@ -269,7 +269,7 @@ const double2* gw_hip_kernel::star_rotate(int64_t iq, int64_t q) {
   b.C = out; b.sCb = NQ2; b.sCm = NQ; b.sCno = 0; b.sCni = 1;
   b.alpha = make_double2(1.0, 0.0);
   b.conjB = tr ? 0 : 1;
-  zgemm_f64(b, true, true, stream_);
+  zgemm_f64(b, stream_);
   return out;
 }
 

@@ -69,7 +69,7 @@ void mat_gemm(hipStream_t st, int n, int64_t batch, const double2* A, bool tA, b
   g.accumulate = acc ? 1 : 0;
   g.conjA = cA ? 1 : 0;
   g.conjB = cB ? 1 : 0;
-  zgemm_f64(g, !tA, tB, st);
+  zgemm_f64(g, st);
 }
 
 // C[m] = sum_j op(T)[m][j] X[j] over stacks of NQ^2 matrices; T is rows x cols (row-major).
@@ -84,7 +84,7 @@ void stack_transform(hipStream_t st, const double2* T, int rows, int cols, bool 
   g.C = C; g.sCm = NQ2; g.sCno = 0; g.sCni = 1;
   g.alpha = make_double2(1.0, 0.0);
   g.conjA = trans ? 1 : 0;
-  zgemm_f64(g, !trans, false, st);
+  zgemm_f64(g, st);
 }
 
 }  // namespace
@@ -124,14 +124,14 @@ void gw_hip_kernel::vjp_sandwich(bool has_l, bool has_r, int NB, dim3 grid, cons
       g.B = V.p + tz * V.s_t; g.sBb = V.s_k; g.sBko = 0; g.sBki = V.rs; g.sBno = V.s_q; g.sBni = V.cs;
       g.conjB = V.conj;
       g.C = X.p + tz * X.s_t; g.sCb = X.s_k; g.sCm = X.rs; g.sCno = X.s_q; g.sCni = X.cs;
-      zgemm_f64(g, true, false, stream_);
+      zgemm_f64(g, stream_);
     } else {      // X[k]((Q, r), c) = sum_c' V_Q(r, c') R[k](c', c)
       g.M = (int)(NQ * nao); g.N = (int)nao;
       g.A = V.p + tz * V.s_t; g.sAb = V.s_k; g.sAm = V.rs; g.sAko = 0; g.sAki = V.cs;
       g.conjA = V.conj;
       g.B = orb_G_; g.sBb = nao2; g.sBko = 0; g.sBki = nao; g.sBno = 0; g.sBni = 1;
       g.C = X.p + tz * X.s_t; g.sCb = X.s_k; g.sCm = X.rs; g.sCno = 0; g.sCni = X.cs;
-      zgemm_f64(g, V.cs == 1, false, stream_);
+      zgemm_f64(g, stream_);
     }
   }
 }
@@ -164,7 +164,7 @@ void gw_hip_kernel::vjp_reduce(bool has_m, int NB, dim3 grid, const OrbArgs& a, 
       z.conjB = C.conj;
       z.C = orb_W_; z.sCb = vq; z.sCm = nao; z.sCno = nao2; z.sCni = 1;
       z.alpha = make_double2(1.0, 0.0);
-      zgemm_f64(z, true, false, stream_);
+      zgemm_f64(z, stream_);
       cp = orb_W_; c_sk = vq; c_sq = nao2; c_rs = nao; c_cs = 1; c_conj = 0;
     }
     ZGemmArgs y{};  // orb_O_[k](i, j) = sum_{Q, m} A_Q(i, m) Z'_Q(m, j)
@@ -175,7 +175,7 @@ void gw_hip_kernel::vjp_reduce(bool has_m, int NB, dim3 grid, const OrbArgs& a, 
     y.conjB = c_conj;
     y.C = orb_O_; y.sCb = nao2; y.sCm = nao; y.sCno = 0; y.sCni = 1;
     y.alpha = make_double2(1.0, 0.0);
-    zgemm_f64_splitk(y, ksplit, orb_part_, A.cs == 1, c_rs == 1, stream_);
+    zgemm_f64_splitk(y, ksplit, orb_part_, stream_);
     hipLaunchKernelGGL(orb_scatter_add_kernel, dim3((unsigned)ceil_div(nao2, 256), (unsigned)nk), dim3(256), 0, stream_,
                        a, O, tz, orb_O_);
     GWHIP_CHECK(hipGetLastError());
@@ -312,7 +312,7 @@ void gw_hip_kernel::vjp_device(const double2* G, const double2* Sbar, double2* G
           g.C = scratch_; g.sCb = per_t; g.sCm = nao2; g.sCno = NQ * nao2; g.sCni = 1;
           g.alpha = make_double2(1.0, 0.0);
           g.conjA = 1;
-          zgemm_f64(g, true, false, stream_);
+          zgemm_f64(g, stream_);
         }
         {  // Gbar(tau, k - q)_s += c sum_Q V_Q^H Y_Q
           OrbArgs oc = oa;
@@ -335,7 +335,7 @@ void gw_hip_kernel::vjp_device(const double2* G, const double2* Sbar, double2* G
           g.alpha = make_double2(c, 0.0);
           g.accumulate = 1;
           g.conjA = 1;
-          zgemm_f64(g, true, true, stream_);
+          zgemm_f64_splitk(g, zgemm_auto_ksplit(g, qchunk_ * (int64_t)dyson_per_q()), Pw_, stream_);
         }
       }
     }
@@ -364,7 +364,7 @@ void gw_hip_kernel::vjp_device(const double2* G, const double2* Sbar, double2* G
         g.B = Vp; g.sBb = 0; g.sBko = 0; g.sBki = nao2; g.sBno = NQ * nao2; g.sBni = 1;
         g.C = vW_; g.sCb = per_t; g.sCm = nao2; g.sCno = NQ * nao2; g.sCni = 1;
         g.alpha = make_double2(alpha, 0.0);
-        zgemm_f64(g, true, false, stream_);
+        zgemm_f64(g, stream_);
       }
       const OrbOp Zb{vW_, per_t, NQ * nao2, nao2, nao, 1, 0, 0};
       for (int s = 0; s < d_.pseudo_ns; ++s) {

@@ -281,11 +281,11 @@ double debug_gemm_bench(int which, int NQ, int nk, int nao, int batch, int shape
   a.A = dA; a.B = dB; a.C = dC;
   a.alpha = make_double2(1.0, 0.0);
   a.conjB = 1;
-  zgemm_f64(a, akc, bkc, nullptr, shape);
+  zgemm_f64(a, nullptr, shape);
   GWHIP_CHECK(hipDeviceSynchronize());
   Event e0, e1;
   GWHIP_CHECK(hipEventRecord(e0, nullptr));
-  for (int r = 0; r < reps; ++r) zgemm_f64(a, akc, bkc, nullptr, shape);
+  for (int r = 0; r < reps; ++r) zgemm_f64(a, nullptr, shape);
   GWHIP_CHECK(hipEventRecord(e1, nullptr));
   GWHIP_CHECK(hipEventSynchronize(e1));
   float ms = 0.f;
