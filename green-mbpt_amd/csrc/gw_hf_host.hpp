@@ -153,19 +153,19 @@ void gw_hip_kernel::hf_device(const double2* dm, const double2* S, double madelu
   hipLaunchKernelGGL(hf_direct_add_kernel, dim3((unsigned)ceil_div(nmat * nao2, 256)), dim3(256), 0, stream_, hf_work_, Vd,
                      F, (int)nk, (int)NQ, (int)nao, (int)nso, (int)nspin, x2c ? 1 : 0);
   GWHIP_CHECK(hipGetLastError());
+  // a density matrix that is Hermitian to rounding makes the aa and bb exchange blocks Hermitian
+  hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(64), 0, stream_, reinterpret_cast<int*>(hcheck_), (int64_t)4);
+  hipLaunchKernelGGL(herm_check_kernel, dim3(herm_check_blocks(nmat * nso2)), dim3(256), 0, stream_, dm, nmat, (int)nso,
+                     hcheck_);
+  hipLaunchKernelGGL(herm_flag_kernel, dim3(1), dim3(1), 0, stream_, hcheck_, 1e-15, hf_herm_);
+  GWHIP_CHECK(hipGetLastError());
   // exchange: X[blk][q][k] = sum_Q V(k, k+q)_Q dm(k+q)_blk V(k, k+q)_Q^H for all (k, q) in one
   // launch per spin block, then F(k)_blk -= pref/nk sum_q X[blk][q][k] (fixed order in q)
-  const int NB = (int)ceil_div(nao, 16);
   const int nblk = x2c ? 3 : 1;
   if (!hf_x_) hf_x_ = dalloc<double2>((size_t)nblk * nk * nk * nao2);
   Event ex0, ex1;
   float ex_ms = 0.f;
-  const OrbOp A{Vq_, nk * NQ * nao2, NQ * nao2, nao2, nao, 1, 0, 0};  // V(k, k+q)_Q (i, a)
-  const OrbOp C{Vq_, nk * NQ * nao2, NQ * nao2, nao2, 1, nao, 0, 1};  // V(k, k+q)_Q^H (b, j)
-  OrbArgs oa{(int)nao, (int)NQ, (int)nk, 4, kplus_tab_, kminus_tab_, 1.0};
-  oa.kmap_st = nk;
   for (int64_t s = 0; s < nspin; ++s) {
-    zero(hf_x_, nblk * nk * nk * nao2);
     if (orb_gemm()) {
       GWHIP_CHECK(hipEventRecord(ex0, stream_));
       hf_exchange_gemm(dm + s * nk * nso2, nblk);
@@ -177,10 +177,18 @@ void gw_hip_kernel::hf_device(const double2* dm, const double2* S, double madelu
     }
     for (int bl = 0; bl < nblk && !orb_gemm(); ++bl) {
       const int64_t ro = (bl == 1) ? nao : 0, co = (bl == 0) ? 0 : nao;  // aa, bb, ab
-      const OrbOp M{dm + s * nk * nso2 + ro * nso + co, 0, nso2, 0, nso, 1, 1, 0};
-      const OrbOut O{hf_x_ + bl * nk * nk * nao2, nk * nao2, nao2, 0, nao, 1, 0};
+      HfExchangeArgs a{};
+      a.nao = (int)nao; a.nso = (int)nso; a.nk = (int)nk; a.NQ = (int)NQ;
+      a.dm = dm + s * nk * nso2 + ro * nso + co;
+      a.V = Vq_; a.X = hf_x_ + bl * nk * nk * nao2;
+      a.kplus = kplus_tab_; a.adj = adj_x_dev_;
+      a.herm = bl == 2 ? nullptr : hf_herm_;
       GWHIP_CHECK(hipEventRecord(ex0, stream_));
-      launch_reduce<true>(NB, dim3((unsigned)nk, (unsigned)nk), stream_, oa, A, M, C, O);
+      orb_dispatch([&](auto nb) {
+        constexpr int NB4 = decltype(nb)::value;
+        const dim3 g((unsigned)nk, 1, (unsigned)nk * HfReduce<NB4>::GROUPS);
+        launch_orb(hf_exchange_kernel<NB4>, a, g, HfReduce<NB4>::NT, HfReduce<NB4>::lds_bytes(), stream_);
+      });
       GWHIP_CHECK(hipEventRecord(ex1, stream_));
       GWHIP_CHECK(hipEventSynchronize(ex1));
       float m = 0.f;

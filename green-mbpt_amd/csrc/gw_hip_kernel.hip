@@ -96,6 +96,8 @@ gw_hip_kernel::gw_hip_kernel(const Dims& d, int device, hipStream_t shared_strea
   Ttb_ = dalloc<double2>((size_t)d_.nts * d_.nw_b);
   kplus_tab_ = dalloc<int>((size_t)nk * nk);
   kminus_tab_ = dalloc<int>((size_t)nk * nk);
+  adj_x_dev_ = dalloc<int>((size_t)nk);
+  hf_herm_ = dalloc<int>(1);
   flag_ = dalloc<int>(1);
   dyson_flag_ = dalloc<int>(1);
   GWHIP_CHECK(hipMemset(dyson_flag_, 0, sizeof(int)));
@@ -127,7 +129,7 @@ gw_hip_kernel::~gw_hip_kernel() {
                   (void*)kplus_tab_, (void*)kminus_tab_, (void*)flag_, (void*)dyson_flag_, (void*)leak_P0_, (void*)hcheck_, (void*)hf_work_, (void*)hf_x_, (void*)ksym_idx_, (void*)ksym_U_, (void*)hf_sym_, (void*)q0_qiq_, (void*)q0_A_, (void*)q0_eps_dev_,
                   (void*)q0_S_, (void*)q0_tmp_, (void*)q0_epst_, (void*)qsym_U_, (void*)star_P_, (void*)star_V_,
                   (void*)star_Vs_, (void*)star_eVs_, (void*)star_km_, (void*)star_q0row_, (void*)orb_W_,
-                  (void*)orb_G_, (void*)orb_part_, (void*)orb_O_, (void*)epi_part_})
+                  (void*)orb_G_, (void*)orb_part_, (void*)orb_O_, (void*)epi_part_, (void*)adj_x_dev_, (void*)hf_herm_})
     if (p) (void)hipFree(p);
   if (own_ws_)
     for (void* p : {(void*)Pw_, (void*)scratch_})
@@ -166,6 +168,24 @@ void gw_hip_kernel::upload_maps(const std::vector<int>& kpq, const std::vector<i
         neg_q_[q] = qp;
   for (int q = 0; q < nk; ++q)
     if (neg_q_[q] < 0) throw status_error(GWHIP_ERR_ARG, "k - q map has no matching k + q' row");
+  // V(k1, k2) = V(k2, k1)^H exactly for k1 != k2 (the expansion stores one and its adjoint), so a q whose
+  // pairs reverse onto the other table without a point paired with itself may read either
+  adj_s_.assign(nk, 0);
+  std::vector<int> adj_x((size_t)nk, 0);
+  std::vector<int> p_adj(nk, 0);
+  for (int q = 0; q < nk; ++q) {
+    bool s_ok = true, p_ok = true;
+    for (int k = 0; k < nk; ++k) {
+      const int m = kmq[(size_t)q * nk + k], p = kpq[(size_t)q * nk + k];
+      s_ok = s_ok && m != k && kpq[(size_t)q * nk + m] == k;
+      p_ok = p_ok && p != k && kpq[(size_t)neg_q_[q] * nk + p] == k;
+    }
+    adj_s_[q] = s_ok ? 1 : 0;
+    p_adj[q] = p_ok ? 1 : 0;
+  }
+  for (int q = 0; q < nk; ++q)  // closed under q -> -q, so that every ordered pair still occurs once
+    adj_x[q] = neg_q_[neg_q_[q]] == q && p_adj[q] && p_adj[neg_q_[q]];
+  GWHIP_CHECK(hipMemcpy(adj_x_dev_, adj_x.data(), (size_t)nk * sizeof(int), hipMemcpyHostToDevice));
   kplus_host_.assign((size_t)nk * nk, 0);  // [k][q] for the V expansion
   for (int q = 0; q < nk; ++q)
     for (int k = 0; k < nk; ++k) kplus_host_[(size_t)k * nk + q] = kpq[(size_t)q * nk + k];
@@ -198,6 +218,30 @@ void gw_hip_kernel::set_grid(const double2* T_bt, const double2* T_tb) {
   GWHIP_CHECK(hipMemcpy(Tbt_fold_, fold.data(), fold.size() * sizeof(double2), hipMemcpyHostToDevice));
   GWHIP_CHECK(hipMemcpy(Ttb_, T_tb, (size_t)nts * nwb * sizeof(double2), hipMemcpyHostToDevice));
   Ttb_host_.assign(T_tb, T_tb + (size_t)nts * nwb);
+  // P-tilde(tau) = sum_n T_tb[tau][n] P-tilde(i Omega_n) is Hermitian when, over each set of frequencies
+  // with the same row of T' (hence the same P0 and P-tilde: +-Omega), the imaginary parts of T_tb cancel
+  grid_herm_ = true;
+  double fmax_ = 0.0, tmax = 0.0;
+  for (const double2& v : fold) fmax_ = std::max(fmax_, std::max(std::fabs(v.x), std::fabs(v.y)));
+  for (int64_t i = 0; i < nts * nwb; ++i) tmax = std::max(tmax, std::max(std::fabs(T_tb[i].x), std::fabs(T_tb[i].y)));
+  std::vector<char> done((size_t)nwb, 0);
+  for (int64_t n = 0; n < nwb; ++n) {
+    if (done[n]) continue;
+    std::vector<double> im((size_t)nts, 0.0);
+    for (int64_t m = n; m < nwb; ++m) {
+      bool same = !done[m];
+      for (int64_t t = 0; t < half && same; ++t)
+        same = std::fabs(fold[n * half + t].x - fold[m * half + t].x) <= 1e-12 * fmax_ &&
+               std::fabs(fold[m * half + t].y) <= 1e-12 * fmax_;
+      if (!same) {
+        if (m == n) grid_herm_ = false;
+        continue;
+      }
+      done[m] = 1;
+      for (int64_t t = 0; t < nts; ++t) im[t] += T_tb[t * nwb + m].y;
+    }
+    for (double x : im) grid_herm_ = grid_herm_ && std::fabs(x) <= 1e-11 * tmax;
+  }
   grid_set_ = true;
   stored_valid_ = false;
 }
@@ -290,7 +334,8 @@ bool gw_hip_kernel::detect_hermitian_G(const double2* G) {
   GWHIP_CHECK(hipSetDevice(device_));
   hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(64), 0, stream_, reinterpret_cast<int*>(hcheck_), (int64_t)4);
   const int64_t nmat = d_.nts * d_.ns * d_.nk;
-  hipLaunchKernelGGL(herm_check_kernel, dim3(1024), dim3(256), 0, stream_, G, nmat, (int)d_.nso, hcheck_);
+  hipLaunchKernelGGL(herm_check_kernel, dim3(herm_check_blocks(nmat * d_.nso * d_.nso)), dim3(256), 0, stream_, G, nmat,
+                     (int)d_.nso, hcheck_);
   GWHIP_CHECK(hipGetLastError());
   unsigned long long v[2] = {0, 0};
   GWHIP_CHECK(hipMemcpyAsync(v, hcheck_, sizeof(v), hipMemcpyDeviceToHost, stream_));
@@ -347,13 +392,20 @@ void gw_hip_kernel::ensure_slices() {
     a.conj = 1; a.dst = Vs_p0_; a.exps = eVs_p0_;
     slice_rows(a, ns, stream_);
   }
-  {  // Sigma operand: rows (q, k, (n, j)) = V^Q'_jn(k, k+q) (per-Q transposed in place), elements Q'
+  {  // Sigma operand: rows (q, p, (n, j)) of conj(V^Q'_jn(k, k - q)) = V^Q'_nj(k - q, k), elements Q'
     SliceArgs a{};
-    a.src = Vq_; a.nrows = nk * nk * nao2; a.row_div = nao2; a.s_rhi = NQ * nao2;
-    a.row_div2 = d_.nao; a.s_rlo = 1; a.s_rlo2 = d_.nao;
+    a.src = Vq_; a.nrows = nk * nk * nao2; a.row_div = nao2; a.s_rhi = NQ * nao2; a.s_rlo = 1;
     a.nchunk = 1; a.s_c = 0; a.klen = (int)NQ; a.s_k = nao2; a.kc = (int)kc_s_;
-    a.conj = 1; a.dst = Vs_s_; a.exps = eVs_s_;
+    a.conj = 0; a.dst = Vs_s_; a.exps = eVs_s_;
     slice_rows(a, ns, stream_);
+    for (int64_t q = 0; q < nk; ++q) {
+      if (adj_s_[q]) continue;  // this q's rows hold V(k, k - q): per-Q transposed and conjugated
+      SliceArgs b = a;
+      b.src = sigma_rows(q).V; b.nrows = nk * nao2;
+      b.row_div2 = d_.nao; b.s_rlo = 1; b.s_rlo2 = d_.nao;
+      b.conj = 1; b.dst = Vs_s_ + q * nk * nao2 * OZ_PLANES * ns * kc_s_; b.exps = eVs_s_ + q * nk * nao2;
+      slice_rows(b, ns, stream_);
+    }
   }
   GWHIP_CHECK(hipStreamSynchronize(stream_));
   slices_ns_ = ns;
@@ -420,60 +472,41 @@ void gw_hip_kernel::resolve_timings() {
   pending_.clear();
 }
 
+// f(std::integral_constant<int, NB4>) for the number of 4-wide orbital blocks.  Every size to 40, then
+// every second one (a register-bound kernel gains less from the finer step than it costs to build).
+template <typename F>
+void gw_hip_kernel::orb_dispatch(F&& f) const {
+  switch ((int)ceil_div(d_.nao, 4)) {
+    case 1: return f(std::integral_constant<int, 1>{});
+    case 2: return f(std::integral_constant<int, 2>{});
+    case 3: return f(std::integral_constant<int, 3>{});
+    case 4: return f(std::integral_constant<int, 4>{});
+    case 5: return f(std::integral_constant<int, 5>{});
+    case 6: return f(std::integral_constant<int, 6>{});
+    case 7: return f(std::integral_constant<int, 7>{});
+    case 8: return f(std::integral_constant<int, 8>{});
+    case 9: return f(std::integral_constant<int, 9>{});
+    case 10: return f(std::integral_constant<int, 10>{});
+    case 11: case 12: return f(std::integral_constant<int, 12>{});
+    case 13: case 14: return f(std::integral_constant<int, 14>{});
+    case 15: case 16: return f(std::integral_constant<int, 16>{});
+    default: throw status_error(GWHIP_ERR_UNSUPPORTED, "orbital kernels: nao out of range");
+  }
+}
+
 namespace {
-template <int NB, typename T>
-void launch_z_prep_t(dim3 grid, size_t lds, hipStream_t st, const DevDims& dd, const double2* G, const double2* Vt,
-                     double2* Z, const int* kplus, int t0, int QPW) {
-  allow_lds(z_prep_mfma_kernel<NB, T>, lds);
-  const XcdGrid xg = make_xcd_grid(grid);
-  hipLaunchKernelGGL((z_prep_mfma_kernel<NB, T>), xcd_launch_grid(xg), dim3(256), lds, st, xg, dd, G, Vt, Z, kplus, t0,
-                     QPW);
+template <typename K, typename A>
+void launch_orb(K kern, A& args, dim3 grid, int threads, size_t lds, hipStream_t st) {
+  allow_lds(kern, lds);
+  args.xg = make_xcd_grid(grid, threads);
+  hipLaunchKernelGGL(kern, xcd_launch_grid(args.xg), dim3(threads), lds, st, args);
   GWHIP_CHECK(hipGetLastError());
 }
-// The orbital-size products stay FP64 in both precision modes: FP32 matrix cores here put the
-// Sigma error at ~2.4e-8 relative on the nk = 8, nao = 8, naux = 40 case, above the 1e-8 bar.
-template <int NB>
-void launch_z_prep(dim3 grid, size_t lds, hipStream_t st, const DevDims& dd, const double2* G, const double2* Vt,
-                   double2* Z, const int* kplus, int t0, int QPW) {
-  launch_z_prep_t<NB, double>(grid, lds, st, dd, G, Vt, Z, kplus, t0, QPW);
-}
-template <int NB, int NS, int SB>
-void launch_z_prep_slice_t(dim3 grid, size_t lds, hipStream_t st, const DevDims& dd, const double2* G, const double2* Vt,
-                           int8_t* dst, int* exps, int kc, const int* kplus, int t0, int QPW) {
-  allow_lds(z_prep_slice_kernel<NB, NS, SB>, lds);
-  const XcdGrid xg = make_xcd_grid(grid);
-  hipLaunchKernelGGL((z_prep_slice_kernel<NB, NS, SB>), xcd_launch_grid(xg), dim3(256), lds, st, xg, dd, G, Vt, dst,
-                     exps, kc, kplus, t0, QPW);
-  GWHIP_CHECK(hipGetLastError());
-}
-template <int NB, int SB>
-void launch_z_prep_slice_s(int ns, dim3 grid, size_t lds, hipStream_t st, const DevDims& dd, const double2* G,
-                           const double2* Vt, int8_t* dst, int* exps, int kc, const int* kplus, int t0, int QPW) {
-  if (ns == 5) launch_z_prep_slice_t<NB, 5, SB>(grid, lds, st, dd, G, Vt, dst, exps, kc, kplus, t0, QPW);
-  else if (ns == 4) launch_z_prep_slice_t<NB, 4, SB>(grid, lds, st, dd, G, Vt, dst, exps, kc, kplus, t0, QPW);
-  else launch_z_prep_slice_t<NB, 3, SB>(grid, lds, st, dd, G, Vt, dst, exps, kc, kplus, t0, QPW);
-}
-template <int NB>
-void launch_z_prep_slice(int ns, dim3 grid, size_t lds, hipStream_t st, const DevDims& dd, const double2* G,
-                         const double2* Vt, int8_t* dst, int* exps, int kc, const int* kplus, int t0, int QPW) {
-  if (dd.pseudo_ns == 2) launch_z_prep_slice_s<NB, 2>(ns, grid, lds, st, dd, G, Vt, dst, exps, kc, kplus, t0, QPW);
-  else launch_z_prep_slice_s<NB, 1>(ns, grid, lds, st, dd, G, Vt, dst, exps, kc, kplus, t0, QPW);
-}
-template <int NB, typename T>
-void launch_sigma_epi_t(dim3 grid, size_t lds, hipStream_t st, const DevDims& dd, const double2* G, const double2* Vt,
-                        const double2* R, double2* S, const int* kminus, int nks, int t0, double scale, int upper,
-                        int mirror, double2* part) {
-  allow_lds(sigma_epi_mfma_kernel<NB, T>, lds);
-  const XcdGrid xg = make_xcd_grid(grid);
-  hipLaunchKernelGGL((sigma_epi_mfma_kernel<NB, T>), xcd_launch_grid(xg), dim3(256), lds, st, xg, dd, G, Vt, R, S,
-                     kminus, nks, t0, scale, upper, mirror, (int)grid.y, part);
-  GWHIP_CHECK(hipGetLastError());
-}
-template <int NB>
-void launch_sigma_epi(dim3 grid, size_t lds, hipStream_t st, const DevDims& dd, const double2* G,
-                      const double2* Vt, const double2* R, double2* S, const int* kminus, int nks, int t0,
-                      double scale, int upper, int mirror, double2* part) {
-  launch_sigma_epi_t<NB, double>(grid, lds, st, dd, G, Vt, R, S, kminus, nks, t0, scale, upper, mirror, part);
+// Spin blocks of G that fit the LDS of one work-group (at most 150 KB)
+int prep_spin_blocks(int nb4, int pseudo_ns) {
+  int sb = pseudo_ns;
+  while (sb > 1 && !z_prep_fits(nb4, sb, 0, 0)) sb /= 2;
+  return sb;
 }
 }  // namespace
 
@@ -489,32 +522,56 @@ void gw_hip_kernel::p0_prep(int64_t q, const double2* G, int64_t t0, int64_t tc,
     p0_prep_gemm(q, G, t0, tc);
     return;
   }
-  const int64_t nk = d_.nk, NQ = d_.NQ, nao2 = d_.nao * d_.nao;
-  DevDims dd{(int)d_.nts, (int)d_.ns, (int)nk, (int)d_.nso, (int)d_.nao, (int)NQ, (int)d_.pns, (int)d_.pseudo_ns};
-  const int NB = (int)ceil_div(d_.nao, 16);
-  const size_t lds = (size_t)4 * (16 * NB) * (16 * NB + 1) * sizeof(double);
-  const double2* Vtq = Vq_ + q * nk * NQ * nao2;
-  const dim3 grid((unsigned)ceil_div(NQ, 4 * qpw), (unsigned)nk, (unsigned)tc);
-  const int* kp = kplus_tab_ + q * nk;
-  if (NB == 1) launch_z_prep<1>(grid, lds, stream_, dd, G, Vtq, scratch_, kp, (int)t0, qpw);
-  else if (NB == 2) launch_z_prep<2>(grid, lds, stream_, dd, G, Vtq, scratch_, kp, (int)t0, qpw);
-  else launch_z_prep<3>(grid, lds, stream_, dd, G, Vtq, scratch_, kp, (int)t0, qpw);
+  ZPrepArgs a = prep_args(q, G, t0, qpw);
+  const dim3 grid((unsigned)ceil_div(d_.NQ, 4 * a.qpb), (unsigned)d_.nk, (unsigned)tc);
+  orb_dispatch([&](auto nb) {
+    constexpr int NB4 = decltype(nb)::value;
+    const int sb = prep_spin_blocks(NB4, (int)d_.pseudo_ns);
+    for (int s0 = 0; s0 < d_.pseudo_ns; s0 += sb) {
+      a.s0 = s0;
+      a.sb = sb;
+      launch_orb(z_prep_kernel<NB4, 0>, a, grid, OrbCfg<NB4>::NT, z_prep_lds_bytes(NB4, sb, 0, 0), stream_);
+    }
+  });
+}
+
+ZPrepArgs gw_hip_kernel::prep_args(int64_t q, const double2* G, int64_t t0, int qpw) const {
+  const int64_t row = d_.nk * d_.NQ * d_.nao * d_.nao;
+  ZPrepArgs a{};
+  a.d = dev_dims();
+  a.G = G;
+  a.kplus = kplus_tab_ + q * d_.nk;
+  a.V = Vq_ + q * row;
+  a.Z = scratch_;
+  a.dst = Zs_;
+  a.exps = eZs_;
+  a.kc = (int)kc_p0_;
+  a.t0 = (int)t0;
+  a.qpb = qpw;
+  return a;
+}
+
+DevDims gw_hip_kernel::dev_dims() const {
+  return DevDims{(int)d_.nts, (int)d_.ns, (int)d_.nk, (int)d_.nso, (int)d_.nao, (int)d_.NQ, (int)d_.pns, (int)d_.pseudo_ns};
 }
 
 // Split precision, one or two collinear spin blocks: Z slices for q and tau in [t0, t0 + tc)
 // straight into Zs_.
 void gw_hip_kernel::p0_prep_slice(int64_t q, const double2* G, int64_t t0, int64_t tc, int qpw) {
-  const int64_t nk = d_.nk, NQ = d_.NQ, nao2 = d_.nao * d_.nao;
-  DevDims dd{(int)d_.nts, (int)d_.ns, (int)nk, (int)d_.nso, (int)d_.nao, (int)NQ, (int)d_.pns, (int)d_.pseudo_ns};
-  const int NB = (int)ceil_div(d_.nao, 16);
-  const size_t lds = (size_t)d_.pseudo_ns * 4 * (16 * NB) * (16 * NB + 1) * sizeof(double);
-  const double2* Vtq = Vq_ + q * nk * NQ * nao2;
-  const dim3 grid((unsigned)ceil_div(NQ, 4 * qpw), (unsigned)nk, (unsigned)tc);
-  const int* kp = kplus_tab_ + q * nk;
-  const int ns = split_ns_;
-  if (NB == 1) launch_z_prep_slice<1>(ns, grid, lds, stream_, dd, G, Vtq, Zs_, eZs_, (int)kc_p0_, kp, (int)t0, qpw);
-  else if (NB == 2) launch_z_prep_slice<2>(ns, grid, lds, stream_, dd, G, Vtq, Zs_, eZs_, (int)kc_p0_, kp, (int)t0, qpw);
-  else launch_z_prep_slice<3>(ns, grid, lds, stream_, dd, G, Vtq, Zs_, eZs_, (int)kc_p0_, kp, (int)t0, qpw);
+  ZPrepArgs a = prep_args(q, G, t0, qpw);
+  a.sb = (int)d_.pseudo_ns;
+  const dim3 grid((unsigned)ceil_div(d_.NQ, 4 * a.qpb), (unsigned)d_.nk, (unsigned)tc);
+  orb_dispatch([&](auto nb) {
+    constexpr int NB4 = decltype(nb)::value;
+    if constexpr (NB4 <= kFusedMaxNao / 4) {
+      const size_t lds = z_prep_lds_bytes(NB4, a.sb, split_ns_, (int)kc_p0_);
+      if (split_ns_ == 5) launch_orb(z_prep_kernel<NB4, 5>, a, grid, OrbCfg<NB4>::NT, lds, stream_);
+      else if (split_ns_ == 4) launch_orb(z_prep_kernel<NB4, 4>, a, grid, OrbCfg<NB4>::NT, lds, stream_);
+      else launch_orb(z_prep_kernel<NB4, 3>, a, grid, OrbCfg<NB4>::NT, lds, stream_);
+    } else {
+      throw status_error(GWHIP_ERR_UNSUPPORTED, "fused P0 slicing: nao out of range");
+    }
+  });
 }
 
 // P0(t0 .. t0+tc) = -(pref/nk) Z conj(V)^T, FP64 (tile `shape`).
@@ -529,24 +586,33 @@ void gw_hip_kernel::p0_gemm(int64_t q, int64_t tc, double2* Pt0, int shape) {
   a.alpha = make_double2(-d_.prefactor / (double)nk, 0.0);
   a.accumulate = 0; a.conjA = 0; a.conjB = 1;
   a.upper = g_herm_ ? 1 : 0;
-  // partial products in the Dyson work buffer, which only stage_dyson uses
-  zgemm_f64_splitk(a, zgemm_auto_ksplit(a, qchunk_ * (int64_t)dyson_per_q()), Pw_, stream_, shape);
+  // partial products in one q of the Dyson work buffer, which only stage_dyson uses
+  zgemm_f64_autosplit(a, d_.nts / 2, Pw_, (int64_t)dyson_per_q(), stream_, shape);
 }
 
-// R = P-tilde(t0 .. t0+tc) conj(V) into scratch_, FP64 (tile `shape`): Pt0 = P-tilde at t0
-// [tc][NQ^2], Vb = V(k, k - q) of nkb k points [nkb][NQ][nao][nao], read per-Q transposed
-// (column (k, n, j) of the product is V^Q'_jn).
-void gw_hip_kernel::sigma_gemm(const double2* Pt0, const double2* Vb, int64_t nkb, int64_t tc, int shape) {
+// R = P-tilde(t0 .. t0+tc) conj(V) into scratch_, FP64 (tile `shape`): Pt0 = P-tilde at t0 [tc][NQ^2];
+// column (p, n, j) of the product is conj(V^Q'_jn(k, k - q)) = V^Q'_nj(k - q, k), read in the stored order
+// where the rows hold the latter (reading the former per-Q transposed touches a cache line per element).
+// With sigma_half the product takes only A's upper triangle, the diagonal 64 x 64 blocks weighted 1/2: for
+// Hermitian G and P-tilde, Sigma = X + X^H with X = sum V_Q G (U V^H)_Q and U + U^H = P-tilde
+// (finish_sigma adds X^H): 0.6 of the products at naux = 300.  Both together 8.2 -> 5.05 ms per launch at
+// nk = 27, nao = 26, naux = 250.
+void gw_hip_kernel::sigma_gemm(const double2* Pt0, const SigmaRows& r, int64_t tc, int shape) {
   const int64_t NQ = d_.NQ, nao2 = d_.nao * d_.nao, NQ2 = NQ * NQ;
   ZGemmArgs a{};
-  a.M = (int)NQ; a.N = (int)(nkb * nao2); a.K = (int)NQ; a.batch = (int)tc; a.kin = (int)NQ; a.nin = (int)nao2;
+  a.M = (int)NQ; a.N = (int)(r.n * nao2); a.K = (int)NQ; a.batch = (int)tc; a.kin = (int)NQ; a.nin = (int)nao2;
   a.A = Pt0; a.sAb = NQ2; a.sAm = NQ; a.sAko = 0; a.sAki = 1;
-  a.B = Vb; a.sBb = 0; a.sBko = 0; a.sBki = nao2; a.sBno = NQ * nao2; a.sBni = 1;
-  a.nin2 = (int)d_.nao; a.sBni2 = d_.nao;
-  a.C = scratch_; a.sCb = nkb * NQ * nao2; a.sCm = nao2; a.sCno = NQ * nao2; a.sCni = 1;
+  a.B = r.V; a.sBb = 0; a.sBko = 0; a.sBki = nao2; a.sBno = NQ * nao2; a.sBni = 1;
+  if (!r.adj) {
+    a.nin2 = (int)d_.nao;
+    a.sBni2 = d_.nao;
+    a.conjB = 1;
+  }
+  a.C = scratch_; a.sCb = r.n * NQ * nao2; a.sCm = nao2; a.sCno = NQ * nao2; a.sCni = 1;
   a.alpha = make_double2(1.0, 0.0);
-  a.accumulate = 0; a.conjA = 0; a.conjB = 1;
-  zgemm_f64(a, stream_, shape);
+  a.half = sigma_half(false) ? 1 : 0;
+  // the weighted blocks are 64 rows whatever the tile, so that the sums do not depend on it
+  zgemm_f64(a, stream_, a.half && shape == 1 ? 0 : shape);
 }
 
 // Split precision, P0: int8 slices of Z (rows (tau, Q), chunks k) into Zs_.
@@ -598,19 +664,18 @@ void gw_hip_kernel::sigma_slice(const double2* Pt0, int64_t tc) {
   slice_rows(sa, split_ns_, stream_);
 }
 
-// Split precision, R = P-tilde conj(V) into scratch_ from the slices: Vsb / eVsb = the slices and
-// exponents of V(k, k - q) for nkb k points ([nkb][nao^2][2][ns][kc_s], [nkb][nao^2]).
-void gw_hip_kernel::sigma_gemm_split(const int8_t* Vsb, const int* eVsb, int64_t nkb, int64_t tc, int group) {
+// Split precision, R = P-tilde conj(V) into scratch_ from the slices.
+void gw_hip_kernel::sigma_gemm_split(const SigmaRows& r, int64_t tc, int group) {
   const int64_t NQ = d_.NQ, nao2 = d_.nao * d_.nao;
   const int ns = split_ns_;
   OzGemmArgs o{};
-  o.M = (int)NQ; o.N = (int)(nkb * nao2); o.batch = (int)tc; o.kc = (int)kc_s_; o.nchunk = 1; o.nin = (int)nao2;
+  o.M = (int)NQ; o.N = (int)(r.n * nao2); o.batch = (int)tc; o.kc = (int)kc_s_; o.nchunk = 1; o.nin = (int)nao2;
   o.A = Ps_; o.sAm = OZ_PLANES * ns * kc_s_; o.sAb = NQ * o.sAm; o.sAc = 0;
   o.eA = ePs_; o.seAb = NQ; o.seAm = 1;
-  o.B = Vsb; o.sBb = 0; o.sBno = nao2 * OZ_PLANES * ns * kc_s_;
+  o.B = r.Vs; o.sBb = 0; o.sBno = nao2 * OZ_PLANES * ns * kc_s_;
   o.sBni = OZ_PLANES * ns * kc_s_; o.sBc = 0;
-  o.eB = eVsb; o.seBb = 0; o.seBno = nao2; o.seBni = 1;
-  o.C = scratch_; o.sCb = nkb * NQ * nao2; o.sCm = nao2; o.sCno = NQ * nao2; o.sCni = 1;
+  o.eB = r.eVs; o.seBb = 0; o.seBno = nao2; o.seBni = 1;
+  o.C = scratch_; o.sCb = r.n * NQ * nao2; o.sCm = nao2; o.sCno = NQ * nao2; o.sCni = 1;
   o.alpha = make_double2(1.0, 0.0);
   o.accumulate = 0;
   o.group_m = group;
@@ -816,127 +881,105 @@ void gw_hip_kernel::stage_dyson(int64_t nq, const int* q0_row) {
 }
 
 void gw_hip_kernel::stage_sigma(const double2* G, double2* Sigma, bool split) {
-  for (int64_t q = 0; q < d_.nk; ++q)
-    sigma_q(G, Sigma, split, P_ + q * d_.nts * d_.NQ * d_.NQ, Vq_neg(q), Vs_neg(q), eVs_neg(q), kminus_tab_ + q * d_.nk,
-            d_.nk);
+  for (int64_t q = 0; q < d_.nk; ++q) sigma_q(G, Sigma, split, P_ + q * d_.nts * d_.NQ * d_.NQ, sigma_rows(q));
 }
 
-// V(k, k - q) lives in the k + q' store of q' = neg_q_[q], and so do its slices.
-const double2* gw_hip_kernel::Vq_neg(int64_t q) const {
-  return Vq_ + (int64_t)neg_q_[q] * d_.nk * d_.NQ * d_.nao * d_.nao;
-}
-const int8_t* gw_hip_kernel::Vs_neg(int64_t q) const {
-  return Vs_s_ ? Vs_s_ + (int64_t)neg_q_[q] * d_.nk * d_.nao * d_.nao * OZ_PLANES * split_ns_ * kc_s_ : nullptr;
-}
-const int* gw_hip_kernel::eVs_neg(int64_t q) const {
-  return eVs_s_ ? eVs_s_ + (int64_t)neg_q_[q] * d_.nk * d_.nao * d_.nao : nullptr;
+// The full mesh's rows of q: V(k - q, k) of q's own store with p = k - q, or (adj_s_) V(k, k - q), which
+// lives in the k + q' store of q' = neg_q_[q], with p = k.
+SigmaRows gw_hip_kernel::sigma_rows(int64_t q) const {
+  const int64_t nk = d_.nk, nao2 = d_.nao * d_.nao, row = nk * d_.NQ * nao2;
+  SigmaRows r;
+  r.adj = adj_s_[q];
+  r.V = Vq_ + (r.adj ? q : neg_q_[q]) * row;
+  r.gidx = r.adj ? nullptr : kminus_tab_ + q * nk;
+  r.sidx = r.adj ? kplus_tab_ + q * nk : nullptr;
+  if (Vs_s_) {
+    r.Vs = Vs_s_ + q * nk * nao2 * OZ_PLANES * split_ns_ * kc_s_;
+    r.eVs = eVs_s_ + q * nk * nao2;
+  }
+  r.n = nk;
+  return r;
 }
 
-// Sigma += -1/nk sum over the nkb k points of one q: Pq = P-tilde of this q ([nts][NQ^2], the half
-// grid read), Vb / Vsb / eVsb = V(k, k - q) of the nkb points ([nkb][NQ][nao][nao]; slices and
-// exponents for split precision), km = the full-mesh index of k - q for each, Sigma
-// [nts][ns][nkb][nso^2].
-void gw_hip_kernel::sigma_q(const double2* G, double2* Sigma, bool split, const double2* Pq, const double2* Vb,
-                            const int8_t* Vsb, const int* eVsb, const int* km, int64_t nkb) {
-  const int64_t nk = d_.nk, NQ = d_.NQ, NQ2 = NQ * NQ, nts = d_.nts;
-  if (nkb < 1 || nkb > nk) throw status_error(GWHIP_ERR_ARG, "Sigma stage k count out of range");
+// Sigma += -1/nk sum over the rows of one q: Pq = P-tilde of this q ([nts][NQ^2], the half grid read).
+void gw_hip_kernel::sigma_q(const double2* G, double2* Sigma, bool split, const double2* Pq, const SigmaRows& r) {
+  const int64_t NQ2 = d_.NQ * d_.NQ;
+  if (r.n < 1 || r.n > d_.nk) throw status_error(GWHIP_ERR_ARG, "Sigma stage k count out of range");
 
   // P0(beta - tau) = P0(tau) makes P-tilde(beta - tau) = P-tilde(tau) (to the rounding of the
   // tau <-> Omega transforms, ~1e-12 relative on the IR grids), so R = P-tilde conj(V) is formed on
   // the half grid only and serves both tau and beta - tau in the epilogue.
-  const int64_t half = nts / 2;
+  const int64_t half = d_.nts / 2;
   for (int64_t t0 = 0; t0 < half; t0 += tchunk_sigma_) {
     const int64_t tc = std::min(tchunk_sigma_, half - t0);
     if (split) {
       sigma_slice(Pq + t0 * NQ2, tc);
-      timed(K_SIGMA_GEMM, [&] { sigma_gemm_split(Vsb, eVsb, nkb, tc, tune_.s_group); });
+      timed(K_SIGMA_GEMM, [&] { sigma_gemm_split(r, tc, tune_.s_group); });
     } else {
-      timed(K_SIGMA_GEMM, [&] { sigma_gemm(Pq + t0 * NQ2, Vb, nkb, tc, tune_.s_shape); });
+      timed(K_SIGMA_GEMM, [&] { sigma_gemm(Pq + t0 * NQ2, r, tc, tune_.s_shape); });
     }
-    timed(K_SIGMA_EPI, [&] { sigma_epi(G, Sigma, Vb, km, nkb, t0, tc, epi_form()); });
+    timed(K_SIGMA_EPI, [&] { sigma_epi(G, Sigma, r, t0, tc, split); });
   }
 }
 
 // Sigma += -1/nk (V G) R for the 2 tc tau of the half-grid chunk at t0 (R in scratch_) with the
-// register epilogue `form` (epi_form()), or the GEMM form of the orbital products.
-void gw_hip_kernel::sigma_epi(const double2* G, double2* Sigma, const double2* Vb, const int* km, int64_t nkb,
-                              int64_t t0, int64_t tc, int form) {
-  const int64_t nk = d_.nk, NQ = d_.NQ, nts = d_.nts;
-  const double scale = -1.0 / (double)nk;
+// register epilogue, or the GEMM form of the orbital products.
+void gw_hip_kernel::sigma_epi(const double2* G, double2* Sigma, const SigmaRows& r, int64_t t0, int64_t tc,
+                              bool split) {
+  const double scale = -1.0 / (double)d_.nk;
   if (orb_gemm()) {
-    sigma_epi_gemm(G, Sigma, Vb, km, nkb, t0, tc, scale);
+    sigma_epi_gemm(G, Sigma, r, t0, tc, scale);
     return;
   }
-  DevDims dd{(int)nts, (int)d_.ns, (int)nk, (int)d_.nso, (int)d_.nao, (int)NQ, (int)d_.pns, (int)d_.pseudo_ns};
-  const int qs = epi_qsplit(nkb);
-  double2* part = nullptr;
+  const int qs = epi_qsplit(r.n);
+  SigmaEpiArgs a{};
+  a.d = dev_dims();
+  a.G = G; a.V = r.V; a.R = scratch_; a.Sigma = Sigma; a.gidx = r.gidx; a.sidx = r.sidx;
+  a.adj = r.adj; a.nks = (int)r.n; a.t0 = (int)t0; a.scale = scale;
+  a.upper = sigma_upper(split) ? 1 : 0;
+  a.qsplit = qs;
   if (qs > 1) {
-    ensure_epi_part(nkb);
-    part = epi_part_;
-    zero(part, (int64_t)qs * nts * d_.ns * nkb * d_.nso * d_.nso);
+    ensure_epi_part(r.n);
+    a.part = epi_part_;
+    zero(a.part, (int64_t)qs * d_.nts * d_.ns * r.n * d_.nso * d_.nso);
   }
-  const dim3 grid((unsigned)nkb, (unsigned)qs, (unsigned)(2 * tc));
-  const int up = sigma_upper() ? 1 : 0;
-  const int n = (int)nkb, t = (int)t0;
-  const int nb4 = d_.nao <= 8 ? 2 : d_.nao <= 16 ? 4 : d_.nao <= 28 ? 7 : d_.nao <= 32 ? 8 : d_.nao <= 40 ? 10 : 12;
-  const XcdGrid xg = make_xcd_grid(grid);
-  auto go = [&](auto kern, int threads, size_t l4) {
-    allow_lds(kern, l4);
-    hipLaunchKernelGGL(kern, xcd_launch_grid(xg), dim3(threads), l4, stream_, xg, dd, G, Vb, scratch_, Sigma, km, n, t,
-                       scale, up, 1, (int)grid.y, part);
-  };
-  if (form == 1 && d_.nao <= 32) {  // 4 x 4 x 4 MFMAs, every i group in each wave
-    const size_t l4 = sigma_epi4_lds_bytes(nb4);
-    if (nb4 == 2) go(sigma_epi4_kernel<2>, 256, l4);
-    else if (nb4 == 4) go(sigma_epi4_kernel<4>, 256, l4);
-    else if (nb4 == 7) go(sigma_epi4_kernel<7>, 256, l4);
-    else go(sigma_epi4_kernel<8>, 256, l4);
-  } else if (form == 2) {  // 4 x 4 x 4 MFMAs, one i group per wave
-    if (nb4 == 2) go(sigma_epi4w_kernel<2, 4, 4>, 256, sigma_epi4w_lds_bytes<2, 4>());
-    else if (nb4 == 4) go(sigma_epi4w_kernel<4, 4, 4>, 256, sigma_epi4w_lds_bytes<4, 4>());
-    else if (nb4 == 7) go(sigma_epi4w_kernel<7, 2, 4>, 256, sigma_epi4w_lds_bytes<7, 2>());
-    else if (nb4 == 8) go(sigma_epi4w_kernel<8, 2, 4>, 256, sigma_epi4w_lds_bytes<8, 2>());
-    else if (nb4 == 10) go(sigma_epi4w_kernel<10, 1, 3>, 192, sigma_epi4w_lds_bytes<10, 1>());
-    else go(sigma_epi4w_kernel<12, 1, 3>, 192, sigma_epi4w_lds_bytes<12, 1>());
-  } else {  // 16 x 16 x 4 MFMAs
-    const int NB = (int)ceil_div(d_.nao, 16);
-    const size_t lds = ((size_t)2 * (16 * NB) * (16 * NB + 1) + (size_t)NB * NB * 8 * 64) * sizeof(double);
-    if (NB == 1) launch_sigma_epi<1>(grid, lds, stream_, dd, G, Vb, scratch_, Sigma, km, n, t, scale, up, 1, part);
-    else if (NB == 2) launch_sigma_epi<2>(grid, lds, stream_, dd, G, Vb, scratch_, Sigma, km, n, t, scale, up, 1, part);
-    else launch_sigma_epi<3>(grid, lds, stream_, dd, G, Vb, scratch_, Sigma, km, n, t, scale, up, 1, part);
-  }
-  GWHIP_CHECK(hipGetLastError());
+  const dim3 grid((unsigned)r.n, (unsigned)qs, (unsigned)(2 * tc * d_.pseudo_ns));
+  orb_dispatch([&](auto nb) {
+    constexpr int NB4 = decltype(nb)::value;
+    const dim3 g(grid.x, grid.y, grid.z * RedCfg<NB4>::GROUPS);
+    launch_orb(sigma_epi_kernel<NB4>, a, g, RedCfg<NB4>::NT, OrbReduce<NB4, false>::lds_bytes(), stream_);
+  });
   if (qs > 1) {
-    const int64_t per_tau = d_.ns * nkb * d_.nso * d_.nso;
+    const int64_t per_tau = d_.ns * r.n * d_.nso * d_.nso;
     const int64_t nel = 2 * tc * per_tau;
     hipLaunchKernelGGL(epi_part_reduce_kernel, dim3((unsigned)std::min<int64_t>(4096, ceil_div(nel, 256))), dim3(256), 0,
-                       stream_, part, Sigma, qs, nts * per_tau, per_tau, t, (int)tc, (int)nts);
+                       stream_, a.part, Sigma, qs, d_.nts * per_tau, per_tau, (int)t0, (int)tc, (int)d_.nts);
     GWHIP_CHECK(hipGetLastError());
   }
 }
 
-// Sigma of Hermitian G is Hermitian; with one spin block per (tau, s, k) only its upper 16 x 16
-// blocks were accumulated, so fill the rest from them.
-bool gw_hip_kernel::sigma_upper() const { return g_herm_ && d_.pns == 1 && !orb_gemm(); }
+// FP64, Hermitian G and P-tilde: R from the upper triangle of P-tilde (sigma_gemm) and Sigma = X + X^H at the
+// end.  Not in split precision: there the products' errors of the two triangles are independent, and the
+// half form would count one of them twice.
+bool gw_hip_kernel::sigma_half(bool split) const { return g_herm_ && grid_herm_ && !split; }
 
-// The fused P0 prep + slicing kernel takes one or two collinear spin blocks (their G planes share
-// the work-group's LDS: 150 KB at nao = 48 with two).
-bool gw_hip_kernel::fused_p0() const { return d_.pns == 1 && d_.pseudo_ns <= 2 && !orb_gemm(); }
+// Sigma of Hermitian G is Hermitian; with one spin block per (tau, s, k) and the whole P-tilde in R only its
+// upper 4 x 4 blocks are accumulated, and the rest filled from them.
+bool gw_hip_kernel::sigma_upper(bool split) const {
+  return g_herm_ && d_.pns == 1 && !orb_gemm() && !sigma_half(split);
+}
 
-// The register Sigma epilogue for this nao: the tuned form where it applies, else by measurement
-// (one MI355X, split Sigma-evals): 4 x 4 x 4 MFMAs with all i groups per wave up to nao = 32
-// (nao = 26: 12.2 ms per launch against 13.6 for 16 x 16 x 4), one i group per wave up to 40
-// (nao = 40, ns = 2: 55.7 against 63.9 ms), and 16 x 16 x 4 above, where both pad to 48 (nao = 48:
-// 29.0 against 31.3 ms).
-int gw_hip_kernel::epi_form() const {
-  if (tune_.epi_form == 1 && d_.nao <= 32) return 1;
-  if (tune_.epi_form == 2 || tune_.epi_form == 3) return tune_.epi_form;
-  return d_.nao <= 32 ? 1 : d_.nao <= 40 ? 2 : 3;
+// The fused P0 prep + slicing kernel takes one or two collinear spin blocks, as far as their G blocks and
+// a quad's digits fit the work-group's LDS (with two and four slices: nao = 36).
+bool gw_hip_kernel::fused_p0() const {
+  if (d_.pns != 1 || d_.pseudo_ns > 2 || d_.nao > kFusedMaxNao || orb_gemm()) return false;
+  const int nb4 = (int)ceil_div(d_.nao, 4), kc = (int)ceil_div(d_.nao * d_.nao, 64) * 64;
+  return z_prep_fits(nb4 > 10 ? 12 : nb4, (int)d_.pseudo_ns, split_ns_, kc);
 }
 
 int gw_hip_kernel::epi_qsplit(int64_t nks) const {
-  // the full-mesh launch has nks x nts work-groups; under ~2048 (eight per CU) the Q loop is split
-  const int64_t blocks = nks * d_.nts;
+  // the full-mesh launch has nks x nts x spin blocks work-groups; under ~2048 (eight per CU) the Q loop is split
+  const int64_t blocks = nks * d_.nts * d_.pseudo_ns;
   if (orb_gemm() || blocks >= 2048 || d_.NQ < 32) return 1;
   return (int)std::min<int64_t>(4, std::min<int64_t>(ceil_div(2048, blocks), d_.NQ / 16));
 }
@@ -954,7 +997,7 @@ void gw_hip_kernel::ensure_epi_part(int64_t nks) {
 
 void gw_hip_kernel::ensure_orb_buffers() {
   ensure_epi_part(d_.nk);
-  if (!orb_gemm()) return;
+  if (!vjp_gemm()) return;
   if (!orb_W_) orb_W_ = dalloc<double2>((size_t)d_.nk * d_.NQ * d_.nao * d_.nao);
   if (!orb_G_) orb_G_ = dalloc<double2>((size_t)d_.nk * d_.nso * d_.nso);
   if (!orb_part_) orb_part_ = dalloc<double2>((size_t)kOrbKsplit * d_.nk * d_.nao * d_.nao);
@@ -1013,21 +1056,23 @@ void gw_hip_kernel::p0_prep_gemm(int64_t q, const double2* G, int64_t t0, int64_
 //   XT[k][Q][n][i] = sum_m G(k)[m][n] V_Q[i][m],   G = G(tau, is, km[k]) block (a, b), i.e. X = V_Q G
 //   Sigma(tau, is, k)[a,b](i, j) += scale sum_{Q, n} X[i][Q, n] R[k][Q][n][j]
 // (sigma_epi_mfma_kernel's products, src/gw_cpu_kernel.cpp:359-373).
-void gw_hip_kernel::sigma_epi_gemm(const double2* G, double2* Sigma, const double2* Vb, const int* km, int64_t nkb,
-                                   int64_t t0, int64_t tc, double scale) {
-  const int64_t NQ = d_.NQ, nao = d_.nao, nao2 = nao * nao, nso = d_.nso, nso2 = nso * nso, vq = NQ * nao2;
+void gw_hip_kernel::sigma_epi_gemm(const double2* G, double2* Sigma, const SigmaRows& r, int64_t t0, int64_t tc,
+                                   double scale) {
+  const int64_t NQ = d_.NQ, nao = d_.nao, nao2 = nao * nao, nso = d_.nso, nso2 = nso * nso, vq = NQ * nao2, nkb = r.n;
   if (!orb_W_ || !orb_G_) throw status_error(GWHIP_ERR_STATE, "orbital GEMM buffers not allocated");
   for (int64_t tz = 0; tz < tc; ++tz)
     for (int side = 0; side < 2; ++side) {
       const int64_t tau = side ? d_.nts - 1 - (t0 + tz) : t0 + tz;
       for (int64_t s = 0; s < d_.pseudo_ns; ++s) {
         const int64_t is = s / (d_.pns * d_.pns), a = (s / d_.pns) % d_.pns, b = s % d_.pns;
-        gather_g(G, tau, is, km, nkb);
+        gather_g(G, tau, is, r.gidx, nkb);
         ZGemmArgs x{};
         x.M = (int)nao; x.N = (int)(NQ * nao); x.K = (int)nao; x.batch = (int)nkb; x.kin = (int)nao;
         x.nin = (int)nao;
         x.A = orb_G_ + a * nao * nso + b * nao; x.sAb = nso2; x.sAm = 1; x.sAko = 0; x.sAki = nso;
-        x.B = Vb; x.sBb = vq; x.sBko = 0; x.sBki = 1; x.sBno = nao2; x.sBni = nao;
+        // V_Q[i][m], or with adj the conjugate of the stored V_Q[m][i]
+        x.B = r.V; x.sBb = vq; x.sBko = 0; x.sBki = r.adj ? nao : 1; x.sBno = nao2; x.sBni = r.adj ? 1 : nao;
+        x.conjB = r.adj;
         x.C = orb_W_; x.sCb = vq; x.sCm = nao; x.sCno = nao2; x.sCni = 1;
         x.alpha = make_double2(1.0, 0.0);
         zgemm_f64(x, stream_);
@@ -1040,20 +1085,32 @@ void gw_hip_kernel::sigma_epi_gemm(const double2* G, double2* Sigma, const doubl
         y.sCno = 0; y.sCni = 1;
         y.alpha = make_double2(scale, 0.0);
         y.accumulate = 1;
+        if (r.sidx) {  // permuted outputs: whole blocks first, then added to their places
+          y.C = orb_O_; y.sCb = nao2; y.sCm = nao;
+          y.accumulate = 0;
+        }
         // only nkb x (nao / 64)^2 output tiles, each over K = NQ nao: cut K so that ~1024 blocks run
         const int64_t tiles = nkb * ceil_div(nao, 64) * ceil_div(nao, 64);
         const int ksplit = (int)std::min<int64_t>(kOrbKsplit, std::max<int64_t>(1, ceil_div(1024, tiles)));
         zgemm_f64_splitk(y, ksplit, orb_part_, stream_);
+        if (r.sidx) {
+          hipLaunchKernelGGL(scatter_block_add_kernel, dim3((unsigned)ceil_div(nao2, 256), (unsigned)nkb), dim3(256), 0,
+                             stream_, orb_O_, Sigma + (tau * d_.ns + is) * nkb * nso2 + a * nao * nso + b * nao, r.sidx,
+                             (int)nao, nso, nso2);
+          GWHIP_CHECK(hipGetLastError());
+        }
       }
     }
 }
 
-void gw_hip_kernel::finish_sigma(double2* Sigma, int64_t nkS) {
-  if (!sigma_upper()) return;
+void gw_hip_kernel::finish_sigma(double2* Sigma, int64_t nkS, bool split) {
+  const bool half = sigma_half(split);
+  if (!half && !sigma_upper(split)) return;
   const int64_t n = d_.nso, nmat = d_.nts * d_.ns * nkS;
   for (int64_t m0 = 0; m0 < nmat; m0 += 65535) {  // grid.y limit
     const int64_t mc = std::min<int64_t>(65535, nmat - m0);
-    mirror_upper(Sigma + m0 * n * n, (int)n, n * n, mc, stream_);
+    if (half) hermitize(Sigma + m0 * n * n, (int)n, n * n, mc, stream_, 1.0);
+    else mirror_upper(Sigma + m0 * n * n, (int)n, n * n, mc, stream_);
     GWHIP_CHECK(hipGetLastError());
   }
 }
@@ -1065,7 +1122,7 @@ void gw_hip_kernel::enqueue_eval(const double2* G, double2* Sigma, int precision
   stage_p0(G, p0_split(precision));
   stage_dyson(d_.nk, q0_qiq_);
   stage_sigma(G, Sigma, sigma_split(precision));
-  finish_sigma(Sigma, d_.nk);
+  finish_sigma(Sigma, d_.nk, sigma_split(precision));
   if (nonfinite_flag) {
     hipLaunchKernelGGL(nonfinite_kernel, dim3(1024), dim3(256), 0, stream_, Sigma, nsig, nonfinite_flag);
     GWHIP_CHECK(hipGetLastError());
@@ -1103,7 +1160,7 @@ void gw_hip_kernel::solve_device(const double2* G, double2* Sigma, int precision
   q0_eps_ = false;
   GWHIP_CHECK(hipEventRecord(t2, stream_));
   stage_sigma(G, Sigma, sigma_split(precision));
-  finish_sigma(Sigma, d_.nk);
+  finish_sigma(Sigma, d_.nk, sigma_split(precision));
   if (q0_on_ && q0_apply) apply_q0(Sigma, G, d_.nk);
   GWHIP_CHECK(hipEventRecord(t3, stream_));
   hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(64), 0, stream_, flag_, (int64_t)1);
@@ -1165,7 +1222,7 @@ void gw_hip_kernel::autotune(const double2* G, int precision) {
     const int shapes[3] = {0, 1, 2};
     p0_prep(0, G, 0, tcp, tune_.qpw);
     tune_.p0_shape = best_of(3, shapes, [&](int c) { p0_gemm(0, tcp, P_, c); });
-    tune_.s_shape = best_of(3, shapes, [&](int c) { sigma_gemm(P_, Vq_neg(0), d_.nk, tcs, c); });
+    tune_.s_shape = best_of(3, shapes, [&](int c) { sigma_gemm(P_, sigma_rows(d_.nk - 1), tcs, c); });
   } else {
     if (fused_p0()) {  // fused prep + slicing vs the two kernels
       const int fz[2] = {0, 1};
@@ -1193,37 +1250,11 @@ void gw_hip_kernel::autotune(const double2* G, int precision) {
     sigma_slice(P_, tcs);
     tune_.s_oz_tile = best_of(2, tiles, [&](int c) {
       tune_.s_oz_tile = c;
-      sigma_gemm_split(Vs_neg(0), eVs_neg(0), d_.nk, tcs, tune_.s_group);
+      sigma_gemm_split(sigma_rows(0), tcs, tune_.s_group);
     });
-    tune_.s_group = best_of(7, groups, [&](int c) { sigma_gemm_split(Vs_neg(0), eVs_neg(0), d_.nk, tcs, c); });
+    tune_.s_group = best_of(7, groups, [&](int c) { sigma_gemm_split(sigma_rows(0), tcs, c); });
   }
-  // register Sigma epilogue form, on the R of q = 0 the Sigma GEMMs above left in scratch_ (Sigma
-  // into a temporary buffer; where device memory cannot hold one, the form stays chosen by nao)
-  double2* S = nullptr;
-  const size_t nsig = (size_t)d_.nts * d_.ns * d_.nk * d_.nso * d_.nso;
-  if (!orb_gemm()) {
-    try {
-      S = dalloc<double2>(nsig);
-    } catch (const status_error& e) {
-      if (e.status != GWHIP_ERR_OOM) throw;
-      tune_.epi_form = 0;
-    }
-  }
-  if (S) {
-    const int forms[3] = {1, 2, 3};
-    const int first = d_.nao <= 32 ? 0 : 1;  // the all-groups form covers nao <= 32
-    try {
-      tune_.epi_form = best_of(3 - first, forms + first,
-                               [&](int c) { sigma_epi(G, S, Vq_neg(0), kminus_tab_, d_.nk, 0, tcs, c); });
-    } catch (...) {
-      (void)hipFree(S);
-      bytes_ -= nsig * sizeof(double2);
-      throw;
-    }
-    GWHIP_CHECK(hipStreamSynchronize(stream_));
-    (void)hipFree(S);
-    bytes_ -= nsig * sizeof(double2);
-  }
+  tune_.epi_form = 1;
   stored_valid_ = false;
   ++generation_;
 }
@@ -1274,8 +1305,7 @@ void gw_hip_kernel::solve_device_in(const double2* G, double2* Sigma, int precis
   if (!precision_valid(precision)) throw status_error(GWHIP_ERR_ARG, "unknown precision");
   if (!G || !Sigma || !ws) throw status_error(GWHIP_ERR_ARG, "null G, Sigma or workspace");
   if ((uintptr_t)ws % kWsAlign != 0) throw status_error(GWHIP_ERR_ARG, "workspace not 256-byte aligned");
-  if (orb_gemm())
-    throw status_error(GWHIP_ERR_UNSUPPORTED, "the orbital GEMM form (nao > 48 or tuned on) needs buffers of its own");
+  if (vjp_gemm()) throw status_error(GWHIP_ERR_UNSUPPORTED, "nao > 48 or the orbital GEMM form");
   if (q0_on_) throw status_error(GWHIP_ERR_UNSUPPORTED, "the q -> 0 correction runs a host fit between stages");
   const bool split = any_split(precision);
   if (split && !split_ready())
@@ -1412,9 +1442,8 @@ void gw_hip_kernel::eval_one_q_host(const double2* G, int64_t q, int precision, 
   if (Pt) GWHIP_CHECK(hipMemcpy(Pt, P_, (size_t)d_.nts * n2 * sizeof(double2), hipMemcpyDeviceToHost));
   if (Sq) {
     zero(S_dev_, (int64_t)nsig);
-    sigma_q(G_dev_, S_dev_, sigma_split(precision), P_, Vq_neg(q), Vs_neg(q), eVs_neg(q), kminus_tab_ + q * d_.nk,
-            d_.nk);
-    finish_sigma(S_dev_, d_.nk);
+    sigma_q(G_dev_, S_dev_, sigma_split(precision), P_, sigma_rows(q));
+    finish_sigma(S_dev_, d_.nk, sigma_split(precision));
     GWHIP_CHECK(hipStreamSynchronize(stream_));
     GWHIP_CHECK(hipMemcpy(Sq, S_dev_, nsig * sizeof(double2), hipMemcpyDeviceToHost));
   }

@@ -46,11 +46,10 @@ struct Tuning {
                                       // 4 (64 x 64, 32 x 32 x 32 MFMAs, staged by LDS DMA)
   int p0_fused = 1;  // split precision, one or two collinear spin blocks: P0 orbital kernel writes int8
                      // slices directly
-  int orb_gemm = 0;  // orbital contractions as batched FP64 GEMMs (always so for nao > 48)
+  int orb_gemm = 0;  // orbital contractions as batched FP64 GEMMs (always so for nao > 64)
   int p0_kchunks = 4;  // split precision: k chunks per launch of the int8 P0 GEMM (0: all in one), so
                        // that each launch's operand window stays in L2
-  int epi_form = 0;  // register Sigma epilogue: 0 by nao, 1 4x4x4 all i groups per wave (nao <= 32),
-                     // 2 4x4x4 one i group per wave, 3 16x16x4
+  int epi_form = 0;  // 0 .. 3 accepted; one form of the Sigma epilogue is left, so it has no effect
   static constexpr int count = 11;
   void to_array(int* v) const {
     const int a[count] = {p0_shape, s_shape, qpw, p0_group, s_group, p0_oz_tile, s_oz_tile, p0_fused, orb_gemm,
@@ -81,6 +80,21 @@ struct Workspace {
   size_t exp_elems = 0;
 };
 
+// The k points of one q in the Sigma stage, in the order p of V's rows: G is read at gidx[p], Sigma written
+// at sidx[p] (null: p).  V: rows V(k, k - q) [n][NQ][nao^2], or with adj V(k - q, k) = V(k, k - q)^H;
+// Vs, eVs: the slices and exponents of conj(V(k, k - q)) per (p, (n, j)) for split precision.
+struct SigmaRows {
+  const double2* V = nullptr;
+  int adj = 0;
+  const int8_t* Vs = nullptr;
+  const int* eVs = nullptr;
+  const int* gidx = nullptr;
+  const int* sidx = nullptr;
+  int64_t n = 0;
+};
+
+struct ZPrepArgs;
+struct DevDims;
 struct OrbOp;
 struct OrbOut;
 struct OrbArgs;
@@ -189,7 +203,7 @@ public:
   // over Q ranges (full mesh); allocates, so call before a capture
   void ensure_orb_buffers();
   // the register-chained orbital kernels handle nao up to 3 x 16
-  static constexpr int64_t kOrbMaxNao = 48;
+  static constexpr int64_t kOrbMaxNao = 64, kVjpMaxNao = 48, kFusedMaxNao = 48;
   bool has_inputs() const { return grid_set_ && v_set_; }
   // after the stream has drained: whether the last evaluation's Dyson step met a matrix I - P0
   // that is not positive definite
@@ -240,7 +254,7 @@ private:
   int64_t kc_p0_ = 0, kc_s_ = 0;
   int8_t* Vs_p0_ = nullptr;   // [nq][NQ][nk][2][ns][kc_p0]
   int* eVs_p0_ = nullptr;     // [nq][NQ][nk]
-  int8_t* Vs_s_ = nullptr;    // [nq][nk][nao^2][2][ns][kc_s]
+  int8_t* Vs_s_ = nullptr;    // [nq][nk][nao^2][2][ns][kc_s], rows as SigmaRows
   int* eVs_s_ = nullptr;      // [nq][nk][nao^2]
   int8_t* Zs_ = nullptr;      // [tc][NQ][nk][2][ns][kc_p0]  (P0 stage)
   int* eZs_ = nullptr;
@@ -305,6 +319,12 @@ private:
   double2* hf_sym_ = nullptr;
   int64_t hf_exchange_launches_ = 0;
   std::vector<int> kplus_host_, kminus_host_, neg_q_, q0_qiq_host_;
+  // whether V(k, k - q) (Sigma) and V(k, k') (exchange) of q are read as the adjoint of the stored V of the
+  // reversed pair
+  std::vector<int> adj_s_;
+  int* adj_x_dev_ = nullptr;     // [nq]
+  int* hf_herm_ = nullptr;       // Hartree-Fock: the density matrix is Hermitian to rounding
+  bool grid_herm_ = false;       // Hermitian P-tilde(i Omega) give a Hermitian P-tilde(tau)
 
   double region_ms_[R_COUNT] = {0};
   KernelStat kstat_[K_COUNT];
@@ -326,11 +346,11 @@ private:
   std::vector<int> q0_samples() const;
   void apply_q0(double2* Sigma, const double2* G, int64_t nkS);
   void p0_prep(int64_t q, const double2* G, int64_t t0, int64_t tc, int qpw);
-  // orbital contractions as batched GEMMs (nao > 48, or tuning orb_gemm)
+  // orbital contractions as batched GEMMs (nao > 64, or tuning orb_gemm); the VJP's from nao > 48 on
   bool orb_gemm() const { return d_.nao > kOrbMaxNao || tune_.orb_gemm != 0; }
+  bool vjp_gemm() const { return d_.nao > kVjpMaxNao || tune_.orb_gemm != 0; }
   void p0_prep_gemm(int64_t q, const double2* G, int64_t t0, int64_t tc);
-  void sigma_epi_gemm(const double2* G, double2* Sigma, const double2* Vb, const int* km, int64_t nkb, int64_t t0,
-                      int64_t tc, double scale);
+  void sigma_epi_gemm(const double2* G, double2* Sigma, const SigmaRows& r, int64_t t0, int64_t tc, double scale);
   void gather_g(const double2* G, int64_t tau, int64_t is, const int* map, int64_t n);
   void gather_mats(const double2* base, const int* map, int64_t n);
   void hf_exchange_gemm(const double2* dm_s, int nblk);
@@ -340,13 +360,15 @@ private:
   void vjp_reduce(bool has_m, int NB, dim3 grid, const OrbArgs& a, const OrbOp& A, const OrbOp& M, const OrbOp& C,
                   const OrbOut& O);
   void orb_gather_view(const OrbArgs& a, const OrbOp& op, int tz, int64_t n);
+  ZPrepArgs prep_args(int64_t q, const double2* G, int64_t t0, int qpw) const;
+  DevDims dev_dims() const;
   void p0_prep_slice(int64_t q, const double2* G, int64_t t0, int64_t tc, int qpw);
   void p0_gemm(int64_t q, int64_t tc, double2* Pt0, int shape);
-  void sigma_gemm(const double2* Pt0, const double2* Vb, int64_t nkb, int64_t tc, int shape);
+  void sigma_gemm(const double2* Pt0, const SigmaRows& r, int64_t tc, int shape);
   void p0_slice(int64_t tc);
   void p0_gemm_split(int64_t q, int64_t tc, double2* Pt0, int group, int kchunks);
   void sigma_slice(const double2* Pt0, int64_t tc);
-  void sigma_gemm_split(const int8_t* Vsb, const int* eVsb, int64_t nkb, int64_t tc, int group);
+  void sigma_gemm_split(const SigmaRows& r, int64_t tc, int group);
   void stage_p0(const double2* G, bool split, const std::vector<int>* qs = nullptr);
   void p0_one_q(int64_t q, const double2* G, bool split, double2* Pq);
   // in-place inverse of nmat Hermitian positive-definite NQ x NQ matrices by block Gauss-Jordan steps
@@ -355,21 +377,19 @@ private:
   void check_dyson_flag();  // reads dyson_flag_ (synchronous) and throws when it is set
   void stage_dyson(int64_t nq, const int* q0_row);
   void stage_sigma(const double2* G, double2* Sigma, bool split);
-  void sigma_epi(const double2* G, double2* Sigma, const double2* Vb, const int* km, int64_t nkb, int64_t t0,
-                 int64_t tc, int form);
-  void sigma_q(const double2* G, double2* Sigma, bool split, const double2* Pq, const double2* Vb, const int8_t* Vsb,
-               const int* eVsb, const int* km, int64_t nkb);
-  const double2* Vq_neg(int64_t q) const;  // V(k, k - q) for every k: the k + q' rows of q' = -q
-  const int8_t* Vs_neg(int64_t q) const;
-  const int* eVs_neg(int64_t q) const;
-  bool sigma_upper() const;
-  int epi_form() const;
+  void sigma_epi(const double2* G, double2* Sigma, const SigmaRows& r, int64_t t0, int64_t tc, bool split);
+  void sigma_q(const double2* G, double2* Sigma, bool split, const double2* Pq, const SigmaRows& r);
+  SigmaRows sigma_rows(int64_t q) const;  // the full mesh's rows of q
+  bool sigma_upper(bool split) const;
+  bool sigma_half(bool split) const;
   bool fused_p0() const;
   // Q ranges of the register-chained Sigma epilogue for nks k points: 1 when nks x nts work-groups
   // fill the chip, up to 4 otherwise; ensure_epi_part sizes epi_part_ for it
   int epi_qsplit(int64_t nks) const;
   void ensure_epi_part(int64_t nks);
-  void finish_sigma(double2* Sigma, int64_t nkS);
+  void finish_sigma(double2* Sigma, int64_t nkS, bool split);
+  template <typename F>
+  void orb_dispatch(F&& f) const;
   void star_tables();
   const double2* star_rotate(int64_t iq, int64_t q);
   void solve_star_device(const double2* G_ibz, double2* Sigma_ibz, int precision);

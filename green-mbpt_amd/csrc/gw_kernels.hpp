@@ -22,13 +22,14 @@ __device__ __forceinline__ int64_t g_index(const DevDims& d, int t, int is, int 
 }
 
 // ---------------------------------------------------------------------------------------
-// X = (X + X^H)/2 for a batch of N x N matrices (common_defs.h:104-115), with coalesced accesses:
+// X = f (X + X^H), f = 1/2 (common_defs.h:104-115) or 1, for a batch of N x N matrices, with coalesced
+// accesses:
 // block (y = matrix) takes the tile pair (I, J), I <= J,
 // of 32 x 32 tiles (blockIdx.x enumerates the upper tile triangle), stages tile (I, J) and tile (J, I)
-// in LDS, and writes h = (A[a][b] + conj(B[b][a]))/2 to (I, J) and conj(h) to (J, I) (on a diagonal
+// in LDS, and writes h = f (A[a][b] + conj(B[b][a])) to (I, J) and conj(h) to (J, I) (on a diagonal
 // tile the same formula is Hermitian by construction, with a real diagonal).
 constexpr int HERM_TILE = 32;
-__global__ __launch_bounds__(256) void hermitize_tiled_kernel(double2* X, int N, int64_t stride) {
+__global__ __launch_bounds__(256) void hermitize_tiled_kernel(double2* X, int N, int64_t stride, double f) {
   __shared__ double2 ta[HERM_TILE][HERM_TILE + 1], tb[HERM_TILE][HERM_TILE + 1];
   const int T = (N + HERM_TILE - 1) / HERM_TILE;
   // blockIdx.x -> (I, J) with I <= J, row-major over the upper triangle
@@ -50,7 +51,7 @@ __global__ __launch_bounds__(256) void hermitize_tiled_kernel(double2* X, int N,
     const int a = e / HERM_TILE, b = e % HERM_TILE;
     if (i0 + a >= N || j0 + b >= N) continue;
     const double2 u = ta[a][b], l = tb[b][a];
-    ta[a][b] = make_double2(0.5 * (u.x + l.x), 0.5 * (u.y - l.y));
+    ta[a][b] = make_double2(f * (u.x + l.x), f * (u.y - l.y));
   }
   __syncthreads();
   for (int e = threadIdx.x; e < HERM_TILE * HERM_TILE; e += blockDim.x) {
@@ -63,11 +64,11 @@ __global__ __launch_bounds__(256) void hermitize_tiled_kernel(double2* X, int N,
   }
 }
 
-// (X + X^H)/2 for nmat N x N matrices at `stride` apart (nmat <= 65535).
-inline void hermitize(double2* X, int N, int64_t stride, int64_t nmat, hipStream_t st) {
+// f (X + X^H) for nmat N x N matrices at `stride` apart (nmat <= 65535).
+inline void hermitize(double2* X, int N, int64_t stride, int64_t nmat, hipStream_t st, double f = 0.5) {
   const int T = (N + HERM_TILE - 1) / HERM_TILE;
   hipLaunchKernelGGL(hermitize_tiled_kernel, dim3((unsigned)(T * (T + 1) / 2), (unsigned)nmat), dim3(256), 0, st, X, N,
-                     stride);
+                     stride, f);
 }
 
 // Upper triangle -> Hermitian matrix: X[i][j] = conj(X[j][i]) below the diagonal, real diagonal.
@@ -108,26 +109,46 @@ inline void mirror_upper(double2* X, int N, int64_t stride, int64_t nmat, hipStr
 }
 
 // max_(i,j) |X[i][j] - conj(X[j][i])| and max |X| over nmat N x N matrices, as the bit patterns
-// of non-negative doubles (ordered like the values) combined with atomicMax.
-__global__ void herm_check_kernel(const double2* X, int64_t nmat, int N, unsigned long long* out) {
+// of non-negative doubles (ordered like the values) combined with atomicMax; a NaN counts as infinity.
+// One pair of atomics per work-group on a grid of a few per CU (one pair per wave of 1024 work-groups
+// took 96 us on the nk = 8, nao = 8 system, all of it the 8192 atomics on two addresses).
+__global__ __launch_bounds__(256) void herm_check_kernel(const double2* X, int64_t nmat, int N, unsigned long long* out) {
+  __shared__ double red[2][4];
   const int64_t n2 = (int64_t)N * N, total = nmat * n2;
   const int64_t step = (int64_t)gridDim.x * blockDim.x;
   double dmax = 0.0, amax = 0.0;
+  auto up = [](double m, double x) { return x <= m ? m : (x > m ? x : __builtin_huge_val()); };
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += step) {
-    const int64_t m = e / n2, r = e - m * n2;
-    const int i = (int)(r / N), j = (int)(r - (r / N) * N);
+    const int64_t m = e / n2;
+    const int r = (int)(e - m * n2), i = r / N, j = r - (r / N) * N;
     const double2 a = X[e], b = X[m * n2 + (int64_t)j * N + i];
-    dmax = fmax(dmax, fmax(fabs(a.x - b.x), fabs(a.y + b.y)));
-    amax = fmax(amax, fmax(fabs(a.x), fabs(a.y)));
+    dmax = up(up(dmax, fabs(a.x - b.x)), fabs(a.y + b.y));
+    amax = up(up(amax, fabs(a.x)), fabs(a.y));
   }
   for (int o = 32; o > 0; o >>= 1) {
     dmax = fmax(dmax, __shfl_xor(dmax, o, 64));
     amax = fmax(amax, __shfl_xor(amax, o, 64));
   }
   if ((threadIdx.x & 63) == 0) {
-    atomicMax(out + 0, (unsigned long long)__double_as_longlong(dmax));
-    atomicMax(out + 1, (unsigned long long)__double_as_longlong(amax));
+    red[0][threadIdx.x >> 6] = dmax;
+    red[1][threadIdx.x >> 6] = amax;
   }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    dmax = fmax(fmax(red[0][0], red[0][1]), fmax(red[0][2], red[0][3]));
+    amax = fmax(fmax(red[1][0], red[1][1]), fmax(red[1][2], red[1][3]));
+    if (dmax > 0.0) atomicMax(out + 0, (unsigned long long)__double_as_longlong(dmax));
+    if (amax > 0.0) atomicMax(out + 1, (unsigned long long)__double_as_longlong(amax));
+  }
+}
+inline unsigned herm_check_blocks(int64_t elems) {
+  return (unsigned)(elems < (int64_t)512 * 256 ? (elems + 255) / 256 : 512);
+}
+
+// flag = the matrices of a herm_check_kernel are Hermitian to rel (max |X - X^H| <= rel max |X|, finite)
+__global__ void herm_flag_kernel(const unsigned long long* c, double rel, int* flag) {
+  const double d = __longlong_as_double((long long)c[0]), a = __longlong_as_double((long long)c[1]);
+  *flag = isfinite(d) && d <= rel * a ? 1 : 0;
 }
 
 // P0 half-grid symmetrisation for all q: Hermitise P[q][t] for t < nts/2
@@ -381,14 +402,27 @@ __global__ void zero_kernel(double2* X, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += step) X[i] = make_double2(0.0, 0.0);
 }
 
-// Out[k] = G[base + map[k] nso^2 ...] for k < grid.y: one (tau, spin) slice of G at mapped k
-// points, whole nso x nso matrices.
+// Out[k] = G[base + map[k] nso^2 ...] for k < grid.y (null map: k): one (tau, spin) slice of G at mapped
+// k points, whole nso x nso matrices.
 __global__ void gather_g_kernel(const double2* __restrict__ G, double2* __restrict__ out,
                                 const int* __restrict__ map, int64_t nso2) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= nso2) return;
   const int64_t k = blockIdx.y;
-  out[k * nso2 + e] = G[(int64_t)map[k] * nso2 + e];
+  out[k * nso2 + e] = G[(int64_t)(map ? map[k] : (int)k) * nso2 + e];
+}
+
+// S[sidx[p]](i, j) += O[p](i, j) for nao x nao blocks (leading dimension nso, matrix stride nso2) of the
+// matrices of p = blockIdx.y; sidx is one-to-one.
+__global__ void scatter_block_add_kernel(const double2* __restrict__ O, double2* __restrict__ S,
+                                         const int* __restrict__ sidx, int nao, int64_t nso, int64_t nso2) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nao * nao) return;
+  const int64_t p = blockIdx.y;
+  double2* dst = S + (int64_t)sidx[p] * nso2 + (int64_t)(e / nao) * nso + e % nao;
+  const double2 o = O[p * nao * nao + e];
+  dst->x += o.x;
+  dst->y += o.y;
 }
 
 __global__ void zero_int_kernel(int* X, int64_t n) {

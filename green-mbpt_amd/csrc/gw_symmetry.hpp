@@ -319,16 +319,26 @@ void gw_hip_kernel::solve_star_device(const double2* G_ibz, double2* Sigma_ibz, 
   for (int64_t iq = 0; iq < inq_; ++iq)
     for (int q : qstar_[iq]) {
       const double2* Pq = star_rotate(iq, q);
-      launch_gather_rows(Vq_neg(q), star_V_, rows, NQ * nao2, ink, stream_);
+      // the irreducible points' rows of the full mesh's (p = k - q with adj, else p = k)
+      SigmaRows r = sigma_rows(q);
+      const int* km = star_km_ + (int64_t)q * ink;
+      const int* from = r.adj ? km : rows;
+      launch_gather_rows(r.V, star_V_, from, NQ * nao2, ink, stream_);
       if (split) {
-        const int64_t len = nao2 * OZ_PLANES * split_ns_ * kc_s_;  // a multiple of 64 bytes (kc_s is of 64)
-        launch_gather_rows(reinterpret_cast<const uint4*>(Vs_neg(q)), reinterpret_cast<uint4*>(star_Vs_), rows,
-                           len / 16, ink, stream_);
-        launch_gather_rows(eVs_neg(q), star_eVs_, rows, nao2, ink, stream_);
+        const int64_t len = nao2 * OZ_PLANES * split_ns_ * kc_s_;  // a multiple of 64 bytes (kc_s_ is of 64)
+        launch_gather_rows(reinterpret_cast<const uint4*>(r.Vs), reinterpret_cast<uint4*>(star_Vs_), from, len / 16,
+                           ink, stream_);
+        launch_gather_rows(r.eVs, star_eVs_, from, nao2, ink, stream_);
       }
-      sigma_q(G_dev_, Sigma_ibz, split, Pq, star_V_, star_Vs_, star_eVs_, star_km_ + (int64_t)q * ink, ink);
+      r.V = star_V_;
+      r.Vs = star_Vs_;
+      r.eVs = star_eVs_;
+      r.gidx = km;
+      r.sidx = nullptr;
+      r.n = ink;
+      sigma_q(G_dev_, Sigma_ibz, split, Pq, r);
     }
-  finish_sigma(Sigma_ibz, ink);
+  finish_sigma(Sigma_ibz, ink, split);
   if (q0_on_) apply_q0(Sigma_ibz, G_ibz, ink);  // on the irreducible points, as the reference does
   GWHIP_CHECK(hipEventRecord(t3, stream_));
   hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(64), 0, stream_, flag_, (int64_t)1);

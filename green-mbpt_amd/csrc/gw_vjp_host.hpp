@@ -97,12 +97,12 @@ void gw_hip_kernel::orb_gather_view(const OrbArgs& a, const OrbOp& op, int tz, i
   GWHIP_CHECK(hipGetLastError());
 }
 
-// X_Q = L V_Q R for the grid's (k, tz): the kernel, or (orb_gemm()) one batched GEMM over k per
+// X_Q = L V_Q R for the grid's (k, tz): the kernel, or (vjp_gemm()) one batched GEMM over k per
 // tz with the other factor gathered per k.  The GEMM form takes the shapes the VJP uses: exactly
 // one of L, R; V and X without a k map; rows (Q, r) of V and X equally spaced when R is present.
 void gw_hip_kernel::vjp_sandwich(bool has_l, bool has_r, int NB, dim3 grid, const OrbArgs& a, const OrbOp& L,
                                  const OrbOp& V, const OrbOp& R, const OrbOut& X) {
-  if (!orb_gemm()) {
+  if (!vjp_gemm()) {
     if (has_l && !has_r) launch_sandwich<true, false>(NB, grid, stream_, a, L, V, R, X);
     else if (!has_l && has_r) launch_sandwich<false, true>(NB, grid, stream_, a, L, V, R, X);
     else launch_sandwich<true, true>(NB, grid, stream_, a, L, V, R, X);
@@ -136,12 +136,12 @@ void gw_hip_kernel::vjp_sandwich(bool has_l, bool has_r, int NB, dim3 grid, cons
   }
 }
 
-// O(tz, kidx(k)) += scale sum_Q A_Q M C_Q: the kernel, or (orb_gemm()) per tz Z'_Q = M C_Q as one
+// O(tz, kidx(k)) += scale sum_Q A_Q M C_Q: the kernel, or (vjp_gemm()) per tz Z'_Q = M C_Q as one
 // batched GEMM (M gathered per k), then sum_{Q, m} A_Q(i, m) Z'_Q(m, j) as a split-K GEMM per k,
 // then added to O through the k map.  The GEMM form needs A and C without a k map.
 void gw_hip_kernel::vjp_reduce(bool has_m, int NB, dim3 grid, const OrbArgs& a, const OrbOp& A, const OrbOp& M,
                                const OrbOp& C, const OrbOut& O) {
-  if (!orb_gemm()) {
+  if (!vjp_gemm()) {
     if (has_m) launch_reduce<true>(NB, grid, stream_, a, A, M, C, O);
     else launch_reduce<false>(NB, grid, stream_, a, A, M, C, O);
     return;
@@ -335,7 +335,7 @@ void gw_hip_kernel::vjp_device(const double2* G, const double2* Sbar, double2* G
           g.alpha = make_double2(c, 0.0);
           g.accumulate = 1;
           g.conjA = 1;
-          zgemm_f64_splitk(g, zgemm_auto_ksplit(g, qchunk_ * (int64_t)dyson_per_q()), Pw_, stream_);
+          zgemm_f64_autosplit(g, nts, Pw_, (int64_t)dyson_per_q(), stream_);
         }
       }
     }

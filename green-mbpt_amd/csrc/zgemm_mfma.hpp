@@ -54,7 +54,7 @@ struct ZGemmArgs {
   int conjA, conjB;
   int upper;       // 1: skip block tiles that lie wholly below the diagonal (Hermitian products)
   int half;        // 1: K == M, A Hermitian, and a row tile [m0, m0 + BM) sums K from m0 on only, its
-                   // diagonal block weighted 1/2: U with U + U^H = A
+                   // diagonal block weighted 1/2: U with U + U^H = A (see sigma_gemm)
   int tiles_m, tiles_n;
   int64_t nblocks;   // batch * tiles_m * tiles_n * ksplit
   int64_t per_xcd;   // ceil(nblocks / 8)
@@ -368,24 +368,41 @@ inline void zgemm_f64_splitk(ZGemmArgs p, int ksplit, double2* part, hipStream_t
 // for a block's first loads and stores, and s > 1 adds writing and summing the partial products (about
 // 60 s per element) and a launch.  P0 at nk = 27, nao = 26, naux = 250 (500 upper tiles, K = 18252): one
 // slice leaves a few XCDs a second round, 9.9 ms per launch, against 6.6 ms with the three chosen here.
-// The rule looks at 64 x 64 tiles whatever the tile, so that the sums do not depend on the tile.
-inline int zgemm_auto_ksplit(const ZGemmArgs& p, int64_t part_elems) {
+// `batch` is the product's batch over a whole evaluation and the rule looks at 64 x 64 tiles, so that the
+// sums depend neither on how a call is chunked nor on the tile.
+inline int zgemm_auto_ksplit(const ZGemmArgs& p, int64_t batch, int smax) {
   const int64_t tm = ceil_div(p.M, 64), tn = ceil_div(p.N, 64);
   int64_t active = tm * tn;
   if (p.upper) {
     active = 0;
     for (int64_t i = 0; i < tm; ++i) active += std::max<int64_t>(0, tn - i);
   }
-  const double tiles = (double)active * p.batch;
+  const double tiles = (double)active * batch;
   int best = 1;
   double best_t = 0.0;
-  for (int s = 1; s <= 16; ++s) {
-    if (s > 1 && (p.K / s < 64 || (int64_t)s * p.batch * p.M * p.N > part_elems)) break;
+  for (int s = 1; s <= smax && (s == 1 || p.K / s >= 64); ++s) {
     const double t = std::ceil(tiles * s / 768.0) * ((double)p.K / s + 64.0) +
                      (s > 1 ? 60.0 * s * tiles / 768.0 + 200.0 : 0.0);
     if (s == 1 || t < best_t) best = s, best_t = t;
   }
   return best;
+}
+
+// zgemm_f64 with that number of K slices; the partial products live in part, and the batch is cut where
+// it does not hold them all (part_elems >= smax M N).
+inline void zgemm_f64_autosplit(const ZGemmArgs& p, int64_t batch, double2* part, int64_t part_elems, hipStream_t stream,
+                                int shape = 0) {
+  const int64_t mn = (int64_t)p.M * p.N;
+  const int s = zgemm_auto_ksplit(p, batch, (int)std::min<int64_t>(16, part_elems / mn));
+  const int64_t step = s > 1 ? std::max<int64_t>(1, part_elems / (s * mn)) : p.batch;
+  for (int64_t b = 0; b < p.batch; b += step) {
+    ZGemmArgs q = p;
+    q.batch = (int)std::min<int64_t>(step, p.batch - b);
+    q.A += b * p.sAb;
+    q.B += b * p.sBb;
+    q.C += b * p.sCb;
+    zgemm_f64_splitk(q, s, part, stream, shape);
+  }
 }
 
 }  // namespace gwhip
