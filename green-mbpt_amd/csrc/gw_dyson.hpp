@@ -3,8 +3,9 @@
 // compute_number_of_electrons (src/dyson.cpp:70-236):
 //   Sigma1, Sigma(tau) made Hermitian in place (make_hermitian, :183-188)
 //   Sigma(i w_n) = T_ft Sigma(tau)                                  one FP64 GEMM over all (s, k)
-//   G(i w_n) = [(i w_n + mu) S - H - Sigma1 - Sigma(i w_n)]^-1       dyson_invert_kernel, one
-//                                                                   workgroup per matrix, LDS
+//   G(i w_n) = [(i w_n + mu) S - H - Sigma1 - Sigma(i w_n)]^-1       dyson_invert_wave_kernel, a
+//                                                                   matrix per 16 to 64 lanes (nso <= 48), or
+//                                                                   dyson_invert_kernel, one per work-group;
 //                                                                   Gauss-Jordan with row pivoting
 //   G(tau) = T_tf G(i w_n)                                          one FP64 GEMM
 // The electron count N(mu) = -pref Re sum_n T_tf[nts-1][n] sum_{s,k} (w_k / nk) tr(G(i w_n; mu) S)
@@ -135,6 +136,110 @@ __global__ __launch_bounds__(256) void dyson_invert_kernel(const double2* __rest
   if (tid == 0) {
     const double f = wk[sk % ink];
     out[(int64_t)w * nsk + sk] = make_double2(f * red[0][0], f * red[1][0]);
+  }
+}
+
+// The same for n <= 48, eliminated in registers: a group of LG = 16, 32 or 64 lanes holds a matrix (64 / LG
+// matrices per wave), lane i the i-th row of M^T in N >= n registers.  M^T, because lane i then reads column i
+// of M and writes row entries next to its neighbours'; its inverse is the transpose of M^-1.  Rows are not
+// moved: step p takes as pivot row r_p the unused lane with the largest |first element| (ties: the lowest), so
+// that afterwards lane r_p, column q holds (M^T)^-1[p][r_q].  Every lane shifts its elements down by one
+// register as it eliminates, so that column p is always the first one and nothing is indexed by p.  The pivot
+// row reaches the other lanes through LDS, within the wave and without a barrier.
+// Bound: LDS reads of the pivot rows and FP64 FMAs about equally.  6400 matrices of 26 (nk = 64, 100 w_n):
+// 120 us, 242 with a work-group per matrix in LDS (two barriers and a few LDS latencies per phase of a step).
+// Above 48 the rows of a wave no longer fit its registers.
+template <int N>
+struct DysonWave {
+  static constexpr int LG = N <= 16 ? 16 : (N <= 32 ? 32 : 64), PER = 64 / LG;
+};
+
+template <int N, bool TRACE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+void dyson_invert_wave_kernel(const double2* __restrict__ HS1, const double2* __restrict__ S,
+                              const double2* __restrict__ Sw, const double* __restrict__ wn, double mu, int n, int nsk,
+                              int ink, const double* __restrict__ wk, double2* __restrict__ out, int64_t nmat) {
+  constexpr int LG = DysonWave<N>::LG, PER = DysonWave<N>::PER;
+  __shared__ double2 rows[PER][N];
+  const int lane = threadIdx.x, g = lane / LG, i = lane % LG;
+  const int64_t m0 = (int64_t)blockIdx.x * PER + g;
+  const bool live = m0 < nmat;
+  const int64_t m = live ? m0 : nmat - 1;
+  const int w = (int)(m / nsk), sk = (int)(m - (int64_t)w * nsk);
+  const int n2 = n * n, ic = i < n ? i : n - 1;
+  const double2* s = S + (int64_t)sk * n2 + ic;
+  const double2* h = HS1 + (int64_t)sk * n2 + ic;
+  const double2* x = Sw + m * n2 + ic;
+  const double zr = mu, zi = wn[w];
+  double2 a[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    a[j] = make_double2(0.0, 0.0);
+    if (j < n) {
+      const double2 sv = s[j * n], hv = h[j * n], xv = x[j * n];
+      if (i < n) a[j] = make_double2(zr * sv.x - zi * sv.y - hv.x - xv.x, zr * sv.y + zi * sv.x - hv.y - xv.y);
+    }
+  }
+  bool used = i >= n;
+  int pos = 0, rp = 0;  // this lane's step as pivot row; r_i
+  for (int p = 0; p < n; ++p) {
+    const double2 c = a[0];
+    // the high word of a double >= 0 orders like the double; its low bits make room for the lane
+    const unsigned hi = (unsigned)(__builtin_bit_cast(unsigned long long, c.x * c.x + c.y * c.y) >> 32);
+    unsigned key = used ? 0u : (hi & ~(unsigned)(LG - 1)) | (unsigned)(LG - 1 - i);
+    key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0xb1, 0xf, 0xf, true));   // lanes ^ 1
+    key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0x4e, 0xf, 0xf, true));   // lanes ^ 2
+    key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0x141, 0xf, 0xf, true));  // mirrored in 8
+    key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0x140, 0xf, 0xf, true));  // mirrored in 16
+    if (LG > 16) key = max(key, (unsigned)__shfl_xor((int)key, 16));
+    if (LG > 32) key = max(key, (unsigned)__shfl_xor((int)key, 32));
+    const int r = LG - 1 - (int)(key & (unsigned)(LG - 1));
+    if (i == p) rp = r;
+    double2* row = rows[g];
+    if (i == r) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        row[j] = a[j];
+        a[j] = make_double2(0.0, 0.0);
+      }
+      pos = p;
+      used = true;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const double2 pv = row[0];
+    const double den = pv.x * pv.x + pv.y * pv.y;
+    const double2 inv = make_double2(pv.x / den, -pv.y / den), t = cmul(c, inv);
+    // every row takes base + f (pivot row): the pivot row itself is 0 + row / pivot
+    const double2 f = i == r ? inv : make_double2(-t.x, -t.y);
+#pragma unroll
+    for (int j = 1; j < N; ++j) a[j - 1] = cfma(f, row[j], a[j]);
+    a[N - 1] = f;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  }
+  // column q of the inverse is in register q + N - n
+  double tr = 0.0, ti = 0.0;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int q = j - (N - n);
+    if (q < 0) continue;
+    const int rq = __shfl(rp, g * LG + q);
+    if (i >= n) continue;
+    const int64_t e = (int64_t)rq * n + pos;  // M^-1[r_q][pos]
+    if (TRACE) {  // times S[pos][r_q], read as its mirror image: S has been made exactly Hermitian
+      const double2 b = S[(int64_t)sk * n2 + e];
+      tr += a[j].x * b.x + a[j].y * b.y;
+      ti += a[j].y * b.x - a[j].x * b.y;
+    } else if (live) {
+      out[m * n2 + e] = a[j];
+    }
+  }
+  if (TRACE) {
+#pragma unroll
+    for (int o = LG / 2; o > 0; o >>= 1) {
+      tr += __shfl_xor(tr, o);
+      ti += __shfl_xor(ti, o);
+    }
+    if (live && i == 0) out[m] = make_double2(wk[sk % ink] * tr, wk[sk % ink] * ti);
   }
 }
 
@@ -458,8 +563,31 @@ private:
                        HS1_, S_, Sw_, wn_, mu, n, nsk, (int)d_.ink, wk_, out, Gw_);
     GWHIP_CHECK(hipGetLastError());
   }
+  template <int N, bool TRACE>
+  void launch_invert_wave(double mu, double2* out) {
+    const int nsk = (int)(d_.ns * d_.ink);
+    const int64_t nmat = d_.nw * nsk, blocks = ceil_div(nmat, DysonWave<N>::PER);
+    if (blocks > 0x3ffffff) throw status_error(GWHIP_ERR_UNSUPPORTED, "too many Dyson matrices");
+    hipLaunchKernelGGL((dyson_invert_wave_kernel<N, TRACE>), dim3((unsigned)blocks), dim3(64), 0, stream_, HS1_, S_, Sw_,
+                       wn_, mu, (int)d_.nso, nsk, (int)d_.ink, wk_, out, nmat);
+    GWHIP_CHECK(hipGetLastError());
+  }
   template <bool TRACE>
   void launch_invert(double mu, double2* out) {
+    switch ((int)ceil_div(d_.nso, 4)) {
+      case 1: return launch_invert_wave<4, TRACE>(mu, out);
+      case 2: return launch_invert_wave<8, TRACE>(mu, out);
+      case 3: return launch_invert_wave<12, TRACE>(mu, out);
+      case 4: return launch_invert_wave<16, TRACE>(mu, out);
+      case 5: return launch_invert_wave<20, TRACE>(mu, out);
+      case 6: return launch_invert_wave<24, TRACE>(mu, out);
+      case 7: return launch_invert_wave<28, TRACE>(mu, out);
+      case 8: return launch_invert_wave<32, TRACE>(mu, out);
+      case 9: return launch_invert_wave<36, TRACE>(mu, out);
+      case 10: return launch_invert_wave<40, TRACE>(mu, out);
+      case 11: return launch_invert_wave<44, TRACE>(mu, out);
+      case 12: return launch_invert_wave<48, TRACE>(mu, out);
+    }
     if (d_.nso <= DYSON_MAX_N) launch_invert_t<TRACE, false>(mu, out);
     else launch_invert_t<TRACE, true>(mu, out);
   }

@@ -119,6 +119,11 @@ gw_hip_kernel::gw_hip_kernel(const Dims& d, int device, hipStream_t shared_strea
   tchunk_p0_ = std::min<int64_t>(d_.nts / 2, tmax);
   Pw_ = dalloc<double2>((size_t)qchunk_ * dyson_per_q());
   scratch_elems_ = std::max(tchunk_sigma_, tchunk_p0_) * nk * NQ * nao2;
+  // block_inverse's panels of all matrices of a q chunk at once where that is not much memory: the orbital
+  // scratch of a small system holds them for a few matrices only (32 of 99 at nk = 1, nao = 10, naux = 154),
+  // and each batch is a chain of launches of its own
+  const int64_t nb = std::min<int64_t>(64, NQ), panels = qchunk_ * d_.nw_b * (2 * NQ * nb + nb * nb);
+  scratch_elems_ = std::max(scratch_elems_, std::min(panels, (int64_t)(0.02 * budget / sizeof(double2))));
   scratch_ = dalloc<double2>((size_t)scratch_elems_);
 }
 
@@ -744,7 +749,7 @@ void gw_hip_kernel::block_inverse(double2* X, int64_t nmat) {
   const int64_t per = 2 * n * nb + (int64_t)nb * nb;
   const int64_t mb_max = std::min<int64_t>(65535, scratch_elems_ / per);
   if (mb_max < 1) throw status_error(GWHIP_ERR_UNSUPPORTED, "scratch too small for the Dyson inverse panels");
-  const size_t gj_lds = (size_t)(GJ_NB * GJ_NB + nb * GJ_NB) * sizeof(double2);
+  static_assert(GJ_MAX_N >= 64, "gj_inverse_kernel takes the pivot blocks");
   for (int64_t m0 = 0; m0 < nmat; m0 += mb_max) {
     const int64_t mb = std::min(mb_max, nmat - m0);
     double2* A = X + m0 * n2;
@@ -757,8 +762,7 @@ void gw_hip_kernel::block_inverse(double2* X, int64_t nmat) {
       hipLaunchKernelGGL(hgj_panel_kernel, dim3((unsigned)ceil_div(n * jb, 256), (unsigned)mb), dim3(256), 0, stream_,
                          A, (int)n, n2, J0, jb, P, sP, D, sD);
       GWHIP_CHECK(hipGetLastError());
-      hipLaunchKernelGGL(gj_inverse_kernel, dim3((unsigned)mb), dim3(256), gj_lds, stream_, D, jb, sD, GJ_NB,
-                         dyson_flag_);
+      hipLaunchKernelGGL(gj_inverse_kernel, dim3((unsigned)mb), dim3(256), 0, stream_, D, jb, sD, dyson_flag_);
       GWHIP_CHECK(hipGetLastError());
       {  // Q = D^-1 P
         ZGemmArgs a{};
