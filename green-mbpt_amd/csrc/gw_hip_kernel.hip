@@ -413,6 +413,14 @@ void gw_hip_kernel::ensure_slices() {
     }
   }
   GWHIP_CHECK(hipStreamSynchronize(stream_));
+  if (!tuned_) {
+    // row-tile group of the Sigma product: with 64 x 64 tiles four row panels of A (nk = 27, nao = 26, naux = 250:
+    // 57.6 ms an evaluation, 65.8 with eight, 69.4 with sixteen)
+    tune_.p0_oz_tile = ozaki_default_tile(ns, nk, kc_p0_);
+    tune_.s_oz_tile = ozaki_default_tile(ns, 1, kc_s_);
+    tune_.s_group = 4;
+    tune_.p0_kchunks = 0;
+  }
   slices_ns_ = ns;
   ++generation_;
 }
@@ -635,11 +643,9 @@ void gw_hip_kernel::p0_gemm_split(int64_t q, int64_t tc, double2* Pt0, int group
   const int64_t nk = d_.nk, NQ = d_.NQ, NQ2 = NQ * NQ;
   const int ns = split_ns_;
   const int64_t sc = OZ_PLANES * ns * kc_p0_;  // bytes of one k chunk of a row
-  // K = nk chunks of kc: in launches over `kchunks` consecutive chunks each, the first writing C
-  // and the others adding to it, so that one launch's A and B chunks are reused from L2 by all
-  // its tiles instead of streaming the whole K past every tile (partial sums in FP64, as between
-  // chunks inside a launch).  At nk = 64, naux = 300: 770 ms per evaluation in one launch per
-  // (q, tau chunk), 604 ms with 4 chunks per launch.
+  // K = nk chunks of kc: all in one launch, K split where the tiles alone do not fill the chip, or (tuning key
+  // p0_kchunks) in launches over that many consecutive chunks each, the first writing C and the others adding
+  // to it (partial sums in FP64, as between chunks inside a launch)
   const int64_t nsl = kchunks <= 0 ? 1 : ceil_div(nk, std::min<int64_t>(kchunks, nk));
   for (int64_t sl = 0; sl < nsl; ++sl) {
     const int64_t c0 = nk * sl / nsl, c1 = nk * (sl + 1) / nsl;
@@ -655,7 +661,9 @@ void gw_hip_kernel::p0_gemm_split(int64_t q, int64_t tc, double2* Pt0, int group
     o.group_m = group;
     o.upper = g_herm_ ? 1 : 0;
     o.tile = tune_.p0_oz_tile;
-    zgemm_ozaki(o, ns, stream_);
+    // partial products in one q of the Dyson work buffer, which only stage_dyson uses
+    if (nsl == 1) zgemm_ozaki_autosplit(o, ns, d_.nts / 2, Pw_, (int64_t)dyson_per_q(), stream_);
+    else zgemm_ozaki(o, ns, stream_);
   }
 }
 
@@ -1259,6 +1267,7 @@ void gw_hip_kernel::autotune(const double2* G, int precision) {
     tune_.s_group = best_of(7, groups, [&](int c) { sigma_gemm_split(sigma_rows(0), tcs, c); });
   }
   tune_.epi_form = 1;
+  tuned_ = true;
   stored_valid_ = false;
   ++generation_;
 }

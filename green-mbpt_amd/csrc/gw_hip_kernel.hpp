@@ -35,7 +35,7 @@ struct KernelStat {
 };
 
 // Launch parameters picked by the autotuner (defaults = the best measured at nk = 64, nao = 26,
-// naux = 300): FP64 GEMM tile of the P0 and Sigma contractions (0: 64x64, 1: 128x64,
+// naux = 300; those of the int8 GEMMs by ensure_slices when the slice stores are built): FP64 GEMM tile of the P0 and Sigma contractions (0: 64x64, 1: 128x64,
 // 2: 64x128), the number of aux indices per wave of the P0 prep kernel, and for split precision
 // the row-tile group of the int8 GEMM's L2-aware tile order and whether the P0 orbital kernel
 // writes the int8 slices itself.
@@ -196,6 +196,7 @@ public:
   const Tuning& tuning() const { return tune_; }
   void set_tuning(const Tuning& t) {
     tune_ = t;
+    tuned_ = true;
     ++generation_;
   }
   void set_timing(bool on) { timing_ = on; }
@@ -227,6 +228,7 @@ private:
   };
   std::vector<Pending> pending_;  // kernel timings read once the stream has drained
   Tuning tune_;
+  bool tuned_ = false;  // set by the autotuner or the caller
   uint64_t generation_ = 0;  // bumped whenever buffers or launch parameters change
   bool g_herm_ = false;      // G of the evaluation being enqueued is Hermitian
   unsigned long long* hcheck_ = nullptr;
@@ -252,13 +254,13 @@ private:
   // per-evaluation slices of Z and P-tilde (zgemm_ozaki.hpp)
   int split_ns_ = 4, slices_ns_ = 0;
   int64_t kc_p0_ = 0, kc_s_ = 0;
-  int8_t* Vs_p0_ = nullptr;   // [nq][NQ][nk][2][ns][kc_p0]
+  int8_t* Vs_p0_ = nullptr;   // [nq][NQ][nk], 2 ns kc_p0 bytes each
   int* eVs_p0_ = nullptr;     // [nq][NQ][nk]
-  int8_t* Vs_s_ = nullptr;    // [nq][nk][nao^2][2][ns][kc_s], rows as SigmaRows
+  int8_t* Vs_s_ = nullptr;    // [nq][nk][nao^2], 2 ns kc_s bytes each, rows as SigmaRows
   int* eVs_s_ = nullptr;      // [nq][nk][nao^2]
-  int8_t* Zs_ = nullptr;      // [tc][NQ][nk][2][ns][kc_p0]  (P0 stage)
+  int8_t* Zs_ = nullptr;      // [tc][NQ][nk], 2 ns kc_p0 bytes each (P0 stage)
   int* eZs_ = nullptr;
-  int8_t* Ps_ = nullptr;      // [tc][NQ][2][ns][kc_s]       (Sigma stage; same memory as Zs_)
+  int8_t* Ps_ = nullptr;      // [tc][NQ], 2 ns kc_s bytes each    (Sigma stage; same memory as Zs_)
   int* ePs_ = nullptr;
   int64_t qchunk_ = 1, tchunk_p0_ = 1, tchunk_sigma_ = 1;
   // VJP: per-q buffers, a second orbital scratch, and the kept half-grid P0 of the last
@@ -310,7 +312,7 @@ private:
   double2* qsym_U_ = nullptr;       // [nq][NQ^2]
   double2* star_P_ = nullptr;       // [2][nts/2][NQ^2]: rotated P-tilde and U P-tilde
   double2* star_V_ = nullptr;       // [ink][NQ][nao^2]
-  int8_t* star_Vs_ = nullptr;       // [ink][nao^2][2][ns][kc_s]
+  int8_t* star_Vs_ = nullptr;       // [ink][nao^2], 2 ns kc_s bytes each
   int* star_eVs_ = nullptr;         // [ink][nao^2]
   int* star_km_ = nullptr;          // [nq][ink]
   int* star_q0row_ = nullptr;       // [inq]

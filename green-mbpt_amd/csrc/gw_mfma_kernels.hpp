@@ -139,7 +139,7 @@ struct OrbCfg {
 // NS = 0: Z in FP64.  NS > 0: straight into the NS int8 slices of the split-precision contraction, with
 // the arithmetic of slice_rows_kernel: the work-group that forms Z_Q(tau, k) owns the whole slice
 // row-chunk (row (tau, Q), chunk k, nao^2 elements), so the chunk exponent is a maximum over its lanes
-// and waves, and the digits of a quad are put together in LDS.  Slice layout: dst[((tz*NQ + Q)*nk + k)][plane][slice][kc], exps[(tz*NQ + Q)*nk + k].
+// and waves, and the digits of a quad are put together in LDS.  Slice layout: dst[((tz*NQ + Q)*nk + k)], each as in zgemm_ozaki.hpp, exps[(tz*NQ + Q)*nk + k].
 struct ZPrepArgs {
   XcdGrid xg;
   DevDims d;
@@ -329,7 +329,7 @@ void z_prep_kernel(ZPrepArgs p) {
       const int64_t task0 = ((int64_t)tz * d.NQ + 4 * qd) * d.nk + k;  // of lb = 0; the next Q is nk tasks on
       if (live && Q < d.NQ && h == 0 && (lane & 51) == 0) p.exps[task0 + (int64_t)lb * d.nk] = e;
       const double sc = ldexp(OZ_FIRST, -e);
-      // the quad's digits meet in LDS in the store's own layout ([lb][plane][slice][kc]) and leave in whole
+      // the quad's digits meet in LDS ([lb][plane][slice][kc]) and leave in the store's order, in whole
       // lines: stored straight from the lanes they are 4-byte pieces, one cache access each
       int8_t* stage = reinterpret_cast<int8_t*>(wmax + 2 * WS * QW * 4) + (size_t)qw * 4 * OZ_PLANES * NS * p.kc;
       int8_t* out = stage + lb * OZ_PLANES * NS * p.kc;
@@ -374,10 +374,10 @@ void z_prep_kernel(ZPrepArgs p) {
       if (live) {
         const int per = OZ_PLANES * NS * p.kc / 16;  // 16-byte words of one Q (kc is a multiple of 64)
         const int nw = min(4, d.NQ - 4 * qd) * per;
-        const int4* src = reinterpret_cast<const int4*>(stage);
         for (int i = h * 64 + lane; i < nw; i += 64 * WS) {
-          const int b = i / per;
-          reinterpret_cast<int4*>(p.dst + (task0 + (int64_t)b * d.nk) * OZ_PLANES * NS * p.kc)[i - b * per] = src[i];
+          const int b = i / per, w = i - b * per, ps = (w >> 1) % (OZ_PLANES * NS), ks = (w >> 1) / (OZ_PLANES * NS);
+          const int4 v = *reinterpret_cast<const int4*>(stage + (b * OZ_PLANES * NS + ps) * p.kc + 32 * ks + 16 * (w & 1));
+          reinterpret_cast<int4*>(p.dst + (task0 + (int64_t)b * d.nk) * OZ_PLANES * NS * p.kc)[w] = v;
         }
       }
     }

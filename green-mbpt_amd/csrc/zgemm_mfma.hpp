@@ -333,6 +333,12 @@ __global__ void zgemm_splitk_reduce_kernel(ZGemmArgs p, const double2* __restric
   *dst = v;
 }
 
+inline void zgemm_splitk_reduce(const ZGemmArgs& r, const double2* part, int bm, int bn, hipStream_t stream) {
+  const int64_t n = (int64_t)r.batch * r.M * r.N;
+  hipLaunchKernelGGL(zgemm_splitk_reduce_kernel, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, stream, r, part, bm, bn);
+  GWHIP_CHECK(hipGetLastError());
+}
+
 // C (+)= alpha A B with K cut into `ksplit` slices computed by separate blocks (for few, long-K
 // products); part holds ksplit * batch * M * N elements.  The slices are summed in slice order,
 // so the result does not depend on the block schedule.
@@ -357,10 +363,7 @@ inline void zgemm_f64_splitk(ZGemmArgs p, int ksplit, double2* part, hipStream_t
   ZGemmArgs r = p;
   r.ksplit = q.ksplit;
   r.sCk = q.sCk;
-  const int64_t n = (int64_t)p.batch * p.M * p.N;
-  hipLaunchKernelGGL(zgemm_splitk_reduce_kernel, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, stream, r, part,
-                     zgemm_bm(shape), zgemm_bn(shape));
-  GWHIP_CHECK(hipGetLastError());
+  zgemm_splitk_reduce(r, part, zgemm_bm(shape), zgemm_bn(shape), stream);
 }
 
 // K slices for a product whose block tiles alone would not fill the chip evenly.  Unit: K per block.

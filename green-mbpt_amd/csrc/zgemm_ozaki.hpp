@@ -14,7 +14,10 @@
 // pairs with s + t >= NS are dropped.
 //
 // Slice store (int8), for each row (A) or column (B):
-//   [chunk][plane][slice][kc]   planes Re, Im
+//   [chunk][K step of 32][plane][slice][32]   planes Re, Im
+// so that what a K step needs of a row is one contiguous piece (256 bytes at four slices, two whole cache
+// lines): with the plane-slices kc apart, each load took 32 or 64 bytes of a line, and the rest of the line
+// was fetched again for the next step.
 // (B is stored already conjugated when the contraction needs conj(B)), so
 //   Re C = Re A Re B + Im A (-Im B),   Im C = Re A Im B + Im A Re B,
 // with -Im B (32 x 64 tile) or -Im A (64 x 64 tile) negated in registers (digits lie in [-127, 127],
@@ -27,6 +30,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "zgemm_mfma.hpp"
 
 namespace gwhip {
 
@@ -34,6 +38,11 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 
 constexpr int OZ_PLANES = 2;
 constexpr double OZ_FIRST = 127.0, OZ_RADIX = 254.0;
+
+// Byte of element kk of plane-slice ps in a row's chunk (nps plane-slices).
+__host__ __device__ __forceinline__ int oz_offset(int nps, int ps, int kk) {
+  return (kk >> 5) * (nps * 32) + ps * 32 + (kk & 31);
+}
 
 // 254^{-d}, d < 8, correctly rounded
 __device__ __forceinline__ double oz_weight(int d) {
@@ -70,7 +79,7 @@ struct SliceArgs {
   int64_t s_k;
   int kc;        // padded chunk length (multiple of 64)
   int conj;      // slice conj(x)
-  int8_t* dst;   // [row][chunk][plane][slice][kc]
+  int8_t* dst;   // [row][chunk][kc / 32][plane][slice][32]
   int* exps;     // [row][chunk]
 };
 
@@ -136,8 +145,8 @@ __global__ __launch_bounds__(256) void slice_rows_kernel(SliceArgs a) {
     }
 #pragma unroll
     for (int t = 0; t < NS; ++t) {
-      *reinterpret_cast<int*>(out + (int64_t)(0 * NS + t) * a.kc + k0) = wr[t];
-      *reinterpret_cast<int*>(out + (int64_t)(1 * NS + t) * a.kc + k0) = wi[t];
+      *reinterpret_cast<int*>(out + oz_offset(OZ_PLANES * NS, t, k0)) = wr[t];
+      *reinterpret_cast<int*>(out + oz_offset(OZ_PLANES * NS, NS + t, k0)) = wi[t];
     }
   }
 }
@@ -183,9 +192,44 @@ struct OzGemmArgs {
   int64_t nblocks, per_xcd;
   int group_m;  // row tiles (over batch x M) swept together across all column tiles; 0 = heuristic
   int upper;    // 1: skip block tiles that lie wholly below the diagonal (Hermitian products)
+  int ksplit, kslice;  // > 1: slice s of the K chunks, [s kslice, (s + 1) kslice), goes to blocks of its own,
+  int64_t sCk;         // which write its partial product at C + s sCk
   int tile;     // block tile: 2 = 32 x 64 of 16 x 16 x 64 MFMAs (zgemm_ozaki_pipe_kernel), 4 = 64 x 64 of
                 // 32 x 32 x 32 MFMAs (zgemm_ozaki32_kernel); 0 = 2
 };
+
+// Logical tile of hardware block blockIdx.x in the XCD-aware, L2-grouped order: each XCD takes a
+// contiguous range of logical tiles, K slices slowest; within it, groups of group_m row tiles (rows run over
+// batch x M) sweep every column tile, row fastest, so a group's A panels stay in that XCD's L2 while the B
+// panels stream through it once per group.  Narrows p to the block's K slice.  False for the padding blocks
+// of the grid.
+__device__ __forceinline__ bool oz_tile_of(OzGemmArgs& p, int64_t& b, int& tm, int& tn) {
+  const int64_t hw = blockIdx.x;
+  int64_t logical = (hw % 8) * p.per_xcd + hw / 8;
+  if (logical >= p.nblocks) return false;
+  const int64_t rows = (int64_t)p.batch * p.tiles_m;
+  if (p.ksplit > 1) {
+    const int64_t per = rows * p.tiles_n;
+    const int s = (int)(logical / per), c0 = s * p.kslice;
+    logical -= s * per;
+    p.A += c0 * p.sAc;
+    p.B += c0 * p.sBc;
+    p.eA += c0;
+    p.eB += c0;
+    p.C += s * p.sCk;
+    p.nchunk = min(p.kslice, p.nchunk - c0);
+  }
+  const int64_t in_group = (int64_t)p.group_m * p.tiles_n;
+  const int64_t grp = logical / in_group;
+  const int64_t first = grp * p.group_m;
+  const int64_t gsize = rows - first < p.group_m ? rows - first : p.group_m;
+  const int64_t idx = logical - grp * in_group;
+  const int64_t rt = first + idx % gsize;
+  tn = (int)(idx / gsize);
+  b = rt / p.tiles_m;
+  tm = (int)(rt - b * p.tiles_m);
+  return true;
+}
 
 // Output layout of v_mfma_i32_16x16x64_i8: register r of lane l holds row
 // OZ_ROW(l/16, r), column l%16 (checked by the identity-probe test).
@@ -218,22 +262,9 @@ __global__ __launch_bounds__(256, 2) void zgemm_ozaki_pipe_kernel(OzGemmArgs p) 
   constexpr int BUF = NPS * OZ_BM * 64;
   extern __shared__ __attribute__((aligned(16))) int8_t oz_lds[];
 
-  const int64_t hw = blockIdx.x;
-  const int64_t logical = (hw % 8) * p.per_xcd + hw / 8;
-  if (logical >= p.nblocks) return;
-  // Each XCD takes a contiguous range of logical tiles; within it, groups of group_m row tiles
-  // (rows run over batch x M) sweep every column tile, row fastest, so a group's A panels stay in
-  // that XCD's L2 while the B panels stream through it once per group.
-  const int64_t rows = (int64_t)p.batch * p.tiles_m;
-  const int64_t in_group = (int64_t)p.group_m * p.tiles_n;
-  const int64_t grp = logical / in_group;
-  const int64_t first = grp * p.group_m;
-  const int64_t gsize = rows - first < p.group_m ? rows - first : p.group_m;
-  const int64_t idx = logical - grp * in_group;
-  const int64_t rt = first + idx % gsize;
-  const int tn = (int)(idx / gsize);
-  const int64_t b = rt / p.tiles_m;
-  const int tm = (int)(rt - b * p.tiles_m);
+  int64_t b;
+  int tm, tn;
+  if (!oz_tile_of(p, b, tm, tn)) return;
   const int m0 = tm * OZ_BM, n0 = tn * OZ_BN;
   if (p.upper && m0 >= n0 + OZ_BN) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -245,18 +276,18 @@ __global__ __launch_bounds__(256, 2) void zgemm_ozaki_pipe_kernel(OzGemmArgs p) 
   // stored, and unconditional loads keep the memory-counter waits of the pipeline exact (a load
   // under a per-lane branch makes the compiler wait for every load in flight).
   const int a_row = (tid >> 2) & 31, a_piece = tid & 3, a_par = (tid >> 7) & 1;
-  const int8_t* a_ptr = p.A + b * p.sAb + (int64_t)min(m0 + a_row, p.M - 1) * p.sAm + 16 * a_piece;
+  const int8_t* a_ptr = p.A + b * p.sAb + (int64_t)min(m0 + a_row, p.M - 1) * p.sAm + oz_offset(NPS, 0, 16 * a_piece);
   const int a_lds = oz_lds_off(0, OZ_BM, a_row, a_piece);
   const int bcol = min(n0 + wn + lrow, p.N - 1);
   const int8_t* b_ptr;
   {
     const int no = bcol / p.nin;
-    b_ptr = p.B + b * p.sBb + (int64_t)no * p.sBno + (int64_t)(bcol - no * p.nin) * p.sBni + 16 * lg;
+    b_ptr = p.B + b * p.sBb + (int64_t)no * p.sBno + (int64_t)(bcol - no * p.nin) * p.sBni + oz_offset(NPS, 0, 16 * lg);
   }
   const int nks = p.kc / OZ_KS, nsteps = p.nchunk * nks;
   auto b_at = [&](int g) -> const int8_t* {  // this lane's B bytes of K step g
     const int c = g / nks, ks = (g - c * nks) * OZ_KS;
-    return b_ptr + (int64_t)c * p.sBc + ks;
+    return b_ptr + (int64_t)c * p.sBc + ks * NPS;
   };
 
   // NPS = 2 NS is even, so the two parities cover every plane-slice: ps = a_par + 2 j < NPS
@@ -267,7 +298,7 @@ __global__ __launch_bounds__(256, 2) void zgemm_ozaki_pipe_kernel(OzGemmArgs p) 
 #pragma unroll
     for (int j = 0; j < NPC; ++j) {
       const int ps = a_par + 2 * j;
-      a_nx[j] = *reinterpret_cast<const v4i*>(a_ptr + (int64_t)c * p.sAc + (int64_t)ps * p.kc + ks);
+      a_nx[j] = *reinterpret_cast<const v4i*>(a_ptr + (int64_t)c * p.sAc + ps * 32 + ks * NPS);
     }
   };
   auto store_a = [&](int buf) {
@@ -320,7 +351,7 @@ __global__ __launch_bounds__(256, 2) void zgemm_ozaki_pipe_kernel(OzGemmArgs p) 
 #pragma unroll
     for (int pl = 0; pl < OZ_PLANES; ++pl)
 #pragma unroll
-      for (int t = 0; t < NS; ++t) fb[pl][t] = *reinterpret_cast<const v4i*>(bc + (int64_t)(pl * NS + t) * p.kc);
+      for (int t = 0; t < NS; ++t) fb[pl][t] = *reinterpret_cast<const v4i*>(bc + (pl * NS + t) * 32);
   }
   __syncthreads();
 
@@ -358,7 +389,7 @@ __global__ __launch_bounds__(256, 2) void zgemm_ozaki_pipe_kernel(OzGemmArgs p) 
       {
         const int t = NS - 1 - s;
 #pragma unroll
-        for (int pl = 0; pl < OZ_PLANES; ++pl) fb[pl][t] = *reinterpret_cast<const v4i*>(bn + (int64_t)(pl * NS + t) * p.kc);
+        for (int pl = 0; pl < OZ_PLANES; ++pl) fb[pl][t] = *reinterpret_cast<const v4i*>(bn + (pl * NS + t) * 32);
       }
     }
     if (!ONE && chunk_end) {
@@ -395,26 +426,6 @@ __global__ __launch_bounds__(256, 2) void zgemm_ozaki_pipe_kernel(OzGemmArgs p) 
     }
 }
 
-// Logical tile of hardware block blockIdx.x in the XCD-aware, L2-grouped order: each XCD takes a
-// contiguous range of logical tiles; within it, groups of group_m row tiles (rows run over
-// batch x M) sweep every column tile, row fastest.  False for the padding blocks of the grid.
-__device__ __forceinline__ bool oz_tile_of(const OzGemmArgs& p, int64_t& b, int& tm, int& tn) {
-  const int64_t hw = blockIdx.x;
-  const int64_t logical = (hw % 8) * p.per_xcd + hw / 8;
-  if (logical >= p.nblocks) return false;
-  const int64_t rows = (int64_t)p.batch * p.tiles_m;
-  const int64_t in_group = (int64_t)p.group_m * p.tiles_n;
-  const int64_t grp = logical / in_group;
-  const int64_t first = grp * p.group_m;
-  const int64_t gsize = rows - first < p.group_m ? rows - first : p.group_m;
-  const int64_t idx = logical - grp * in_group;
-  const int64_t rt = first + idx % gsize;
-  tn = (int)(idx / gsize);
-  b = rt / p.tiles_m;
-  tm = (int)(rt - b * p.tiles_m);
-  return true;
-}
-
 // ------------------------------------------------------------------------------ 32 x 32 x 32 tile
 // Output layout of v_mfma_i32_32x32x32_i8: register r of lane l holds row OZ32_ROW(l/32, r),
 // column l%32 (checked by the identity-probe test); each operand lane l holds row (A) / column (B)
@@ -431,76 +442,86 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 // Operands go to LDS by direct global -> LDS loads (global_load_lds_dwordx4), double-buffered in two
 // static arrays (distinct objects, so a wave reads one while the loads into the other are in
 // flight); the loads of K step g + 1 leave at the start of step g, and the barrier closing step g
-// waits for them.  A stage is a list of 1 KB chunks -- A's (row block of 32, plane-slice), then B's
-// (column block of 32, plane-slice) -- each in MFMA fragment order, so one wave-wide load fills a
-// chunk and a fragment read is one contiguous ds_read_b128 per lane.  Waves 0-1 load A's row blocks,
-// waves 2-3 B's column blocks.  Rows past M / columns past N load the last valid row / column: they
-// only feed results that are never stored.  Two blocks per CU.
+// waits for them.  A stage holds the 64 rows of A, then the 64 columns of B, each with all its
+// plane-slices of the K step (2 NPS pieces of 16 bytes, as stored), so that a wave-wide load covers whole
+// cache lines; row r has its pieces permuted by XOR with sigma(r), which spreads the 16 rows of a fragment
+// read over all banks.  Rows past M / columns past N load the last valid row / column: they
+// only feed results that are never stored.  Two blocks per CU: what a CU loads per product is half of the
+// 32 x 64 tile's.  ONE: a single K chunk, converted to FP64 after the loop.
 constexpr int OZ32_BM = 64, OZ32_BN = 64, OZ32_KS = 32;
 
-template <int NS>
+template <int NS, bool ONE>
 __global__ __launch_bounds__(256, 2) void zgemm_ozaki32_kernel(OzGemmArgs p) {
-  constexpr int NPU = 2 * NS;                   // plane-slices read: Re and Im
-  constexpr int STAGE = 4 * NPU * 1024;         // 2 row blocks + 2 column blocks, NPU chunks each
-  __shared__ __attribute__((aligned(1024))) int8_t oz_s0[STAGE];
-  __shared__ __attribute__((aligned(1024))) int8_t oz_s1[STAGE];
+  constexpr int NPS = OZ_PLANES * NS, NP = 2 * NPS;  // plane-slices and 16-byte pieces of a row
+  constexpr int ROWB = 32 * NPS;                     // bytes of a row in a stage
+  constexpr int NLD = OZ32_BM * NP / 256;            // loads per thread and operand
+  static_assert(OZ32_BM * NP % 256 == 0 && OZ32_BM == OZ32_BN, "whole loads");
+  __shared__ __attribute__((aligned(1024))) int8_t oz_s0[2 * OZ32_BM * ROWB];
+  __shared__ __attribute__((aligned(1024))) int8_t oz_s1[2 * OZ32_BM * ROWB];
 
   int64_t b;
   int tm, tn;
   if (!oz_tile_of(p, b, tm, tn)) return;
   const int m0 = tm * OZ32_BM, n0 = tn * OZ32_BN;
   if (p.upper && m0 >= n0 + OZ32_BN) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, lg = lane >> 5;
   const int wm = wave & 1, wn = wave >> 1;  // rows 32 wm .. +32, columns 32 wn .. +32
+  // the row stride is a multiple of all 64 banks at eight plane-slices, of 16 at six and ten
+  auto sigma = [](int row) { return NPS == 8 ? row & 15 : (row >> 2) & 3; };
 
-  // this lane's source row (waves 0-1: A row block `wave`) or column (waves 2-3: B column block)
-  const bool loads_a = wave < 2;
-  const int blk = wave & 1;
-  const int8_t* src;
-  int64_t s_chunk;
-  if (loads_a) {
-    const int m = min(m0 + 32 * blk + l32, p.M - 1);
-    src = p.A + b * p.sAb + (int64_t)m * p.sAm + 16 * lg;
-    s_chunk = p.sAc;
-  } else {
-    const int n = min(n0 + 32 * blk + l32, p.N - 1);
-    const int no = n / p.nin;
-    src = p.B + b * p.sBb + (int64_t)no * p.sBno + (int64_t)(n - no * p.nin) * p.sBni + 16 * lg;
-    s_chunk = p.sBc;
+  // this thread's pieces of a stage, as byte offsets from the first row / column of the tile
+  const int no0 = n0 / p.nin;
+  const int64_t col0 = (int64_t)no0 * p.sBno + (int64_t)(n0 - no0 * p.nin) * p.sBni;
+  const int8_t* abase = p.A + b * p.sAb + (int64_t)m0 * p.sAm;
+  const int8_t* bbase = p.B + b * p.sBb + col0;
+  unsigned aoff[NLD], boff[NLD];
+#pragma unroll
+  for (int j = 0; j < NLD; ++j) {
+    const int idx = j * 256 + tid, row = idx / NP, piece = (idx - row * NP) ^ sigma(row);
+    aoff[j] = (unsigned)((int64_t)(min(m0 + row, p.M - 1) - m0) * p.sAm) + 16 * piece;
+    const int n = min(n0 + row, p.N - 1), no = n / p.nin;
+    boff[j] = (unsigned)((int64_t)no * p.sBno + (int64_t)(n - no * p.nin) * p.sBni - col0) + 16 * piece;
   }
-  const int chunk0 = (loads_a ? 0 : 2 * NPU) + blk * NPU;  // first of this wave's NPU chunks
   const int nks = p.kc / OZ32_KS, nsteps = p.nchunk * nks;
   auto load_stage = [&](int8_t* st, int g) {
-    const int c = g / nks, ks = (g - c * nks) * OZ32_KS;
-    const int8_t* s0 = src + (int64_t)c * s_chunk + ks;
+    const int c = g / nks, ks = (g - c * nks) * ROWB;
+    const int8_t* a0 = abase + (int64_t)c * p.sAc + ks;
+    const int8_t* b0 = bbase + (int64_t)c * p.sBc + ks;
 #pragma unroll
-    for (int ps = 0; ps < NPU; ++ps)
-      __builtin_amdgcn_global_load_lds((const void*)(s0 + (int64_t)ps * p.kc),
-                                       (__attribute__((address_space(3))) void*)(st + (chunk0 + ps) * 1024), 16, 0, 0);
+    for (int j = 0; j < NLD; ++j)
+      __builtin_amdgcn_global_load_lds((const void*)(a0 + aoff[j]),
+                                       (__attribute__((address_space(3))) void*)(st + (j * 256 + wave * 64) * 16), 16, 0, 0);
+#pragma unroll
+    for (int j = 0; j < NLD; ++j)
+      __builtin_amdgcn_global_load_lds((const void*)(b0 + boff[j]),
+                                       (__attribute__((address_space(3))) void*)(st + OZ32_BM * ROWB + (j * 256 + wave * 64) * 16),
+                                       16, 0, 0);
   };
 
-  double cr[16], ci[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) { cr[r] = 0.0; ci[r] = 0.0; }
   v16i ar[NS], ai[NS];  // [d] int32 accumulators (Re, Im) of slice level d
+  double cr[16], ci[16];
 #pragma unroll
   for (int d = 0; d < NS; ++d)
 #pragma unroll
     for (int r = 0; r < 16; ++r) { ar[d][r] = 0; ai[d][r] = 0; }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) { cr[r] = 0.0; ci[r] = 0.0; }
 
-  const int bcol = min(n0 + 32 * wn + l32, p.N - 1);
-  auto compute = [&](const int8_t* st, int g) {
+  const int sg = sigma(l32);
+  const int arow = (32 * wm + l32) * ROWB, brow = (OZ32_BM + 32 * wn + l32) * ROWB;
+  auto compute = [&](const int8_t* st) {
     v4i fb[2][NS];
 #pragma unroll
     for (int pl = 0; pl < 2; ++pl)
 #pragma unroll
       for (int t = 0; t < NS; ++t)
-        fb[pl][t] = *reinterpret_cast<const v4i*>(st + (2 * NPU + wn * NPU + pl * NS + t) * 1024 + 16 * lane);
+        fb[pl][t] = *reinterpret_cast<const v4i*>(st + brow + 16 * ((2 * (pl * NS + t) + lg) ^ sg));
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-      const v4i fa_r = *reinterpret_cast<const v4i*>(st + (wm * NPU + 0 * NS + s) * 1024 + 16 * lane);
-      const v4i fa_i = *reinterpret_cast<const v4i*>(st + (wm * NPU + 1 * NS + s) * 1024 + 16 * lane);
+      const v4i fa_r = *reinterpret_cast<const v4i*>(st + arow + 16 * ((2 * s + lg) ^ sg));
+      const v4i fa_i = *reinterpret_cast<const v4i*>(st + arow + 16 * ((2 * (NS + s) + lg) ^ sg));
       const v4i fa_n = neg_i8x16(fa_i);
 #pragma unroll
       for (int t = 0; t + s < NS; ++t) {
@@ -510,42 +531,53 @@ __global__ __launch_bounds__(256, 2) void zgemm_ozaki32_kernel(OzGemmArgs p) {
         ai[s + t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa_i, fb[0][t], ai[s + t], 0, 0, 0);
       }
     }
-    const int c = g / nks;
-    if (g - c * nks == nks - 1) {  // chunk end: int32 -> FP64 with the scale 2^(ea + eb) / 127^2
-      const int no = bcol / p.nin;
-      const int eb = p.eB[b * p.seBb + (int64_t)no * p.seBno + (int64_t)(bcol - no * p.nin) * p.seBni + c];
+  };
+  const int bcol = min(n0 + 32 * wn + l32, p.N - 1);
+  auto convert = [&](int c) {  // chunk end: int32 -> FP64 with the scale 2^(ea + eb) / 127^2
+    const int no = bcol / p.nin;
+    const int eb = p.eB[b * p.seBb + (int64_t)no * p.seBno + (int64_t)(bcol - no * p.nin) * p.seBni + c];
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = min(m0 + 32 * wm + OZ32_ROW(lg, r), p.M - 1);
-        const int ea = p.eA[b * p.seAb + (int64_t)m * p.seAm + c];
-        double sr = 0.0, si = 0.0;
+    for (int r = 0; r < 16; ++r) {
+      const int m = min(m0 + 32 * wm + OZ32_ROW(lg, r), p.M - 1);
+      const int ea = p.eA[b * p.seAb + (int64_t)m * p.seAm + c];
+      double sr = 0.0, si = 0.0;
 #pragma unroll
-        for (int d = 0; d < NS; ++d) {  // exact integers times 254^-d
-          sr = fma((double)ar[d][r], oz_weight(d), sr);
-          si = fma((double)ai[d][r], oz_weight(d), si);
-        }
-        const double sc = ldexp(1.0 / (OZ_FIRST * OZ_FIRST), ea + eb);
-        cr[r] = fma(sr, sc, cr[r]);
-        ci[r] = fma(si, sc, ci[r]);
+      for (int d = 0; d < NS; ++d) {  // exact integers times 254^-d
+        sr = fma((double)ar[d][r], oz_weight(d), sr);
+        si = fma((double)ai[d][r], oz_weight(d), si);
       }
-#pragma unroll
-      for (int d = 0; d < NS; ++d)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) { ar[d][r] = 0; ai[d][r] = 0; }
+      const double sc = ldexp(1.0 / (OZ_FIRST * OZ_FIRST), ea + eb);
+      cr[r] = fma(sr, sc, cr[r]);
+      ci[r] = fma(si, sc, ci[r]);
     }
+  };
+  auto chunk_end = [&](int g) {
+    if (ONE) return;
+    const int c = g / nks;
+    if (g - c * nks != nks - 1) return;
+    convert(c);
+#pragma unroll
+    for (int d = 0; d < NS; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) { ar[d][r] = 0; ai[d][r] = 0; }
+  };
+  auto close = [&]() {  // this wave's loads have landed, and every wave is done with the other buffer
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
   };
 
   load_stage(oz_s0, 0);
-  __syncthreads();
-  for (int g = 0; g < nsteps; g += 2) {
-    if (g + 1 < nsteps) load_stage(oz_s1, g + 1);
-    compute(oz_s0, g);
-    __syncthreads();
-    if (g + 1 >= nsteps) break;
+  close();
+  for (int g = 0; g < nsteps; g += 2) {  // kc is a multiple of 64: an even number of K steps
+    load_stage(oz_s1, g + 1);
+    compute(oz_s0);
+    close();
     if (g + 2 < nsteps) load_stage(oz_s0, g + 2);
-    compute(oz_s1, g + 1);
-    __syncthreads();
+    compute(oz_s1);
+    chunk_end(g + 1);
+    close();
   }
+  if (ONE) convert(0);
 
   const int n = n0 + 32 * wn + l32;
   if (n >= p.N) return;
@@ -581,7 +613,8 @@ inline size_t ozaki_pipe_lds_bytes(int ns) { return (size_t)2 * OZ_PLANES * OZ_B
 template <int NS>
 inline void ozaki_launch(const OzGemmArgs& p, int64_t grid, hipStream_t stream) {
   if (p.tile == 4) {
-    hipLaunchKernelGGL(zgemm_ozaki32_kernel<NS>, dim3((unsigned)grid), dim3(256), 0, stream, p);
+    if (p.nchunk == 1) hipLaunchKernelGGL((zgemm_ozaki32_kernel<NS, true>), dim3((unsigned)grid), dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((zgemm_ozaki32_kernel<NS, false>), dim3((unsigned)grid), dim3(256), 0, stream, p);
     return;
   }
   const size_t lds = ozaki_pipe_lds_bytes(NS);
@@ -594,6 +627,13 @@ inline void ozaki_launch(const OzGemmArgs& p, int64_t grid, hipStream_t stream) 
   }
 }
 
+// The 64 x 64 tile keeps a tile's offsets in 32 bits.
+inline bool ozaki32_fits(const OzGemmArgs& p) {
+  if (p.N > p.nin && p.sBno < (int64_t)p.nin * p.sBni) return false;
+  const int64_t span = (OZ32_BN / p.nin + 1) * p.sBno + std::min(OZ32_BN, p.nin) * p.sBni;
+  return p.sAm >= 0 && p.sBni >= 0 && std::max(OZ32_BM * p.sAm, p.N > p.nin ? span : OZ32_BN * p.sBni) < ((int64_t)1 << 32);
+}
+
 inline bool ozaki_tile_valid(int tile) { return tile == 2 || tile == 4; }
 
 inline void zgemm_ozaki(OzGemmArgs p, int ns, hipStream_t stream) {
@@ -602,9 +642,15 @@ inline void zgemm_ozaki(OzGemmArgs p, int ns, hipStream_t stream) {
   if (p.kc > split_kc_limit(ns)) throw std::runtime_error("zgemm_ozaki: chunk too long for exact int32 sums");
   if (p.tile == 0) p.tile = 2;
   if (!ozaki_tile_valid(p.tile)) throw std::runtime_error("zgemm_ozaki: unknown block tile");
+  if (p.tile == 4 && !ozaki32_fits(p)) p.tile = 2;
   p.tiles_m = (int)ceil_div(p.M, p.tile == 4 ? OZ32_BM : OZ_BM);
   p.tiles_n = (int)ceil_div(p.N, p.tile == 4 ? OZ32_BN : OZ_BN);
   p.nblocks = (int64_t)p.batch * p.tiles_m * p.tiles_n;
+  if (p.ksplit > 1) {
+    if (p.kslice < 1 || (int64_t)(p.ksplit - 1) * p.kslice >= p.nchunk || (int64_t)p.ksplit * p.kslice < p.nchunk)
+      throw std::runtime_error("zgemm_ozaki: bad K split");
+    p.nblocks *= p.ksplit;
+  }
   if (p.group_m <= 0) p.group_m = ozaki_default_group(p.tiles_n);
   p.group_m = (int)std::min<int64_t>(p.group_m, (int64_t)p.batch * p.tiles_m);
   p.per_xcd = ceil_div(p.nblocks, 8);
@@ -615,6 +661,75 @@ inline void zgemm_ozaki(OzGemmArgs p, int ns, hipStream_t stream) {
   else if (ns == 3) ozaki_launch<3>(p, grid, stream);
   else throw std::runtime_error("zgemm_ozaki: slices must be 3, 4 or 5");
   GWHIP_CHECK(hipGetLastError());
+}
+
+// K slices for a product whose tiles alone do not fill the chip evenly.  In microseconds: s slices take
+// ceil(tiles s / 512) rounds (two blocks per CU) of the K steps of nchunk / s chunks, 2 each, plus 4 for a block's
+// first loads and stores; s > 1 adds a launch (12 with its gap) and the partial products of a tile, written and
+// summed (0.033).  Only for a gain of 15 % or more, and decided on 64 x 64 tiles and the whole batch, so that the
+// sums depend neither on how a call is chunked nor on the tile.  P0 per launch: nk = 64, nao = 12, naux = 100 (150
+// upper tiles of 6 K steps a chunk) 0.72 -> 0.49 ms; nk = 27, nao = 18, naux = 160 (300 of 12) 0.87 -> 0.56;
+// nk = 27, nao = 26, naux = 250 (500 of 22) keeps one slice.
+inline int ozaki_auto_ksplit(const OzGemmArgs& p, int64_t batch, int smax) {
+  const int64_t tm = ceil_div(p.M, 64), tn = ceil_div(p.N, 64);
+  int64_t active = tm * tn;
+  if (p.upper) {
+    active = 0;
+    for (int64_t i = 0; i < tm; ++i) active += std::max<int64_t>(0, tn - i);
+  }
+  const double tiles = (double)active * batch, chunk = 2.0 * p.kc / OZ32_KS;
+  int best = 1;
+  double best_t = 0.0;
+  for (int s = 1; s <= std::min(smax, p.nchunk); ++s) {
+    const int64_t slice = ceil_div(p.nchunk, s);
+    if (ceil_div(p.nchunk, slice) != s) continue;
+    const double t = std::ceil(tiles * s / 512.0) * (slice * chunk + 4.0) + (s > 1 ? 12.0 + 0.033 * tiles * s : 0.0);
+    if (s == 1) best_t = 0.85 * t;
+    else if (t < best_t) best = s, best_t = t;
+  }
+  return best;
+}
+
+// Block tile of a product of nchunk chunks of kc.  One chunk: 64 x 64 (nk = 27, nao = 26, naux = 250, five slices 99 ->
+// 84 ms an evaluation, four 77 -> 58, three 55 -> 39).  More: its FP64 sums spill to scratch once a chunk, which long
+// chunks hide at three slices always (51.6 -> 44.5), at four from about 640 on (kc = 704: 81 -> 68 ms; 1600: 12.3 ->
+// 11.4; but 384: 15.2 against 16.3 and 192: 31 against 49), at five never (102 against 119).
+inline int ozaki_default_tile(int ns, int64_t nchunk, int64_t kc) {
+  return nchunk == 1 || ns == 3 || (ns == 4 && kc >= 640) ? 4 : 2;
+}
+
+// zgemm_ozaki with that number of K slices; the partial products live in part (part_elems elements), and the
+// batch is cut where it does not hold them all.
+inline void zgemm_ozaki_autosplit(const OzGemmArgs& p, int ns, int64_t batch, double2* part, int64_t part_elems,
+                                  hipStream_t stream) {
+  const int64_t mn = (int64_t)p.M * p.N;
+  const int s = ozaki_auto_ksplit(p, batch, (int)std::min<int64_t>(16, part_elems / mn));
+  if (s < 2) {
+    zgemm_ozaki(p, ns, stream);
+    return;
+  }
+  const int64_t step = std::max<int64_t>(1, part_elems / (s * mn));
+  for (int64_t b = 0; b < p.batch; b += step) {
+    OzGemmArgs q = p;
+    q.batch = (int)std::min<int64_t>(step, p.batch - b);
+    q.A += b * p.sAb;
+    q.eA += b * p.seAb;
+    q.B += b * p.sBb;
+    q.eB += b * p.seBb;
+    ZGemmArgs r{};
+    r.M = p.M; r.N = p.N; r.batch = q.batch; r.nin = p.nin;
+    r.C = p.C + b * p.sCb; r.sCb = p.sCb; r.sCm = p.sCm; r.sCno = p.sCno; r.sCni = p.sCni;
+    r.alpha = p.alpha; r.accumulate = p.accumulate; r.upper = p.upper;
+    r.ksplit = s; r.sCk = q.batch * mn;
+    q.kslice = (int)ceil_div(p.nchunk, s);
+    q.ksplit = s;
+    q.C = part; q.sCk = r.sCk; q.sCb = mn; q.sCm = p.N; q.sCno = p.nin; q.sCni = 1;
+    q.alpha = make_double2(1.0, 0.0);
+    q.accumulate = 0;
+    zgemm_ozaki(q, ns, stream);
+    // tiles of 64 x 64 that `upper` skips are skipped by the 32 x 64 tile too
+    zgemm_splitk_reduce(r, part, 64, 64, stream);
+  }
 }
 
 inline void slice_rows(const SliceArgs& a, int ns, hipStream_t stream) {

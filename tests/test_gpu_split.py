@@ -256,3 +256,30 @@ def test_fused_slicing_two_spin_blocks(nao):
           f"{rel_err(out[1], out[0]):.2e}", flush=True)
     assert max(errs) < 1e-8
     assert rel_err(out[1], out[0]) < 1e-9
+
+
+@pytest.mark.parametrize("ns", [3, 4, 5])
+@pytest.mark.parametrize("nao,NQ", [(20, 70), (27, 33)])
+def test_k_split_of_p0(ns, nao, NQ):
+    """P0 with its K chunks split over blocks (few tiles, eight chunks), in the chosen and in both block tiles,
+    against one launch per chunk: the same exact chunk sums added in FP64 in another order, so the products
+    agree to a few roundings of FP64 (1e-15 times the condition of I - P0), and the oracle.  nao = 27: every
+    row of a chunk ends inside a K step of 32, at any element."""
+    G, V, T, d = synthetic(8, nao, NQ, beta=20.0, lam=1e3, mesh=(2, 2, 2), seed=5, sigma=0.5 / nao)
+    out = []
+    for tune in (dict(), dict(p0_kchunks=1), dict(p0_kchunks=0, p0_split_tile=2), dict(p0_kchunks=0, p0_split_tile=4)):
+        k = _kernel(d, T)
+        try:
+            k.set_grid(T.T_bt, T.T_tb)
+            k.upload_V(V)
+            k.set_split_slices(ns)
+            if tune:
+                k.set_tuning(**tune)
+            out.append(k.solve(G, gl.PREC_SPLIT))
+        finally:
+            k.close()
+    S_ref = go.gw_sigma(G, V, T.T_bt, T.T_tb, d["nk"], d["nao"], d["nso"], d["ns"], d["NQ"], mesh=d["mesh"])
+    errs = [rel_err(o, S_ref) for o in out]
+    print(f"ns={ns} nao={nao}: vs oracle {errs}, vs one launch per chunk {[rel_err(o, out[1]) for o in out]}", flush=True)
+    assert max(errs) < {3: 1e-4, 4: TOL_SPLIT, 5: 1e-10}[ns]
+    assert max(rel_err(o, out[1]) for o in out) < 1e-12
