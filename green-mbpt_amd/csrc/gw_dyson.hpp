@@ -139,108 +139,181 @@ __global__ __launch_bounds__(256) void dyson_invert_kernel(const double2* __rest
   }
 }
 
-// The same for n <= 48, eliminated in registers: a group of LG = 16, 32 or 64 lanes holds a matrix (64 / LG
-// matrices per wave), lane i the i-th row of M^T in N >= n registers.  M^T, because lane i then reads column i
-// of M and writes row entries next to its neighbours'; its inverse is the transpose of M^-1.  Rows are not
-// moved: step p takes as pivot row r_p the unused lane with the largest |first element| (ties: the lowest), so
-// that afterwards lane r_p, column q holds (M^T)^-1[p][r_q].  Every lane shifts its elements down by one
-// register as it eliminates, so that column p is always the first one and nothing is indexed by p.  The pivot
-// row reaches the other lanes through LDS, within the wave and without a barrier.
-// Bound: LDS reads of the pivot rows and FP64 FMAs about equally.  6400 matrices of 26 (nk = 64, 100 w_n):
-// 120 us, 242 with a work-group per matrix in LDS (two barriers and a few LDS latencies per phase of a step).
-// Above 48 the rows of a wave no longer fit its registers.
+// The same for n <= 48, eliminated in registers: RG = 16, 32 or 64 lanes, one per row of M^T padded by the
+// identity to N >= n, or twice as many that hold C = N / 2 columns each (n <= 32).  M^T, because lane i then reads
+// column i of M and writes row entries next to its neighbours'; its inverse is the transpose of M^-1.  Rows are
+// not moved: the step of column q takes as pivot row r_q the unused row with the largest |element q| (ties: the
+// lowest), so that afterwards row r_q, column q' holds (M^T)^-1[q][q'] with q' counted in pivot order: M^-1 at
+// [r_q'][q].  A round eliminates two columns of each half and rotates the registers by two, so that nothing is
+// indexed by the step.  The pivot row goes through LDS within the wave, without a barrier, and comes back as one
+// element per lane and 16 columns, from where the multiply-adds take it by DPP (row_newbcast).
+// With `paired` (w_n and -w_n at mirrored places of the grid, T_ft conjugate there; the caller has checked both to
+// the bit) only w_n > 0 is inverted, nw / 2 of them from nw / 2 on: M(-i w) = M(i w)^H, as S, H and Sigma(tau) are
+// Hermitian.
+// Bound: the chain of pivots, of which the pivot lane's LDS writes and the multiply-adds are the longest parts;
+// two lanes per row halve both.  6272 matrices of 26 (nk = 64, 98 w_n, traces): 58 us; 71 with a lane per row, 119
+// with the pivot row read by broadcast and every w_n inverted, 242 with a work-group per matrix in LDS (two
+// barriers and a few LDS latencies per phase of a step).  Above 48 the rows no longer fit the registers.
 template <int N>
 struct DysonWave {
-  static constexpr int LG = N <= 16 ? 16 : (N <= 32 ? 32 : 64), PER = 64 / LG;
+  static constexpr int RG = N <= 16 ? 16 : (N <= 32 ? 32 : 64), H = N <= 32 ? 2 : 1, LG = RG * H, PER = 64 / LG, C = N / H;
 };
 
+// a[j] += f x, x = element J of the 16 that the lanes of a DPP row hold; two j at a time.  nfy = -f.y.  The wait
+// covers a value of x written by a vector instruction right before (DPP reads need two states).
+template <int J>
+__device__ __forceinline__ void fmac_bcast2(double2& a0, double2& a1, double2 x, double2 f, double nfy) {
+  asm("s_nop 1\n"
+      "v_fmac_f64_dpp %0, %4, %6 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %5, %6 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %2, %4, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %3, %5, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %5, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %4, %7 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %2, %5, %8 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %3, %4, %7 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n"
+      : "+v"(a0.x), "+v"(a0.y), "+v"(a1.x), "+v"(a1.y)
+      : "v"(x.x), "v"(x.y), "v"(f.x), "v"(f.y), "v"(nfy), "n"(J), "n"(J + 1));
+}
+template <int C, int J>
+__device__ __forceinline__ void fmac_bcast_row(double2 (&a)[C], const double2 (&x)[(C + 15) / 16], double2 f, double nfy) {
+  fmac_bcast2<J % 16>(a[J], a[J + 1], x[J / 16], f, nfy);
+  if constexpr (J + 2 < C) fmac_bcast_row<C, J + 2>(a, x, f, nfy);
+}
 template <int N, bool TRACE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 void dyson_invert_wave_kernel(const double2* __restrict__ HS1, const double2* __restrict__ S,
                               const double2* __restrict__ Sw, const double* __restrict__ wn, double mu, int n, int nsk,
-                              int ink, const double* __restrict__ wk, double2* __restrict__ out, int64_t nmat) {
-  constexpr int LG = DysonWave<N>::LG, PER = DysonWave<N>::PER;
-  __shared__ double2 rows[PER][N];
-  const int lane = threadIdx.x, g = lane / LG, i = lane % LG;
-  const int64_t m0 = (int64_t)blockIdx.x * PER + g;
+                              int ink, const double* __restrict__ wk, double2* __restrict__ out, int nw, int paired) {
+  constexpr int RG = DysonWave<N>::RG, H = DysonWave<N>::H, LG = DysonWave<N>::LG, PER = DysonWave<N>::PER;
+  constexpr int C = DysonWave<N>::C, NX = (C + 15) / 16;
+  static_assert(C % 2 == 0, "columns go two at a time");
+  __shared__ double2 rows[PER][N + 16];
+  const int lane = threadIdx.x, g = lane / LG, i = lane % RG, hl = lane / RG % H;
+  const int w0 = paired ? nw / 2 : 0;
+  const int64_t nmat = (int64_t)(nw - w0) * nsk, m0 = (int64_t)blockIdx.x * PER + g;
   const bool live = m0 < nmat;
-  const int64_t m = live ? m0 : nmat - 1;
-  const int w = (int)(m / nsk), sk = (int)(m - (int64_t)w * nsk);
-  const int n2 = n * n, ic = i < n ? i : n - 1;
-  const double2* s = S + (int64_t)sk * n2 + ic;
-  const double2* h = HS1 + (int64_t)sk * n2 + ic;
-  const double2* x = Sw + m * n2 + ic;
+  const int64_t ml = live ? m0 : nmat - 1;
+  const int w = w0 + (int)(ml / nsk), sk = (int)(ml % nsk);
+  const int64_t m = (int64_t)w * nsk + sk, mp = (int64_t)(nw - 1 - w) * nsk + sk;
+  const int n2 = n * n, ic = min(i, n - 1);
+  // M[hl C + j][i] by 32-bit offsets, Sw from the wave's first matrix on
+  const int64_t first = (int64_t)w0 * nsk + (int64_t)blockIdx.x * PER;
+  const __amdgpu_buffer_rsrc_t sres = buf_rsrc(S, (int64_t)nsk * n2), hres = buf_rsrc(HS1, (int64_t)nsk * n2),
+                               xres = buf_rsrc(Sw + first * n2, min((int64_t)PER, (int64_t)nw * nsk - first) * n2);
+  const int step = n * (int)sizeof(double2);
+  const int so = (sk * n2 + ic) * (int)sizeof(double2), xo = ((int)(m - first) * n2 + ic) * (int)sizeof(double2);
   const double zr = mu, zi = wn[w];
-  double2 a[N];
+  double2 a[C];
 #pragma unroll
-  for (int j = 0; j < N; ++j) {
-    a[j] = make_double2(0.0, 0.0);
-    if (j < n) {
-      const double2 sv = s[j * n], hv = h[j * n], xv = x[j * n];
-      if (i < n) a[j] = make_double2(zr * sv.x - zi * sv.y - hv.x - xv.x, zr * sv.y + zi * sv.x - hv.y - xv.y);
-    }
+  for (int j = 0; j < C; ++j) a[j] = buf_load_z(xres, xo + min(hl * C + j, n - 1) * step);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < C; ++j) {
+    const int e = so + min(hl * C + j, n - 1) * step;
+    const double2 sv = buf_load_z(sres, e), hv = buf_load_z(hres, e);
+    a[j] = make_double2(zr * sv.x - zi * sv.y - hv.x - a[j].x, zr * sv.y + zi * sv.x - hv.y - a[j].y);
+    if (i >= n || hl * C + j >= n) a[j] = make_double2(i == hl * C + j ? 1.0 : 0.0, 0.0);
+    if (j % 8 == 7) __builtin_amdgcn_sched_barrier(0);
   }
-  bool used = i >= n;
-  int pos = 0, rp = 0;  // this lane's step as pivot row; r_i
-  for (int p = 0; p < n; ++p) {
-    const double2 c = a[0];
-    // the high word of a double >= 0 orders like the double; its low bits make room for the lane
-    const unsigned hi = (unsigned)(__builtin_bit_cast(unsigned long long, c.x * c.x + c.y * c.y) >> 32);
-    unsigned key = used ? 0u : (hi & ~(unsigned)(LG - 1)) | (unsigned)(LG - 1 - i);
-    key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0xb1, 0xf, 0xf, true));   // lanes ^ 1
-    key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0x4e, 0xf, 0xf, true));   // lanes ^ 2
-    key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0x141, 0xf, 0xf, true));  // mirrored in 8
-    key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0x140, 0xf, 0xf, true));  // mirrored in 16
-    if (LG > 16) key = max(key, (unsigned)__shfl_xor((int)key, 16));
-    if (LG > 32) key = max(key, (unsigned)__shfl_xor((int)key, 32));
-    const int r = LG - 1 - (int)(key & (unsigned)(LG - 1));
-    if (i == p) rp = r;
-    double2* row = rows[g];
-    if (i == r) {
+  double2* const row = rows[g];
+  bool used = i >= N;
+  int pos = 0, rp = 0;  // the column this row was the pivot row of; r_i
+#pragma unroll 1
+  for (int pb = 0; pb < C; pb += 2) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) {
-        row[j] = a[j];
-        a[j] = make_double2(0.0, 0.0);
+    for (int hu = 0; hu < 2 * H; ++hu) {
+      const int h = hu / 2, u = hu % 2, q = h * C + pb + u;  // register u of half h holds column q
+      double2 c = a[u];
+      if (H > 1) c = make_double2(__shfl(c.x, g * LG + h * RG + i), __shfl(c.y, g * LG + h * RG + i));
+      // the high word of a double >= 0 orders like the double; its low bits make room for the row
+      const unsigned hi = (unsigned)(__builtin_bit_cast(unsigned long long, c.x * c.x + c.y * c.y) >> 32);
+      unsigned key = used ? 0u : (hi & ~(unsigned)(RG - 1)) | (unsigned)(RG - 1 - i);
+      key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0xb1, 0xf, 0xf, true));   // lanes ^ 1
+      key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0x4e, 0xf, 0xf, true));   // lanes ^ 2
+      key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0x141, 0xf, 0xf, true));  // mirrored in 8
+      key = max(key, (unsigned)__builtin_amdgcn_mov_dpp((int)key, 0x140, 0xf, 0xf, true));  // mirrored in 16
+      if (RG > 16) key = max(key, (unsigned)__shfl_xor((int)key, 16));
+      if (RG > 32) key = max(key, (unsigned)__shfl_xor((int)key, 32));
+      const int r = RG - 1 - (int)(key & (unsigned)(RG - 1));
+      if (i == q) rp = r;
+      if (i == r) {
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+          row[hl * C + j] = a[j];
+          a[j] = make_double2(0.0, 0.0);
+        }
+        pos = q;
+        used = true;
       }
-      pos = p;
-      used = true;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    const double2 pv = row[0];
-    const double den = pv.x * pv.x + pv.y * pv.y;
-    const double2 inv = make_double2(pv.x / den, -pv.y / den), t = cmul(c, inv);
-    // every row takes base + f (pivot row): the pivot row itself is 0 + row / pivot
-    const double2 f = i == r ? inv : make_double2(-t.x, -t.y);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      double2 xr[NX];
 #pragma unroll
-    for (int j = 1; j < N; ++j) a[j - 1] = cfma(f, row[j], a[j]);
-    a[N - 1] = f;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  }
-  // column q of the inverse is in register q + N - n
-  double tr = 0.0, ti = 0.0;
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const int q = j - (N - n);
-    if (q < 0) continue;
-    const int rq = __shfl(rp, g * LG + q);
-    if (i >= n) continue;
-    const int64_t e = (int64_t)rq * n + pos;  // M^-1[r_q][pos]
-    if (TRACE) {  // times S[pos][r_q], read as its mirror image: S has been made exactly Hermitian
-      const double2 b = S[(int64_t)sk * n2 + e];
-      tr += a[j].x * b.x + a[j].y * b.y;
-      ti += a[j].y * b.x - a[j].x * b.y;
-    } else if (live) {
-      out[m * n2 + e] = a[j];
+      for (int y = 0; y < NX; ++y) xr[y] = row[hl * C + 16 * y + (lane & 15)];  // past C: not used
+      const double2 pv = row[h * C + u];
+      const double den = pv.x * pv.x + pv.y * pv.y;
+      const double2 inv = make_double2(pv.x / den, -pv.y / den), t = cmul(c, inv);
+      // every row takes base + f (pivot row): the pivot row itself is 0 + row / pivot
+      const double2 f = i == r ? inv : make_double2(-t.x, -t.y);
+      fmac_bcast_row<C, 0>(a, xr, f, -f.y);
+      if (H == 1 || hl == h) a[u] = f;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
+    const double2 t0 = a[0], t1 = a[1];
+#pragma unroll
+    for (int j = 2; j < C; ++j) a[j - 2] = a[j];
+    a[C - 2] = t0;
+    a[C - 1] = t1;
   }
-  if (TRACE) {
+  if (TRACE) {  // M^-1[r_q][pos] times S[pos][r_q], read as its mirror image: S has been made exactly Hermitian
+    double tr = 0.0, ti = 0.0;
+    const int po = (sk * n2 + min(pos, n - 1)) * (int)sizeof(double2);
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const double2 b = buf_load_z(sres, po + min(__shfl(rp, g * LG + hl * C + j), n - 1) * step);
+      if (i < n && hl * C + j < n) {
+        tr += a[j].x * b.x + a[j].y * b.y;
+        ti += a[j].y * b.x - a[j].x * b.y;
+      }
+    }
 #pragma unroll
     for (int o = LG / 2; o > 0; o >>= 1) {
       tr += __shfl_xor(tr, o);
       ti += __shfl_xor(ti, o);
     }
-    if (live && i == 0) out[m] = make_double2(wk[sk % ink] * tr, wk[sk % ink] * ti);
+    if (live && lane % LG == 0) {
+      const double f = wk[sk % ink];
+      out[m] = make_double2(f * tr, f * ti);
+      if (paired) out[mp] = make_double2(f * tr, -(f * ti));
+    }
+  } else {
+    double2* o = out + m * n2 + pos;
+    double2* op = out + mp * n2 + (int64_t)pos * n;
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      const int rq = __shfl(rp, g * LG + hl * C + j);
+      if (live && i < n && hl * C + j < n) {
+        o[rq * n] = a[j];
+        if (paired) op[rq] = make_double2(a[j].x, -a[j].y);
+      }
+    }
   }
+}
+
+// out[w] = sum over sk < nsk of tr[w][sk]; one wave per w.
+__global__ __launch_bounds__(64) void trace_sum_kernel(const double2* __restrict__ tr, int nsk, double2* __restrict__ out) {
+  double sr = 0.0, si = 0.0;
+  for (int sk = threadIdx.x; sk < nsk; sk += 64) {
+    const double2 v = tr[(int64_t)blockIdx.x * nsk + sk];
+    sr += v.x;
+    si += v.y;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    sr += __shfl_xor(sr, o);
+    si += __shfl_xor(si, o);
+  }
+  if (threadIdx.x == 0) out[blockIdx.x] = make_double2(sr, si);
 }
 
 // out[m] = w[m % ink] * tr(A_m B_m) = w sum_ij A_m[i][j] B_m[j][i] for nmat n x n matrices
@@ -321,6 +394,12 @@ public:
     Sw_ = alloc<double2>(big);
     Gw_ = alloc<double2>(big);
     tr_ = alloc<double2>((size_t)d.nw * nsk);
+    void* host = nullptr;
+    if (hipHostMalloc(&host, (size_t)d.nw * sizeof(double2)) != hipSuccess) {
+      (void)hipGetLastError();
+      throw status_error(GWHIP_ERR_OOM, "hipHostMalloc failed in the Dyson solver");
+    }
+    trw_ = static_cast<double2*>(host);
     in_ = alloc<double2>((size_t)(d.nts + 1) * nsk * n2);
     std::vector<double> ones(d.ink, 1.0 / (double)d.nk);
     GWHIP_CHECK(hipMemcpy(wk_, ones.data(), ones.size() * sizeof(double), hipMemcpyHostToDevice));
@@ -334,6 +413,8 @@ public:
       if (p) (void)hipFree(p);
     Tft_ = Ttf_ = H_ = S_ = HS1_ = Sw_ = Gw_ = tr_ = in_ = etr_ = eG_ = nullptr;
     wn_ = wk_ = nullptr;
+    if (trw_) (void)hipHostFree(trw_);
+    trw_ = nullptr;
     if (stream_) (void)hipStreamDestroy(stream_);
     stream_ = nullptr;
   }
@@ -347,6 +428,12 @@ public:
     GWHIP_CHECK(hipMemcpy(Ttf_, T_tf, (size_t)d_.nts * d_.nw * sizeof(double2), hipMemcpyHostToDevice));
     GWHIP_CHECK(hipMemcpy(wn_, wn, (size_t)d_.nw * sizeof(double), hipMemcpyHostToDevice));
     TtB_.assign(T_tf + (size_t)(d_.nts - 1) * d_.nw, T_tf + (size_t)d_.nts * d_.nw);
+    paired_ = d_.nw % 2 == 0;
+    for (int64_t n = 0; n < d_.nw / 2 && paired_; ++n) {
+      const double2 *p = T_ft + n * d_.nts, *q = T_ft + (d_.nw - 1 - n) * d_.nts;
+      paired_ = wn[n] == -wn[d_.nw - 1 - n];
+      for (int64_t t = 0; t < d_.nts && paired_; ++t) paired_ = p[t].x == q[t].x && p[t].y == -q[t].y;
+    }
     grid_set_ = true;
   }
 
@@ -509,9 +596,11 @@ private:
   int device_;
   hipStream_t stream_ = nullptr;
   bool grid_set_ = false, sys_set_ = false;
+  bool paired_ = false;  // w_n in +- pairs at mirrored places, T_ft conjugate between them
   double2 *Tft_ = nullptr, *Ttf_ = nullptr, *H_ = nullptr, *S_ = nullptr, *HS1_ = nullptr, *Sw_ = nullptr,
           *Gw_ = nullptr, *tr_ = nullptr, *in_ = nullptr, *etr_ = nullptr, *eG_ = nullptr;
   double *wn_ = nullptr, *wk_ = nullptr;
+  double2* trw_ = nullptr;    // [nw] in pinned host memory, written by trace_sum_kernel
   std::vector<double2> TtB_;  // row nts-1 of T_tf (tau = beta)
 
   template <typename T>
@@ -523,6 +612,8 @@ private:
     }
     return static_cast<T*>(p);
   }
+  bool in_registers() const { return d_.nso <= 48 && nsk_n2() * (int64_t)sizeof(double2) < ((int64_t)1 << 31); }
+  int64_t first_w() const { return paired_ ? d_.nw / 2 : 0; }  // of the w_n that dyson_invert_wave_kernel inverts
   int64_t nsk_n2() const { return d_.ns * d_.ink * d_.nso * d_.nso; }
   // the host G is staged through Sw_ (free once G(i w_n) is formed)
   double2* Gw_scratch_out() { return Sw_; }
@@ -547,7 +638,8 @@ private:
     hipLaunchKernelGGL(add2_kernel, dim3((unsigned)std::min<int64_t>(4096, ceil_div(N, 256))), dim3(256), 0, stream_,
                        H_, Sigma1, HS1_, N);
     GWHIP_CHECK(hipGetLastError());
-    stack_transform(stream_, Tft_, (int)d_.nw, (int)d_.nts, false, Sigma_tau, N, Sw_);
+    const int64_t w0 = in_registers() ? first_w() : 0;
+    stack_transform(stream_, Tft_ + w0 * d_.nts, (int)(d_.nw - w0), (int)d_.nts, false, Sigma_tau, N, Sw_ + w0 * N);
   }
 
   template <bool TRACE, bool GLOB>
@@ -566,15 +658,16 @@ private:
   template <int N, bool TRACE>
   void launch_invert_wave(double mu, double2* out) {
     const int nsk = (int)(d_.ns * d_.ink);
-    const int64_t nmat = d_.nw * nsk, blocks = ceil_div(nmat, DysonWave<N>::PER);
+    const int64_t blocks = ceil_div((d_.nw - first_w()) * nsk, DysonWave<N>::PER);
     if (blocks > 0x3ffffff) throw status_error(GWHIP_ERR_UNSUPPORTED, "too many Dyson matrices");
     hipLaunchKernelGGL((dyson_invert_wave_kernel<N, TRACE>), dim3((unsigned)blocks), dim3(64), 0, stream_, HS1_, S_, Sw_,
-                       wn_, mu, (int)d_.nso, nsk, (int)d_.ink, wk_, out, nmat);
+                       wn_, mu, (int)d_.nso, nsk, (int)d_.ink, wk_, out, (int)d_.nw, paired_ ? 1 : 0);
     GWHIP_CHECK(hipGetLastError());
   }
   template <bool TRACE>
   void launch_invert(double mu, double2* out) {
-    switch ((int)ceil_div(d_.nso, 4)) {
+    // dyson_invert_wave_kernel reads S by 32-bit offsets
+    switch (in_registers() ? (int)ceil_div(d_.nso, 4) : 0) {
       case 1: return launch_invert_wave<4, TRACE>(mu, out);
       case 2: return launch_invert_wave<8, TRACE>(mu, out);
       case 3: return launch_invert_wave<12, TRACE>(mu, out);
@@ -599,19 +692,12 @@ private:
 
   double count(double mu) {
     invert(mu, true);
-    const int64_t nsk = d_.ns * d_.ink;
-    std::vector<double2> tr((size_t)d_.nw * nsk);
-    GWHIP_CHECK(hipMemcpyAsync(tr.data(), tr_, tr.size() * sizeof(double2), hipMemcpyDeviceToHost, stream_));
+    // summed over (s, k) on the device, into host memory: copying and summing every trace here took 75 us a count
+    hipLaunchKernelGGL(trace_sum_kernel, dim3((unsigned)d_.nw), dim3(64), 0, stream_, tr_, (int)(d_.ns * d_.ink), trw_);
+    GWHIP_CHECK(hipGetLastError());
     GWHIP_CHECK(hipStreamSynchronize(stream_));
     double re = 0.0;
-    for (int64_t w = 0; w < d_.nw; ++w) {
-      double sr = 0.0, si = 0.0;
-      for (int64_t sk = 0; sk < nsk; ++sk) {
-        sr += tr[(size_t)w * nsk + sk].x;
-        si += tr[(size_t)w * nsk + sk].y;
-      }
-      re += TtB_[w].x * sr - TtB_[w].y * si;
-    }
+    for (int64_t w = 0; w < d_.nw; ++w) re += TtB_[w].x * trw_[w].x - TtB_[w].y * trw_[w].y;
     const double pref = (d_.ns == 2 || d_.nso == 2 * d_.nao) ? 1.0 : 2.0;
     return pref * -re;
   }
