@@ -123,7 +123,8 @@ gw_hip_kernel::gw_hip_kernel(const Dims& d, int device, hipStream_t shared_strea
   // scratch of a small system holds them for a few matrices only (32 of 99 at nk = 1, nao = 10, naux = 154),
   // and each batch is a chain of launches of its own
   const int64_t nb = std::min<int64_t>(64, NQ), panels = qchunk_ * d_.nw_b * (2 * NQ * nb + nb * nb);
-  scratch_elems_ = std::max(scratch_elems_, std::min(panels, (int64_t)(0.02 * budget / sizeof(double2))));
+  const int64_t several = p0_q_batch() * (d_.nts / 2) * nk * NQ * nao2;  // Z of the q that P0 takes at once
+  scratch_elems_ = std::max(scratch_elems_, std::min(std::max(panels, several), (int64_t)(0.02 * budget / sizeof(double2))));
   scratch_ = dalloc<double2>((size_t)scratch_elems_);
 }
 
@@ -530,13 +531,14 @@ void gw_hip_kernel::zero(double2* X, int64_t n) {
 }
 
 // Z_Q = sum_s Gb_s V_Q Gq_s for q and tau in [t0, t0 + tc) into scratch_.
-void gw_hip_kernel::p0_prep(int64_t q, const double2* G, int64_t t0, int64_t tc, int qpw) {
+void gw_hip_kernel::p0_prep(int64_t q, const double2* G, int64_t t0, int64_t tc, int qpw, int64_t nq) {
   if (orb_gemm()) {
     p0_prep_gemm(q, G, t0, tc);
     return;
   }
   ZPrepArgs a = prep_args(q, G, t0, qpw);
-  const dim3 grid((unsigned)ceil_div(d_.NQ, 4 * a.qpb), (unsigned)d_.nk, (unsigned)tc);
+  a.kn = (int)(nq * d_.nk);
+  const dim3 grid((unsigned)ceil_div(d_.NQ, 4 * a.qpb), (unsigned)a.kn, (unsigned)tc);
   orb_dispatch([&](auto nb) {
     constexpr int NB4 = decltype(nb)::value;
     const int sb = prep_spin_blocks(NB4, (int)d_.pseudo_ns);
@@ -561,6 +563,7 @@ ZPrepArgs gw_hip_kernel::prep_args(int64_t q, const double2* G, int64_t t0, int 
   a.kc = (int)kc_p0_;
   a.t0 = (int)t0;
   a.qpb = qpw;
+  a.kn = (int)d_.nk;
   return a;
 }
 
@@ -587,20 +590,34 @@ void gw_hip_kernel::p0_prep_slice(int64_t q, const double2* G, int64_t t0, int64
   });
 }
 
-// P0(t0 .. t0+tc) = -(pref/nk) Z conj(V)^T, FP64 (tile `shape`).
-void gw_hip_kernel::p0_gemm(int64_t q, int64_t tc, double2* Pt0, int shape) {
-  const int64_t nk = d_.nk, NQ = d_.NQ, nao2 = d_.nao * d_.nao, NQ2 = NQ * NQ;
+// P0(t0 .. t0+tc) = -(pref/nk) Z conj(V)^T of nq consecutive q, FP64 (tile `shape`); nq > 1: tc is the half grid.
+void gw_hip_kernel::p0_gemm(int64_t q, int64_t tc, double2* Pt0, int shape, int64_t nq) {
+  const int64_t nk = d_.nk, NQ = d_.NQ, nao2 = d_.nao * d_.nao, NQ2 = NQ * NQ, row = nk * NQ * nao2;
   ZGemmArgs a{};
-  a.M = (int)NQ; a.N = (int)NQ; a.K = (int)(nk * nao2); a.batch = (int)tc;
+  a.M = (int)NQ; a.N = (int)NQ; a.K = (int)(nk * nao2); a.batch = (int)(nq * tc);
   a.kin = (int)nao2; a.nin = (int)NQ;
-  a.A = scratch_; a.sAb = nk * NQ * nao2; a.sAm = nao2; a.sAko = NQ * nao2; a.sAki = 1;
-  a.B = Vq_ + q * nk * NQ * nao2; a.sBb = 0; a.sBko = NQ * nao2; a.sBki = 1; a.sBno = 0; a.sBni = nao2;
+  a.bin = (int)tc; a.sAbo = row; a.sBbo = row; a.sCbo = d_.nts * NQ2;
+  a.A = scratch_; a.sAb = nq * row; a.sAm = nao2; a.sAko = NQ * nao2; a.sAki = 1;
+  a.B = Vq_ + q * row; a.sBb = 0; a.sBko = NQ * nao2; a.sBki = 1; a.sBno = 0; a.sBni = nao2;
   a.C = Pt0; a.sCb = NQ2; a.sCm = NQ; a.sCno = 0; a.sCni = 1;
   a.alpha = make_double2(-d_.prefactor / (double)nk, 0.0);
   a.accumulate = 0; a.conjA = 0; a.conjB = 1;
   a.upper = g_herm_ ? 1 : 0;
-  // partial products in one q of the Dyson work buffer, which only stage_dyson uses
-  zgemm_f64_autosplit(a, d_.nts / 2, Pw_, (int64_t)dyson_per_q(), stream_, shape);
+  // partial products in nq q of the Dyson work buffer, which only stage_dyson uses
+  const int64_t half = d_.nts / 2;
+  zgemm_f64_autosplit(a, p0_q_batch() * half, (int)((int64_t)dyson_per_q() / (half * NQ2)), Pw_, stream_, shape);
+}
+
+// How many q the FP64 P0 takes per launch where the scratch and the Dyson buffer hold them: one q of a small
+// system is a few hundred work-groups of a few microseconds, less than the launches and the gaps between them
+// (nk = 8, nao = 8, naux = 40: 1.41 ms an evaluation q by q, 0.97 all eight at once).  Only where the tiles of one q
+// fill less than half of the chip (768 places, see zgemm_auto_ksplit): with K split for one q at a time naux = 200
+// takes 213 ms an evaluation (nk = 8, nao = 50), four q at once 239.  By the system alone, as the K split of the
+// product follows from it.
+int64_t gw_hip_kernel::p0_q_batch() const {
+  const int64_t tm = ceil_div(d_.NQ, 64), tiles = tm * (tm + 1) / 2 * (d_.nts / 2);
+  if (orb_gemm() || tiles >= 384) return 1;
+  return std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(d_.nk, ceil_div(1536, tiles)), 32768 / d_.nts));
 }
 
 // R = P-tilde(t0 .. t0+tc) conj(V) into scratch_, FP64 (tile `shape`): Pt0 = P-tilde at t0 [tc][NQ^2];
@@ -698,8 +715,26 @@ void gw_hip_kernel::sigma_gemm_split(const SigmaRows& r, int64_t tc, int group) 
 
 // P0 of every q in `qs` (all q of the mesh when null): the i-th into P_ row i.
 void gw_hip_kernel::stage_p0(const double2* G, bool split, const std::vector<int>* qs) {
-  const int64_t n = qs ? (int64_t)qs->size() : d_.nk;
-  for (int64_t i = 0; i < n; ++i) p0_one_q(qs ? (*qs)[i] : i, G, split, P_ + i * d_.nts * d_.NQ * d_.NQ);
+  const int64_t n = qs ? (int64_t)qs->size() : d_.nk, NQ2 = d_.NQ * d_.NQ, half = d_.nts / 2;
+  const int64_t fit = scratch_elems_ / (half * (int64_t)scratch_per_t());
+  const int64_t nq = split || qs || tchunk_p0_ < half ? 1 : std::max<int64_t>(1, std::min(p0_q_batch(), std::min(fit, qchunk_)));
+  if (nq == 1) {
+    for (int64_t i = 0; i < n; ++i) p0_one_q(qs ? (*qs)[i] : i, G, split, P_ + i * d_.nts * NQ2);
+    return;
+  }
+  for (int64_t q = 0; q < n; q += nq) {
+    const int64_t qc = std::min(nq, n - q);
+    double2* Pq = P_ + q * d_.nts * NQ2;
+    timed(K_P0_PREP, [&] { p0_prep(q, G, 0, half, tune_.qpw, qc); });
+    timed(K_P0_GEMM, [&] { p0_gemm(q, half, Pq, tune_.p0_shape, qc); });
+    // with the unused upper half of each q's grid between them
+    const int64_t nmat = (qc - 1) * d_.nts + half;
+    if (g_herm_)
+      mirror_upper(Pq, (int)d_.NQ, NQ2, nmat, stream_);
+    else
+      hermitize(Pq, (int)d_.NQ, NQ2, nmat, stream_);
+    GWHIP_CHECK(hipGetLastError());
+  }
 }
 
 // P0(tau, q) for the half tau grid into Pq[t][Q][Q'] (t < nts/2), Hermitised.
@@ -953,7 +988,8 @@ void gw_hip_kernel::sigma_epi(const double2* G, double2* Sigma, const SigmaRows&
   if (qs > 1) {
     ensure_epi_part(r.n);
     a.part = epi_part_;
-    zero(a.part, (int64_t)qs * d_.nts * d_.ns * r.n * d_.nso * d_.nso);
+    // the blocks below the diagonal that the kernel leaves out are read with the others (and replaced at the end)
+    if (a.upper) zero(a.part, (int64_t)qs * d_.nts * d_.ns * r.n * d_.nso * d_.nso);
   }
   const dim3 grid((unsigned)r.n, (unsigned)qs, (unsigned)(2 * tc * d_.pseudo_ns));
   orb_dispatch([&](auto nb) {

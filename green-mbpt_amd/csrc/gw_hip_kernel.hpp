@@ -347,7 +347,7 @@ private:
   void gather_ibz(const double2* Full, double2* Ibz, int64_t nb);
   std::vector<int> q0_samples() const;
   void apply_q0(double2* Sigma, const double2* G, int64_t nkS);
-  void p0_prep(int64_t q, const double2* G, int64_t t0, int64_t tc, int qpw);
+  void p0_prep(int64_t q, const double2* G, int64_t t0, int64_t tc, int qpw, int64_t nq = 1);
   // orbital contractions as batched GEMMs (nao > 64, or tuning orb_gemm); the VJP's from nao > 48 on
   bool orb_gemm() const { return d_.nao > kOrbMaxNao || tune_.orb_gemm != 0; }
   bool vjp_gemm() const { return d_.nao > kVjpMaxNao || tune_.orb_gemm != 0; }
@@ -365,7 +365,8 @@ private:
   ZPrepArgs prep_args(int64_t q, const double2* G, int64_t t0, int qpw) const;
   DevDims dev_dims() const;
   void p0_prep_slice(int64_t q, const double2* G, int64_t t0, int64_t tc, int qpw);
-  void p0_gemm(int64_t q, int64_t tc, double2* Pt0, int shape);
+  void p0_gemm(int64_t q, int64_t tc, double2* Pt0, int shape, int64_t nq = 1);
+  int64_t p0_q_batch() const;
   void sigma_gemm(const double2* Pt0, const SigmaRows& r, int64_t tc, int shape);
   void p0_slice(int64_t tc);
   void p0_gemm_split(int64_t q, int64_t tc, double2* Pt0, int group, int kchunks);

@@ -132,7 +132,7 @@ struct OrbCfg {
 // Gq_s = G(tau, k + q) block (a, b)); src/gw_cpu_kernel.cpp:170-213 regrouped.
 //   W[p][n] = sum_m V_Q[p][m] Gq[m][n]     A = V_Q block of the quad, B = Gq (the same for the four Q)
 //   Z[t][n] = sum_p Gb[t][p] W[p][n]       A = Gb (the same), B = W
-// grid: (ceil(NQ / (4 QPB)), nk, tcount), QPB quads per work-group.  LDS: SB spin blocks of Gb
+// grid: (ceil(NQ / (4 QPB)), rows, tcount), QPB quads per work-group.  LDS: SB spin blocks of Gb
 // (transposed) and Gq, zero-padded [N4][N4]; a launch covers the spin blocks s0 .. s0 + SB and adds to Z
 // when s0 > 0.  V_Q is streamed once per wave and spin block (the waves of a work-group and the tau
 // neighbours find it in L1 and L2).
@@ -151,6 +151,7 @@ struct ZPrepArgs {
   int* exps;
   int kc;
   int t0, qpb, s0, sb;
+  int kn;                // rows of the launch: nk, or those of several consecutive q (FP64), row q nk + k
 };
 
 __device__ __forceinline__ int quad_bcast(int w, int i) {
@@ -182,7 +183,7 @@ void z_prep_kernel(ZPrepArgs p) {
   int bx, by, bz;
   if (!xcd_block(p.xg, bx, by, bz)) return;
   const int tz = bz, tau = p.t0 + tz, tt = d.nts - 1 - tau;
-  const int k = by, kq = p.kplus[k];
+  const int row = by, k = row % d.nk, kq = p.kplus[row];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lk = lane >> 4, l4 = lane & 3, lb = (lane >> 2) & 3;
@@ -216,7 +217,7 @@ void z_prep_kernel(ZPrepArgs p) {
   }
   const int nb0 = 2 * h, nb1 = 2 * h + 1;
   const int64_t per_k = (int64_t)d.NQ * nao2;
-  const double2* vk = p.V + k * per_k;
+  const double2* vk = p.V + row * per_k;
   const int vlane = lb * nao2 + l4 * nao + lk;
   const int nq = (d.NQ + 3) / 4;
   const int iters = (p.qpb + QW - 1) / QW;
@@ -290,7 +291,7 @@ void z_prep_kernel(ZPrepArgs p) {
     }
     if constexpr (NS == 0) {
       if (!live || Q >= d.NQ) return;
-      double2* zq = p.Z + (((int64_t)tz * d.nk + k) * d.NQ + Q) * nao2;
+      double2* zq = p.Z + (((int64_t)tz * p.kn + row) * d.NQ + Q) * nao2;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int n = 4 * (u ? nb1 : nb0) + l4;

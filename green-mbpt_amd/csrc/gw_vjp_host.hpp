@@ -335,7 +335,7 @@ void gw_hip_kernel::vjp_device(const double2* G, const double2* Sbar, double2* G
           g.alpha = make_double2(c, 0.0);
           g.accumulate = 1;
           g.conjA = 1;
-          zgemm_f64_autosplit(g, nts, Pw_, (int64_t)dyson_per_q(), stream_);
+          zgemm_f64_autosplit(g, nts, (int)((int64_t)dyson_per_q() / (nts * NQ2)), Pw_, stream_);
         }
       }
     }

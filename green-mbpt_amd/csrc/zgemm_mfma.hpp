@@ -10,6 +10,7 @@
 // (with nin2 > 0 the inner part splits once more: ni = n % nin -> (ni / nin2)*sBni + (ni % nin2)*sBni2,
 // which reads a per-block transposed operand in place)
 //   C(m, n) = C + b*sCb + m*sCm + (n / nin)*sCno + (n % nin)*sCni
+// and with bin > 0 the batch index has two levels, b = bo*bin + bi at bo*sXbo + bi*sXb,
 // which lets one kernel run the P0 contraction, the Sigma contraction, the IR transforms
 // and the Dyson products straight out of their resident layouts.
 //
@@ -41,6 +42,8 @@ namespace gwhip {
 struct ZGemmArgs {
   int M, N, K, batch;
   int kin, nin;
+  int bin;           // 0: the batch index is one level; > 0: split as above
+  int64_t sAbo, sBbo, sCbo;
   const double2* A;
   int64_t sAb, sAm, sAko, sAki;
   const double2* B;
@@ -98,9 +101,10 @@ __global__ __launch_bounds__(256, BM * BN > 4096 ? 1 : 3) void zgemm_f64_kernel(
   if (p.upper && m0 >= n0 + BN) return;
   if (p.half) kbeg = m0;
 
-  const double2* __restrict__ A = p.A + b * p.sAb;
-  const double2* __restrict__ B = p.B + b * p.sBb;
-  double2* __restrict__ C = p.C + b * p.sCb + cks;
+  const int64_t bo = p.bin > 0 ? b / p.bin : 0, bi = b - bo * p.bin;
+  const double2* __restrict__ A = p.A + bo * p.sAbo + bi * p.sAb;
+  const double2* __restrict__ B = p.B + bo * p.sBbo + bi * p.sBb;
+  double2* __restrict__ C = p.C + bo * p.sCbo + bi * p.sCb + cks;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -323,7 +327,9 @@ __global__ void zgemm_splitk_reduce_kernel(ZGemmArgs p, const double2* __restric
     si += v.y;
   }
   const int no = n / p.nin;
-  double2* dst = p.C + b * p.sCb + (int64_t)m * p.sCm + (int64_t)no * p.sCno + (int64_t)(n - no * p.nin) * p.sCni;
+  const int64_t bo = p.bin > 0 ? b / p.bin : 0, bi = b - bo * p.bin;
+  double2* dst = p.C + bo * p.sCbo + bi * p.sCb + (int64_t)m * p.sCm + (int64_t)no * p.sCno +
+                 (int64_t)(n - no * p.nin) * p.sCni;
   double2 v = make_double2(p.alpha.x * sr - p.alpha.y * si, p.alpha.x * si + p.alpha.y * sr);
   if (p.accumulate) {
     const double2 o = *dst;
@@ -354,6 +360,7 @@ inline void zgemm_f64_splitk(ZGemmArgs p, int ksplit, double2* part, hipStream_t
   q.sCk = (int64_t)p.batch * p.M * p.N;
   q.C = part;
   q.sCb = (int64_t)p.M * p.N;
+  q.sCbo = p.bin * q.sCb;
   q.sCm = p.N;
   q.sCno = p.nin;
   q.sCni = 1;
@@ -385,27 +392,16 @@ inline int zgemm_auto_ksplit(const ZGemmArgs& p, int64_t batch, int smax) {
   double best_t = 0.0;
   for (int s = 1; s <= smax && (s == 1 || p.K / s >= 64); ++s) {
     const double t = std::ceil(tiles * s / 768.0) * ((double)p.K / s + 64.0) +
-                     (s > 1 ? 60.0 * s * tiles / 768.0 + 200.0 : 0.0);
+                     (s > 1 ? 60.0 * s * tiles / 768.0 + 60.0 : 0.0);
     if (s == 1 || t < best_t) best = s, best_t = t;
   }
   return best;
 }
 
-// zgemm_f64 with that number of K slices; the partial products live in part, and the batch is cut where
-// it does not hold them all (part_elems >= smax M N).
-inline void zgemm_f64_autosplit(const ZGemmArgs& p, int64_t batch, double2* part, int64_t part_elems, hipStream_t stream,
+// zgemm_f64 with that number of K slices, at most smax; part holds smax p.batch M N elements.
+inline void zgemm_f64_autosplit(const ZGemmArgs& p, int64_t batch, int smax, double2* part, hipStream_t stream,
                                 int shape = 0) {
-  const int64_t mn = (int64_t)p.M * p.N;
-  const int s = zgemm_auto_ksplit(p, batch, (int)std::min<int64_t>(16, part_elems / mn));
-  const int64_t step = s > 1 ? std::max<int64_t>(1, part_elems / (s * mn)) : p.batch;
-  for (int64_t b = 0; b < p.batch; b += step) {
-    ZGemmArgs q = p;
-    q.batch = (int)std::min<int64_t>(step, p.batch - b);
-    q.A += b * p.sAb;
-    q.B += b * p.sBb;
-    q.C += b * p.sCb;
-    zgemm_f64_splitk(q, s, part, stream, shape);
-  }
+  zgemm_f64_splitk(p, zgemm_auto_ksplit(p, batch, std::min(16, smax)), part, stream, shape);
 }
 
 }  // namespace gwhip

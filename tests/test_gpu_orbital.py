@@ -92,3 +92,10 @@ def test_exchange_every_block_count(nao, hermitian):
     finally:
         k.close()
     assert rel_err(F, ho.hf_fock(dm, V, S, mad, 3, nao, nao, 1, 6)) < 1e-10
+
+
+@pytest.mark.parametrize("hermitian", [True, False])
+@pytest.mark.parametrize("nk,nao,NQ", [(8, 2, 16), (9, 3, 130), (10, 2, 129)])
+def test_several_q_per_launch(nk, nao, NQ, hermitian):
+    """P0 of several q in one launch: all of them at once, and groups with a shorter last one."""
+    _check(*_system(nk, nao, NQ, hermitian))
