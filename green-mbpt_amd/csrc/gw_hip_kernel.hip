@@ -226,6 +226,7 @@ void gw_hip_kernel::set_grid(const double2* T_bt, const double2* T_tb) {
   Ttb_host_.assign(T_tb, T_tb + (size_t)nts * nwb);
   // P-tilde(tau) = sum_n T_tb[tau][n] P-tilde(i Omega_n) is Hermitian when, over each set of frequencies
   // with the same row of T' (hence the same P0 and P-tilde: +-Omega), the imaginary parts of T_tb cancel
+  const bool was = grid_herm_;
   grid_herm_ = true;
   double fmax_ = 0.0, tmax = 0.0;
   for (const double2& v : fold) fmax_ = std::max(fmax_, std::max(std::fabs(v.x), std::fabs(v.y)));
@@ -248,6 +249,7 @@ void gw_hip_kernel::set_grid(const double2* T_bt, const double2* T_tb) {
     }
     for (double x : im) grid_herm_ = grid_herm_ && std::fabs(x) <= 1e-11 * tmax;
   }
+  if (grid_herm_ != was) ++generation_;  // a captured graph holds the Sigma product of the other kind (sigma_half)
   grid_set_ = true;
   stored_valid_ = false;
 }

@@ -229,7 +229,7 @@ private:
   std::vector<Pending> pending_;  // kernel timings read once the stream has drained
   Tuning tune_;
   bool tuned_ = false;  // set by the autotuner or the caller
-  uint64_t generation_ = 0;  // bumped whenever buffers or launch parameters change
+  uint64_t generation_ = 0;  // bumped whenever buffers, launch parameters or what else a graph holds change
   bool g_herm_ = false;      // G of the evaluation being enqueued is Hermitian
   unsigned long long* hcheck_ = nullptr;
   size_t bytes_ = 0;
