@@ -1013,10 +1013,10 @@ void gw_hip_kernel::sigma_epi(const double2* G, double2* Sigma, const SigmaRows&
 // half form would count one of them twice.
 bool gw_hip_kernel::sigma_half(bool split) const { return g_herm_ && grid_herm_ && !split; }
 
-// Sigma of Hermitian G is Hermitian; with one spin block per (tau, s, k) and the whole P-tilde in R only its
-// upper 4 x 4 blocks are accumulated, and the rest filled from them.
+// Sigma of Hermitian G and P-tilde is Hermitian; with one spin block per (tau, s, k) and the whole P-tilde in R
+// only its upper 4 x 4 blocks are accumulated, and the rest filled from them.
 bool gw_hip_kernel::sigma_upper(bool split) const {
-  return g_herm_ && d_.pns == 1 && !orb_gemm() && !sigma_half(split);
+  return g_herm_ && grid_herm_ && d_.pns == 1 && !orb_gemm() && !sigma_half(split);
 }
 
 // The fused P0 prep + slicing kernel takes one or two collinear spin blocks, as far as their G blocks and
