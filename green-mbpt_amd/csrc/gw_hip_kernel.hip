@@ -225,12 +225,19 @@ void gw_hip_kernel::set_grid(const double2* T_bt, const double2* T_tb) {
   GWHIP_CHECK(hipMemcpy(Ttb_, T_tb, (size_t)nts * nwb * sizeof(double2), hipMemcpyHostToDevice));
   Ttb_host_.assign(T_tb, T_tb + (size_t)nts * nwb);
   // P-tilde(tau) = sum_n T_tb[tau][n] P-tilde(i Omega_n) is Hermitian when, over each set of frequencies
-  // with the same row of T' (hence the same P0 and P-tilde: +-Omega), the imaginary parts of T_tb cancel
+  // with the same row of T' (hence the same P0 and P-tilde: +-Omega), the imaginary parts of T_tb cancel.  What is
+  // left of them, im_c per set c, gives the anti-Hermitian part sum_c im_c P-tilde(i Omega_c), which the half product
+  // drops.  A row's sum of T_tb P-tilde cancels by a few hundred, so both bounds are relative to the row and well
+  // below the accuracy asked of Sigma (1e-10), the one on the sum over c for errors of one sign.  Rounding leaves at
+  // most 1.1e-13 per set and 1.4e-13 in sum on the IR grids (Lambda = 1e3, 1e4; beta 1 to 3000).
   const bool was = grid_herm_;
   grid_herm_ = true;
-  double fmax_ = 0.0, tmax = 0.0;
+  double fmax_ = 0.0;
   for (const double2& v : fold) fmax_ = std::max(fmax_, std::max(std::fabs(v.x), std::fabs(v.y)));
-  for (int64_t i = 0; i < nts * nwb; ++i) tmax = std::max(tmax, std::max(std::fabs(T_tb[i].x), std::fabs(T_tb[i].y)));
+  std::vector<double> row_max((size_t)nts, 0.0), im_sum((size_t)nts, 0.0);
+  for (int64_t t = 0; t < nts; ++t)
+    for (int64_t n = 0; n < nwb; ++n)
+      row_max[t] = std::max(row_max[t], std::max(std::fabs(T_tb[t * nwb + n].x), std::fabs(T_tb[t * nwb + n].y)));
   std::vector<char> done((size_t)nwb, 0);
   for (int64_t n = 0; n < nwb; ++n) {
     if (done[n]) continue;
@@ -247,8 +254,12 @@ void gw_hip_kernel::set_grid(const double2* T_bt, const double2* T_tb) {
       done[m] = 1;
       for (int64_t t = 0; t < nts; ++t) im[t] += T_tb[t * nwb + m].y;
     }
-    for (double x : im) grid_herm_ = grid_herm_ && std::fabs(x) <= 1e-11 * tmax;
+    for (int64_t t = 0; t < nts; ++t) {
+      grid_herm_ = grid_herm_ && std::fabs(im[t]) <= 1e-12 * row_max[t];
+      im_sum[t] += im[t];
+    }
   }
+  for (int64_t t = 0; t < nts; ++t) grid_herm_ = grid_herm_ && std::fabs(im_sum[t]) <= 5e-13 * row_max[t];
   if (grid_herm_ != was) ++generation_;  // a captured graph holds the Sigma product of the other kind (sigma_half)
   grid_set_ = true;
   stored_valid_ = false;
