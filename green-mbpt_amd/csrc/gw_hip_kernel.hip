@@ -427,15 +427,29 @@ void gw_hip_kernel::ensure_slices() {
     }
   }
   GWHIP_CHECK(hipStreamSynchronize(stream_));
-  if (!tuned_) {
-    // row-tile group of the Sigma product: with 64 x 64 tiles four row panels of A (nk = 27, nao = 26, naux = 250:
-    // 57.6 ms an evaluation, 65.8 with eight, 69.4 with sixteen)
-    tune_.p0_oz_tile = ozaki_default_tile(ns, nk, kc_p0_);
-    tune_.s_oz_tile = ozaki_default_tile(ns, 1, kc_s_);
-    tune_.s_group = 4;
-    tune_.p0_kchunks = 0;
-  }
   slices_ns_ = ns;
+  ++generation_;
+}
+
+// tune_ with the keys that are left to the sizes filled in.  Row-tile group of the Sigma product: 256 rows of A
+// whichever the tile (64 x 64, nk = 27, nao = 26, naux = 250: 57.6 ms an evaluation with four row tiles, 65.8 with
+// eight, 69.4 with sixteen).
+Tuning gw_hip_kernel::tuning() const {
+  Tuning t = tune_;
+  if (!t.p0_oz_tile) t.p0_oz_tile = ozaki_default_tile(split_ns_, d_.nk, ceil_div(d_.nao * d_.nao, 64) * 64);
+  if (!t.s_oz_tile) t.s_oz_tile = ozaki_default_tile(split_ns_, 1, ceil_div(d_.NQ, 64) * 64);
+  if (!t.s_group) t.s_group = t.s_oz_tile == 4 ? 4 : 8;
+  return t;
+}
+
+// A key set to the value it has by the sizes goes on following them: callers set all keys at once, those that they
+// do not mean to change to what tuning() gave.
+void gw_hip_kernel::set_tuning(Tuning t) {
+  const Tuning now = tuning();
+  if (t.p0_oz_tile == now.p0_oz_tile) t.p0_oz_tile = tune_.p0_oz_tile;
+  if (t.s_oz_tile == now.s_oz_tile) t.s_oz_tile = tune_.s_oz_tile;
+  if (t.s_group == now.s_group) t.s_group = tune_.s_group;
+  tune_ = t;
   ++generation_;
 }
 
@@ -690,7 +704,7 @@ void gw_hip_kernel::p0_gemm_split(int64_t q, int64_t tc, double2* Pt0, int group
     o.accumulate = sl > 0 ? 1 : 0;
     o.group_m = group;
     o.upper = g_herm_ ? 1 : 0;
-    o.tile = tune_.p0_oz_tile;
+    o.tile = tuning().p0_oz_tile;
     // partial products in one q of the Dyson work buffer, which only stage_dyson uses
     if (nsl == 1) zgemm_ozaki_autosplit(o, ns, d_.nts / 2, Pw_, (int64_t)dyson_per_q(), stream_);
     else zgemm_ozaki(o, ns, stream_);
@@ -722,7 +736,7 @@ void gw_hip_kernel::sigma_gemm_split(const SigmaRows& r, int64_t tc, int group) 
   o.alpha = make_double2(1.0, 0.0);
   o.accumulate = 0;
   o.group_m = group;
-  o.tile = tune_.s_oz_tile;
+  o.tile = tuning().s_oz_tile;
   zgemm_ozaki(o, ns, stream_);
 }
 
@@ -974,7 +988,7 @@ void gw_hip_kernel::sigma_q(const double2* G, double2* Sigma, bool split, const 
     const int64_t tc = std::min(tchunk_sigma_, half - t0);
     if (split) {
       sigma_slice(Pq + t0 * NQ2, tc);
-      timed(K_SIGMA_GEMM, [&] { sigma_gemm_split(r, tc, tune_.s_group); });
+      timed(K_SIGMA_GEMM, [&] { sigma_gemm_split(r, tc, tuning().s_group); });
     } else {
       timed(K_SIGMA_GEMM, [&] { sigma_gemm(Pq + t0 * NQ2, r, tc, tune_.s_shape); });
     }
@@ -1311,12 +1325,11 @@ void gw_hip_kernel::autotune(const double2* G, int precision) {
     sigma_slice(P_, tcs);
     tune_.s_oz_tile = best_of(2, tiles, [&](int c) {
       tune_.s_oz_tile = c;
-      sigma_gemm_split(sigma_rows(0), tcs, tune_.s_group);
+      sigma_gemm_split(sigma_rows(0), tcs, tuning().s_group);
     });
     tune_.s_group = best_of(7, groups, [&](int c) { sigma_gemm_split(sigma_rows(0), tcs, c); });
   }
   tune_.epi_form = 1;
-  tuned_ = true;
   stored_valid_ = false;
   ++generation_;
 }

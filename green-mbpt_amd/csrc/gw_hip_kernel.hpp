@@ -34,21 +34,20 @@ struct KernelStat {
   double ms = 0.0;
 };
 
-// Launch parameters picked by the autotuner (defaults = the best measured at nk = 64, nao = 26,
-// naux = 300; those of the int8 GEMMs by ensure_slices when the slice stores are built): FP64 GEMM tile of the P0 and Sigma contractions (0: 64x64, 1: 128x64,
-// 2: 64x128), the number of aux indices per wave of the P0 prep kernel, and for split precision
-// the row-tile group of the int8 GEMM's L2-aware tile order and whether the P0 orbital kernel
-// writes the int8 slices itself.
+// Launch parameters, defaults or picked by the autotuner: FP64 GEMM tile of the P0 and Sigma contractions
+// (0: 64x64, 1: 128x64, 2: 64x128), the number of aux indices per wave of the P0 prep kernel, and for split
+// precision the row-tile group of the int8 GEMM's L2-aware tile order and whether the P0 orbital kernel writes
+// the int8 slices itself.  Keys of the int8 GEMMs that are 0 here follow the slice count and the sizes
+// (gw_hip_kernel::tuning gives their values) until the autotuner or the caller changes them.
 struct Tuning {
   int p0_shape = 0, s_shape = 0, qpw = 4;
-  int p0_group = 1, s_group = 8;  // split precision: row tiles per L2 group of the int8 GEMMs
-  int p0_oz_tile = 2, s_oz_tile = 2;  // int8 GEMM block tile: 2 (32 x 64, 16 x 16 x 64 MFMAs) or
+  int p0_group = 1, s_group = 0;  // split precision: row tiles per L2 group of the int8 GEMMs
+  int p0_oz_tile = 0, s_oz_tile = 0;  // int8 GEMM block tile: 2 (32 x 64, 16 x 16 x 64 MFMAs) or
                                       // 4 (64 x 64, 32 x 32 x 32 MFMAs, staged by LDS DMA)
   int p0_fused = 1;  // split precision, one or two collinear spin blocks: P0 orbital kernel writes int8
                      // slices directly
   int orb_gemm = 0;  // orbital contractions as batched FP64 GEMMs (always so for nao > 64)
-  int p0_kchunks = 4;  // split precision: k chunks per launch of the int8 P0 GEMM (0: all in one), so
-                       // that each launch's operand window stays in L2
+  int p0_kchunks = 0;  // split precision: k chunks per launch of the int8 P0 GEMM (0: all in one)
   int epi_form = 0;  // 0 .. 3 accepted; one form of the Sigma epilogue is left, so it has no effect
   static constexpr int count = 11;
   void to_array(int* v) const {
@@ -193,12 +192,8 @@ public:
   // tiles of P0 are computed and mirrored.  Runs on the stream and synchronises.
   bool detect_hermitian_G(const double2* G_dev);
   void autotune(const double2* G_dev, int precision);
-  const Tuning& tuning() const { return tune_; }
-  void set_tuning(const Tuning& t) {
-    tune_ = t;
-    tuned_ = true;
-    ++generation_;
-  }
+  Tuning tuning() const;
+  void set_tuning(Tuning t);
   void set_timing(bool on) { timing_ = on; }
   // buffers of the GEMM form of the orbital contractions and the Sigma epilogue's partial sums
   // over Q ranges (full mesh); allocates, so call before a capture
@@ -228,7 +223,6 @@ private:
   };
   std::vector<Pending> pending_;  // kernel timings read once the stream has drained
   Tuning tune_;
-  bool tuned_ = false;  // set by the autotuner or the caller
   uint64_t generation_ = 0;  // bumped whenever buffers, launch parameters or what else a graph holds change
   bool g_herm_ = false;      // G of the evaluation being enqueued is Hermitian
   unsigned long long* hcheck_ = nullptr;

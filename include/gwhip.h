@@ -156,13 +156,13 @@ int gwhip_eval_sigma_device_noalloc(gwhip_handle* h, const void* G_dev, void* Si
 
 /* ---- launch-parameter autotuning ------------------------------------------------------
  * Time the candidate launch parameters of this system on its own operands (G in device memory)
- * and keep the fastest: the FP64 GEMM tiles of the P0 and Sigma contractions (0: 64x64,
- * 1: 128x64, 2: 64x128), the aux indices per wave of the P0 orbital kernel (1, 2, 4, 8) and, for
- * the split-precision modes, the block tile of each int8 GEMM, the number of row tiles that sweep
+ * and keep the fastest: the aux indices per wave of the P0 orbital kernel (1, 2, 4, 8); in FP64
+ * the GEMM tiles of the P0 and Sigma contractions (0: 64x64, 1: 128x64, 2: 64x128); in the
+ * split-precision modes the block tile of each int8 GEMM, the number of row tiles that sweep
  * the column tiles together in the int8 GEMMs' L2-aware tile order (1 .. 64), the k chunks per
- * launch of the int8 P0 GEMM and the fused or separate slicing of the P0 operand; in both
- * precisions the form of the register Sigma epilogue.
- * Results change only by rounding (the epilogue forms and the k chunks add in another order).
+ * launch of the int8 P0 GEMM and the fused or separate slicing of the P0 operand.  Parameters of
+ * the other mode stay as they are.
+ * Results change only by rounding (the k chunks add in another order).
  * No reference counterpart. */
 int gwhip_autotune(gwhip_handle* h, const void* G_dev, int precision);
 /* The tuning as an array of GWHIP_TUNING_COUNT ints: [0] FP64 P0 GEMM tile, [1] FP64 Sigma GEMM
@@ -171,11 +171,11 @@ int gwhip_autotune(gwhip_handle* h, const void* G_dev, int precision);
  * MFMAs, A staged through registers; 4: 64x64 of 32x32x32 MFMAs; results bit-identical),
  * [7] split P0 orbital kernel writes the int8 slices itself (1) or via a separate pass (0),
  * [8] orbital-size products (Z = Gb V Gq of P0, V G R of Sigma) as batched FP64 GEMMs (1) or the
- * register-chained MFMA kernels (0); always 1 in effect for nao > 48, [9] int8 P0 GEMM: k chunks
- * per launch (0: all in one launch), so that each launch's operands stay in L2, [10] register
- * Sigma epilogue: 0 chosen by nao, 1 4x4x4 MFMAs with every 16-row group of i in each wave
- * (nao <= 32; otherwise as 0), 2 4x4x4 MFMAs with one 16-row group per wave, 3 16x16x4 MFMAs
- * (results agree to rounding). */
+ * register-chained MFMA kernels (0); always 1 in effect for nao > 64 (the exchange of the Fock
+ * build and the VJP: nao > 48), [9] int8 P0 GEMM: k chunks per launch (0: all in one launch),
+ * [10] accepted from 0 to 3 and without effect (the Sigma epilogue has one form).
+ * Until the autotuner sets them or gwhip_set_tuning changes their values, [4], [5] and [6] follow
+ * the slice count and the sizes of the system; gwhip_get_tuning returns what they are. */
 #define GWHIP_TUNING_COUNT 11
 int gwhip_get_tuning(const gwhip_handle* h, int* values, int n);
 int gwhip_set_tuning(gwhip_handle* h, const int* values, int n);

@@ -283,3 +283,40 @@ def test_k_split_of_p0(ns, nao, NQ):
     print(f"ns={ns} nao={nao}: vs oracle {errs}, vs one launch per chunk {[rel_err(o, out[1]) for o in out]}", flush=True)
     assert max(errs) < {3: 1e-4, 4: TOL_SPLIT, 5: 1e-10}[ns]
     assert max(rel_err(o, out[1]) for o in out) < 1e-12
+
+
+def test_int8_defaults_survive_other_tuning():
+    """The int8 GEMMs' parameters follow the slice count and the sizes until they themselves are changed: not
+    after an FP64 autotune or another key, not for the key that the caller did set."""
+    import torch
+
+    G, V, T, d = synthetic(2, 26, 12, beta=20.0, lam=1e3, mesh=(2, 1, 1), seed=4, sigma=0.02)
+    G_d = torch.tensor(G, device="cuda:0")
+    torch.cuda.synchronize()
+    keys = ("sigma_group", "p0_split_tile", "sigma_split_tile", "p0_kchunks")
+    seen = {}
+    for name in ("nothing", "another key", "FP64 autotune", "sigma_split_tile", "p0_kchunks"):
+        k = _kernel(d, T)
+        try:
+            k.set_grid(T.T_bt, T.T_tb)
+            k.upload_V(V)
+            if name == "another key":
+                k.set_tuning(aux_per_wave=8, epi_form=2)
+            elif name == "FP64 autotune":
+                k.autotune(G_d.data_ptr())
+            elif name == "sigma_split_tile":
+                k.set_tuning(sigma_split_tile=2)
+            elif name == "p0_kchunks":
+                k.set_tuning(p0_kchunks=1)
+            k.solve(G, gl.PREC_SPLIT)
+            four = tuple(k.tuning()[x] for x in keys)
+            k.set_split_slices(5)
+            k.solve(G, gl.PREC_SPLIT)
+            seen[name] = four, tuple(k.tuning()[x] for x in keys)
+        finally:
+            k.close()
+    print(seen, flush=True)
+    assert seen["nothing"] == ((4, 4, 4, 0), (4, 2, 4, 0))
+    assert seen["another key"] == seen["FP64 autotune"] == seen["nothing"]
+    assert seen["sigma_split_tile"] == ((8, 4, 2, 0), (8, 2, 2, 0))
+    assert seen["p0_kchunks"] == ((4, 4, 4, 1), (4, 2, 4, 1))
