@@ -566,13 +566,21 @@ void gw_hip_kernel::p0_prep(int64_t q, const double2* G, int64_t t0, int64_t tc,
   ZPrepArgs a = prep_args(q, G, t0, qpw);
   a.kn = (int)(nq * d_.nk);
   const dim3 grid((unsigned)ceil_div(d_.NQ, 4 * a.qpb), (unsigned)a.kn, (unsigned)tc);
+  if (z_prep16_takes(d_.nao)) {
+    const int sb = d_.pseudo_ns > 1 ? 2 : 1;
+    for (a.s0 = 0; a.s0 < d_.pseudo_ns; a.s0 += sb)
+      launch_orb(sb == 2 ? z_prep16_kernel<0, 2> : z_prep16_kernel<0, 1>, a, grid, 256, z_prep16_lds_bytes(sb), stream_);
+    return;
+  }
   orb_dispatch([&](auto nb) {
     constexpr int NB4 = decltype(nb)::value;
-    const int sb = prep_spin_blocks(NB4, (int)d_.pseudo_ns);
-    for (int s0 = 0; s0 < d_.pseudo_ns; s0 += sb) {
-      a.s0 = s0;
-      a.sb = sb;
-      launch_orb(z_prep_kernel<NB4, 0>, a, grid, OrbCfg<NB4>::NT, z_prep_lds_bytes(NB4, sb, 0, 0), stream_);
+    if constexpr (!z_prep16_takes(4 * NB4)) {
+      const int sb = prep_spin_blocks(NB4, (int)d_.pseudo_ns);
+      for (int s0 = 0; s0 < d_.pseudo_ns; s0 += sb) {
+        a.s0 = s0;
+        a.sb = sb;
+        launch_orb(z_prep_kernel<NB4, 0>, a, grid, OrbCfg<NB4>::NT, z_prep_lds_bytes(NB4, sb, 0, 0), stream_);
+      }
     }
   });
 }
@@ -604,12 +612,21 @@ void gw_hip_kernel::p0_prep_slice(int64_t q, const double2* G, int64_t t0, int64
   ZPrepArgs a = prep_args(q, G, t0, qpw);
   a.sb = (int)d_.pseudo_ns;
   const dim3 grid((unsigned)ceil_div(d_.NQ, 4 * a.qpb), (unsigned)d_.nk, (unsigned)tc);
+  const int ns = split_ns_;
+  if (z_prep16_takes(d_.nao)) {
+    auto go = [&](auto k3, auto k4, auto k5) {
+      launch_orb(ns == 5 ? k5 : ns == 4 ? k4 : k3, a, grid, 256, z_prep16_lds_bytes(a.sb), stream_);
+    };
+    if (a.sb == 2) go(z_prep16_kernel<3, 2>, z_prep16_kernel<4, 2>, z_prep16_kernel<5, 2>);
+    else go(z_prep16_kernel<3, 1>, z_prep16_kernel<4, 1>, z_prep16_kernel<5, 1>);
+    return;
+  }
   orb_dispatch([&](auto nb) {
     constexpr int NB4 = decltype(nb)::value;
-    if constexpr (NB4 <= kFusedMaxNao / 4) {
-      const size_t lds = z_prep_lds_bytes(NB4, a.sb, split_ns_, (int)kc_p0_);
-      if (split_ns_ == 5) launch_orb(z_prep_kernel<NB4, 5>, a, grid, OrbCfg<NB4>::NT, lds, stream_);
-      else if (split_ns_ == 4) launch_orb(z_prep_kernel<NB4, 4>, a, grid, OrbCfg<NB4>::NT, lds, stream_);
+    if constexpr (NB4 <= kFusedMaxNao / 4 && !z_prep16_takes(4 * NB4)) {
+      const size_t lds = z_prep_lds_bytes(NB4, a.sb, ns, (int)kc_p0_);
+      if (ns == 5) launch_orb(z_prep_kernel<NB4, 5>, a, grid, OrbCfg<NB4>::NT, lds, stream_);
+      else if (ns == 4) launch_orb(z_prep_kernel<NB4, 4>, a, grid, OrbCfg<NB4>::NT, lds, stream_);
       else launch_orb(z_prep_kernel<NB4, 3>, a, grid, OrbCfg<NB4>::NT, lds, stream_);
     } else {
       throw status_error(GWHIP_ERR_UNSUPPORTED, "fused P0 slicing: nao out of range");
@@ -1044,12 +1061,15 @@ bool gw_hip_kernel::sigma_upper(bool split) const {
   return g_herm_ && grid_herm_ && d_.pns == 1 && !orb_gemm() && !sigma_half(split);
 }
 
-// The fused P0 prep + slicing kernel takes one or two collinear spin blocks, as far as their G blocks and
-// a quad's digits fit the work-group's LDS (with two and four slices: nao = 36).
+// The fused P0 prep + slicing kernels take one or two collinear spin blocks: z_prep_kernel as far as their G blocks
+// and a quad's digits fit the work-group's LDS (with two and four slices: nao = 36), z_prep16_kernel always.  Of
+// the sizes between, prep and slicing in two kernels at nao = 40, two spin blocks, nk = 8, naux = 300: 214 ms an
+// evaluation, 228 with the 16-wide fused kernel and epilogue that this size had before.
 bool gw_hip_kernel::fused_p0() const {
   if (d_.pns != 1 || d_.pseudo_ns > 2 || d_.nao > kFusedMaxNao || orb_gemm()) return false;
+  if (z_prep16_takes(d_.nao)) return true;
   const int nb4 = (int)ceil_div(d_.nao, 4), kc = (int)ceil_div(d_.nao * d_.nao, 64) * 64;
-  return z_prep_fits(nb4 > 10 ? 12 : nb4, (int)d_.pseudo_ns, split_ns_, kc);
+  return z_prep_fits(nb4, (int)d_.pseudo_ns, split_ns_, kc);
 }
 
 int gw_hip_kernel::epi_qsplit(int64_t nks) const {

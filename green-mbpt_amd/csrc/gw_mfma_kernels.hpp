@@ -124,7 +124,7 @@ template <int NB4>
 struct OrbCfg {
   static constexpr int WS = (NB4 + 1) / 2, QW = WS == 1 ? 4 : (WS == 2 ? 2 : 1);
   static constexpr int N4 = 4 * NB4, NT = 64 * WS * QW;
-  static constexpr bool DBL = NB4 <= 10;  // P0 prep: above, G and a quad's digits leave no room for a second slab
+  static constexpr bool DBL = NB4 <= 10;  // P0 prep (nao up to 40, or above 48): G leaves no room for a second slab above
 };
 
 // ---------------------------------------------------------------------------------------
@@ -386,6 +386,167 @@ void z_prep_kernel(ZPrepArgs p) {
   for (int it = 0; it < iters; ++it) {
     if (NB4 % 2 == 0 || nb1 < NB4) quad(it, std::true_type{});
     else quad(it, std::false_type{});
+  }
+}
+
+// The same for nao of 41 to 48 on v_mfma_f64_16x16x4f64, three 16-wide blocks a side.  In column blocks those
+// sizes make six waves for four SIMDs, and G leaves no room for a second slab of V_Q: the kernel above waits.
+// Here each of four waves has a SIMD and its whole register file to itself, holds Z_Q and W, loads V_Q a slab
+// ahead and meets no barrier.  Bound: FP64 matrix cores (two thirds of their 16x16x4 rate) and the first slab.
+// Register r of a 16x16 result holds row lane/16 + 4 r, column lane%16: the operand layout of the next product.
+// Per launch (nk = 8, naux = 300, 50 tau), and in column blocks: FP64 4.2 ms at nao 41 (5.5), 4.7 at 48 (5.8); four
+// slices 4.5 (6.5) and 4.8 (7.0); two spin blocks at nao 44 7.7 (10.5), four at nk = 4, nao 41 6.2 (7.9).
+// LDS: SB spin blocks of Gb and Gq as zero-padded planes [48][49].  A work-group takes 4 qpb consecutive Q.
+constexpr int ZP16_N = 48, ZP16_LD = ZP16_N + 1, ZP16_PL = ZP16_N * ZP16_LD;
+inline size_t z_prep16_lds_bytes(int sb) { return (size_t)sb * 4 * ZP16_PL * sizeof(double); }
+constexpr bool z_prep16_takes(int64_t nao) { return nao > 40 && nao <= ZP16_N; }
+
+template <int NS, int SB>
+__global__ __launch_bounds__(256, 1) void z_prep16_kernel(ZPrepArgs p) {
+  constexpr int NB = 3, LD = ZP16_LD, PL = ZP16_PL;
+  extern __shared__ double zp16_lds[];  // [SB][Gb re | Gb im | Gq re | Gq im]
+  const DevDims& d = p.d;
+  const int nao = d.nao, nao2 = nao * nao;
+  int bx, by, bz;
+  if (!xcd_block(p.xg, bx, by, bz)) return;
+  const int tz = bz, tau = p.t0 + tz, tt = d.nts - 1 - tau;
+  const int row = by, k = row % d.nk, kq = p.kplus[row];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int lrow = lane & 15, lk = lane >> 4;
+  const int nslab = (nao + 3) / 4;
+  for (int s = 0; s < SB; ++s) {
+    const int ss = p.s0 + s, is = ss / (d.pns * d.pns), a = (ss / d.pns) % d.pns, b = ss % d.pns;
+    const double2* Gbar = p.G + g_index(d, tt, is, k);
+    const double2* Gk = p.G + g_index(d, tau, is, kq);
+    double* g = zp16_lds + (size_t)s * 4 * PL;
+    for (int e = tid; e < ZP16_N * ZP16_N; e += 256) {
+      const int r = e / ZP16_N, c = e - (e / ZP16_N) * ZP16_N;
+      double2 vb = make_double2(0.0, 0.0), vq = make_double2(0.0, 0.0);
+      if (r < nao && c < nao) {
+        vb = Gbar[(int64_t)(b * nao + r) * d.nso + a * nao + c];  // Gb[t = r][p = c]
+        vq = Gk[(int64_t)(a * nao + r) * d.nso + b * nao + c];    // Gq[m = r][n = c]
+      }
+      g[r * LD + c] = vb.x;
+      g[PL + r * LD + c] = vb.y;
+      g[2 * PL + r * LD + c] = vq.x;
+      g[3 * PL + r * LD + c] = vq.y;
+    }
+  }
+  __syncthreads();
+  // V_Q[16 bp + lane%16][4 sl + lane/16]; elements of other rows and of the next Q only meet zeros of G
+  const __amdgpu_buffer_rsrc_t vres = buf_rsrc(p.V + (int64_t)row * d.NQ * nao2, (int64_t)d.NQ * nao2);
+  const int vlane = (lrow * nao + lk) * 16;
+  for (int qi = 0; qi < p.qpb; ++qi) {
+    const int Q = (bx * 4 + wave) * p.qpb + qi;
+    if (Q >= d.NQ) break;
+    const int vq = Q * nao2 * 16 + vlane;
+    auto load_v = [&](int sl, double2 (&v)[NB]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int bp = 0; bp < NB; ++bp) v[bp] = buf_load_z(vres, vq + (16 * bp * nao + 4 * sl) * 16);
+    };
+    v4d zr[NB][NB], zi[NB][NB];  // [bn][bt]
+#pragma unroll
+    for (int bn = 0; bn < NB; ++bn)
+#pragma unroll
+      for (int x = 0; x < NB; ++x) zr[bn][x] = zi[bn][x] = v4zero();
+#pragma unroll 1
+    for (int s = 0; s < SB; ++s) {
+      const double* g = zp16_lds + (size_t)s * 4 * PL;
+      v4d wr[NB][NB], wi[NB][NB];  // [bn][bp]
+#pragma unroll
+      for (int bn = 0; bn < NB; ++bn)
+#pragma unroll
+        for (int x = 0; x < NB; ++x) wr[bn][x] = wi[bn][x] = v4zero();
+      double2 av[NB], nx[NB];  // this slab of V_Q and the next
+      load_v(0, av);
+#pragma unroll 1
+      for (int sl = 0; sl < nslab; ++sl) {
+        load_v(sl + 1, nx);
+        const double* gm = g + 2 * PL + (4 * sl + lk) * LD + lrow;
+#pragma unroll
+        for (int bn = 0; bn < NB; ++bn) {
+          const double br = gm[16 * bn], bi = gm[PL + 16 * bn];
+#pragma unroll
+          for (int bp = 0; bp < NB; ++bp) cmfma(wr[bn][bp], wi[bn][bp], av[bp].x, av[bp].y, br, bi);
+        }
+#pragma unroll
+        for (int bp = 0; bp < NB; ++bp) av[bp] = nx[bp];
+      }
+      // every column block at once, so that an element of Gb read from LDS serves them all
+#pragma unroll
+      for (int bp = 0; bp < NB; ++bp)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (16 * bp + 4 * r >= nao) continue;  // wholly padding
+          const int c = 16 * bp + lk + 4 * r;
+#pragma unroll
+          for (int bt = 0; bt < NB; ++bt) {
+            const int t = 16 * bt + lrow;
+            const double gr = g[t * LD + c], gi = g[PL + t * LD + c];
+#pragma unroll
+            for (int bn = 0; bn < NB; ++bn) cmfma(zr[bn][bt], zi[bn][bt], gr, gi, wr[bn][bp][r], wi[bn][bp][r]);
+          }
+        }
+    }
+    if constexpr (NS == 0) {
+      double2* zq = p.Z + (((int64_t)tz * p.kn + row) * d.NQ + Q) * nao2;
+#pragma unroll
+      for (int bn = 0; bn < NB; ++bn) {
+        const int n = 16 * bn + lrow;
+#pragma unroll
+        for (int bt = 0; bt < NB; ++bt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int t = 16 * bt + lk + 4 * r;
+            if (t >= nao || n >= nao) continue;
+            double2 o = make_double2(zr[bn][bt][r], zi[bn][bt][r]);
+            if (p.s0 > 0) {
+              const double2 old = zq[t * nao + n];
+              o.x += old.x;
+              o.y += old.y;
+            }
+            zq[t * nao + n] = o;
+          }
+      }
+    } else {
+      // the wave owns the slice row-chunk: its exponent, then the digits of both planes
+      double mx = 0.0;
+#pragma unroll
+      for (int bn = 0; bn < NB; ++bn)
+#pragma unroll
+        for (int bt = 0; bt < NB; ++bt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) mx = fmax(mx, fmax(fabs(zr[bn][bt][r]), fabs(zi[bn][bt][r])));
+      mx = wave_max(mx);
+      int e = 0;
+      if (mx > 0.0) (void)frexp(mx, &e);
+      const int64_t task = ((int64_t)tz * d.NQ + Q) * d.nk + k;
+      if (lane == 0) p.exps[task] = e;
+      const double sc = ldexp(OZ_FIRST, -e);
+      int8_t* out = p.dst + task * (int64_t)OZ_PLANES * NS * p.kc;
+#pragma unroll
+      for (int bn = 0; bn < NB; ++bn)
+#pragma unroll
+        for (int bt = 0; bt < NB; ++bt)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int t = 16 * bt + lk + 4 * r, n = 16 * bn + lrow;
+            if (n >= nao || t >= nao) continue;
+            int dr[NS], di[NS];
+            oz_element_digits<NS>(zr[bn][bt][r], zi[bn][bt][r], sc, dr, di);
+            int8_t* o = out + oz_offset(OZ_PLANES * NS, 0, t * nao + n);
+#pragma unroll
+            for (int sl = 0; sl < NS; ++sl) {
+              o[sl * 32] = (int8_t)dr[sl];
+              o[(NS + sl) * 32] = (int8_t)di[sl];
+            }
+          }
+      const int padn = p.kc - nao2;  // the chunk padding [nao^2, kc) of every plane-slice
+      for (int i = lane; i < OZ_PLANES * NS * padn; i += 64) {
+        const int ps = i / padn;
+        out[oz_offset(OZ_PLANES * NS, ps, nao2 + (i - ps * padn))] = 0;
+      }
+    }
   }
 }
 

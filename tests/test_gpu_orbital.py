@@ -60,6 +60,12 @@ def test_spin_blocks(case):
     _check(*_system(2, case["nao"], 5, ns=case.get("ns", 1), nso=case.get("nso")))
 
 
+@pytest.mark.parametrize("case", [dict(nao=41), dict(nao=48), dict(nao=45, ns=2), dict(nao=44, nso=88), dict(nao=48, nso=96)])
+def test_three_wide_blocks(case):
+    """nao of 41 to 48, more auxiliary indices than a work-group of the P0 prep takes, and several q per launch."""
+    _check(*_system(2, case["nao"], 19, ns=case.get("ns", 1), nso=case.get("nso")))
+
+
 @pytest.mark.parametrize("hermitian", [True, False])
 @pytest.mark.parametrize("NQ", [63, 64, 65, 128, 129, 200])
 def test_half_product_block_edges(NQ, hermitian):

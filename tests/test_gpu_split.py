@@ -320,3 +320,32 @@ def test_int8_defaults_survive_other_tuning():
     assert seen["another key"] == seen["FP64 autotune"] == seen["nothing"]
     assert seen["sigma_split_tile"] == ((8, 4, 2, 0), (8, 2, 2, 0))
     assert seen["p0_kchunks"] == ((4, 4, 4, 1), (4, 2, 4, 1))
+
+
+@pytest.mark.parametrize("slices", [3, 4, 5])
+@pytest.mark.parametrize("spins", [1, 2])
+@pytest.mark.parametrize("nao", [41, 47, 48])
+def test_fused_slicing_of_three_blocks(nao, spins, slices):
+    """nao of 41 to 48, with a last work-group that is not full: the fused kernel, also with both spin blocks, against
+    the separate pass (the same sums with one spin block, hence the same bits; with two they are added in another
+    order, up to the last digit's rounding) and against the oracle."""
+    G, V, T, d = synthetic(2, nao, 21, ns=spins, beta=20.0, lam=1e3, mesh=(2, 1, 1), seed=29, sigma=0.5 / nao)
+    out = []
+    for fused in (0, 1):
+        k = _kernel(d, T)
+        try:
+            k.set_grid(T.T_bt, T.T_tb)
+            k.upload_V(V)
+            k.set_split_slices(slices)
+            k.set_tuning(p0_fused_slices=fused)
+            out.append(k.solve(G, gl.PREC_SPLIT))
+        finally:
+            k.close()
+    S_ref = go.gw_sigma(G, V, T.T_bt, T.T_tb, d["nk"], d["nao"], d["nso"], d["ns"], d["NQ"], mesh=d["mesh"])
+    errs = [rel_err(o, S_ref) for o in out]
+    print(f"nao={nao} ns={spins} slices={slices}: separate {errs[0]:.2e}, fused {errs[1]:.2e}, fused vs separate "
+          f"{rel_err(out[1], out[0]):.2e}", flush=True)
+    assert max(errs) < {3: 1e-4, 4: TOL_SPLIT, 5: 1e-10}[slices]
+    if spins == 1:
+        assert np.array_equal(out[0], out[1])
+    assert rel_err(out[1], out[0]) < {3: 1e-4, 4: 1e-9, 5: 1e-10}[slices]
