@@ -1063,7 +1063,7 @@ bool gw_hip_kernel::sigma_upper(bool split) const {
 
 // The fused P0 prep + slicing kernels take one or two collinear spin blocks: z_prep_kernel as far as their G blocks
 // and a quad's digits fit the work-group's LDS (with two and four slices: nao = 36), z_prep16_kernel always.  Of
-// the sizes between, prep and slicing in two kernels at nao = 40, two spin blocks, nk = 8, naux = 300: 214 ms an
+// the sizes between, prep and slicing in two kernels at nao = 40, two spin blocks, nk = 8, naux = 300: 175 ms an
 // evaluation, 228 with the 16-wide fused kernel and epilogue that this size had before.
 bool gw_hip_kernel::fused_p0() const {
   if (d_.pns != 1 || d_.pseudo_ns > 2 || d_.nao > kFusedMaxNao || orb_gemm()) return false;

@@ -571,11 +571,13 @@ inline bool z_prep_fits(int nb4, int sb, int ns, int kc) {
 // first product.  The four Q of a quad keep
 // separate sums, added at the end together with those of the QW waves over other quads.
 // Work-groups are as small as the sets of columns allow, so that a wave with less to do leaves its place to
-// the next one: one set per work-group up to nao = 32 (M takes at most 16 KB of LDS), four above, with one
-// wave per SIMD and the whole register file each.
+// the next one: one set per work-group up to nao = 48 (M takes at most 36 KB of LDS, four work-groups a CU), four
+// above; from nao = 33 on with one wave per SIMD and the whole register file each.  With four sets to a work-group
+// the second one of five or six sets holds four SIMDs for one or two waves: two spin blocks at nao = 40 (nk = 8,
+// naux = 300, split precision) 13.8 ms per launch against 9.0, one at nao = 48 10.5 against 8.3.
 template <int NB4>
 struct RedCfg {
-  static constexpr int SETS = (NB4 + 1) / 2, WS = NB4 <= 8 ? 1 : 4, GROUPS = (SETS + WS - 1) / WS;
+  static constexpr int SETS = (NB4 + 1) / 2, WS = NB4 <= 12 ? 1 : 4, GROUPS = (SETS + WS - 1) / WS;
   static constexpr int QW = NB4 <= 2 ? 4 : (NB4 <= 4 ? 2 : 1);
   static constexpr int N4 = 4 * NB4, NT = 64 * WS * QW, WPE = NB4 <= 8 ? 2 : 1;
 };
