@@ -166,7 +166,7 @@ void gw_hip_kernel::hf_device(const double2* dm, const double2* S, double madelu
   Event ex0, ex1;
   float ex_ms = 0.f;
   for (int64_t s = 0; s < nspin; ++s) {
-    if (orb_gemm()) {
+    if (hf_gemm()) {
       GWHIP_CHECK(hipEventRecord(ex0, stream_));
       hf_exchange_gemm(dm + s * nk * nso2, nblk);
       GWHIP_CHECK(hipEventRecord(ex1, stream_));
@@ -175,7 +175,7 @@ void gw_hip_kernel::hf_device(const double2* dm, const double2* S, double madelu
       GWHIP_CHECK(hipEventElapsedTime(&m, ex0, ex1));
       ex_ms += m;
     }
-    for (int bl = 0; bl < nblk && !orb_gemm(); ++bl) {
+    for (int bl = 0; bl < nblk && !hf_gemm(); ++bl) {
       const int64_t ro = (bl == 1) ? nao : 0, co = (bl == 0) ? 0 : nao;  // aa, bb, ab
       HfExchangeArgs a{};
       a.nao = (int)nao; a.nso = (int)nso; a.nk = (int)nk; a.NQ = (int)NQ;
@@ -186,8 +186,10 @@ void gw_hip_kernel::hf_device(const double2* dm, const double2* S, double madelu
       GWHIP_CHECK(hipEventRecord(ex0, stream_));
       orb_dispatch([&](auto nb) {
         constexpr int NB4 = decltype(nb)::value;
-        const dim3 g((unsigned)nk, 1, (unsigned)nk * HfReduce<NB4>::GROUPS);
-        launch_orb(hf_exchange_kernel<NB4>, a, g, HfReduce<NB4>::NT, HfReduce<NB4>::lds_bytes(), stream_);
+        if constexpr (4 * NB4 <= kHfMaxNao) {
+          const dim3 g((unsigned)nk, 1, (unsigned)nk * HfReduce<NB4>::GROUPS);
+          launch_orb(hf_exchange_kernel<NB4>, a, g, HfReduce<NB4>::NT, HfReduce<NB4>::lds_bytes(), stream_);
+        }
       });
       GWHIP_CHECK(hipEventRecord(ex1, stream_));
       GWHIP_CHECK(hipEventSynchronize(ex1));

@@ -198,8 +198,8 @@ public:
   // buffers of the GEMM form of the orbital contractions and the Sigma epilogue's partial sums
   // over Q ranges (full mesh); allocates, so call before a capture
   void ensure_orb_buffers();
-  // the register-chained orbital kernels handle nao up to 3 x 16
-  static constexpr int64_t kOrbMaxNao = 64, kVjpMaxNao = 48, kFusedMaxNao = 48;
+  // largest nao of the register-chained orbital kernels
+  static constexpr int64_t kOrbMaxNao = 64, kVjpMaxNao = 48, kHfMaxNao = 48, kFusedMaxNao = 48;
   bool has_inputs() const { return grid_set_ && v_set_; }
   // after the stream has drained: whether the last evaluation's Dyson step met a matrix I - P0
   // that is not positive definite
@@ -342,8 +342,11 @@ private:
   std::vector<int> q0_samples() const;
   void apply_q0(double2* Sigma, const double2* G, int64_t nkS);
   void p0_prep(int64_t q, const double2* G, int64_t t0, int64_t tc, int qpw, int64_t nq = 1);
-  // orbital contractions as batched GEMMs (nao > 64, or tuning orb_gemm); the VJP's from nao > 48 on
+  // orbital contractions as batched GEMMs (nao > 64, or tuning orb_gemm); the exchange's and the VJP's from nao > 48
+  // on.  Exchange there, naux = 200: GEMMs 1.24 ms at nk = 8, nao = 52 and 13.5 at nk = 27, nao = 64; the exchange
+  // kernel, whose fourteen or sixteen blocks leave one wave per SIMD, 1.96 and 15.8.
   bool orb_gemm() const { return d_.nao > kOrbMaxNao || tune_.orb_gemm != 0; }
+  bool hf_gemm() const { return d_.nao > kHfMaxNao || tune_.orb_gemm != 0; }
   bool vjp_gemm() const { return d_.nao > kVjpMaxNao || tune_.orb_gemm != 0; }
   void p0_prep_gemm(int64_t q, const double2* G, int64_t t0, int64_t tc);
   void sigma_epi_gemm(const double2* G, double2* Sigma, const SigmaRows& r, int64_t t0, int64_t tc, double scale);

@@ -117,3 +117,18 @@ def test_hf_gemm_form(c):
     assert rel_err(F, F_ref) < 1e-10
     if not c["gemm_only"]:
         assert rel_err(F, F_kern) < 1e-13
+
+
+@pytest.mark.parametrize("nao", [49, 64])
+def test_exchange_above_48_is_the_gemm_form(nao):
+    """By itself above nao = 48, where the exchange kernel is slower: the same bits as with the GEMM form asked for."""
+    dm, Vp, S, mad = random_system(3, nao, nao, 1, 6, 700 + nao)
+    k = _kernel(3, nao, nao, 1, 6, mesh=(3, 1, 1))
+    try:
+        k.upload_V(Vp)
+        F = k.hf(dm, S, mad)
+        k.set_tuning(orbital_gemm=1)
+        F_gemm = k.hf(dm, S, mad)
+    finally:
+        k.close()
+    assert np.array_equal(F, F_gemm)
