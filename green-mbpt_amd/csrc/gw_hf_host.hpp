@@ -177,20 +177,31 @@ void gw_hip_kernel::hf_device(const double2* dm, const double2* S, double madelu
     }
     for (int bl = 0; bl < nblk && !hf_gemm(); ++bl) {
       const int64_t ro = (bl == 1) ? nao : 0, co = (bl == 0) ? 0 : nao;  // aa, bb, ab
-      HfExchangeArgs a{};
-      a.nao = (int)nao; a.nso = (int)nso; a.nk = (int)nk; a.NQ = (int)NQ;
-      a.dm = dm + s * nk * nso2 + ro * nso + co;
-      a.V = Vq_; a.X = hf_x_ + bl * nk * nk * nao2;
-      a.kplus = kplus_tab_; a.adj = adj_x_dev_;
-      a.herm = bl == 2 ? nullptr : hf_herm_;
       GWHIP_CHECK(hipEventRecord(ex0, stream_));
-      orb_dispatch([&](auto nb) {
-        constexpr int NB4 = decltype(nb)::value;
-        if constexpr (4 * NB4 <= kHfMaxNao) {
-          const dim3 g((unsigned)nk, 1, (unsigned)nk * HfReduce<NB4>::GROUPS);
-          launch_orb(hf_exchange_kernel<NB4>, a, g, HfReduce<NB4>::NT, HfReduce<NB4>::lds_bytes(), stream_);
-        }
-      });
+      if (hf_16()) {
+        const OrbOp A{Vq_, nk * NQ * nao2, NQ * nao2, nao2, nao, 1, 0, 0};  // V(k, k+q)_Q (i, a)
+        const OrbOp C{Vq_, nk * NQ * nao2, NQ * nao2, nao2, 1, nao, 0, 1};  // V(k, k+q)_Q^H (b, j)
+        const OrbOp M{dm + s * nk * nso2 + ro * nso + co, 0, nso2, 0, nso, 1, 1, 0};
+        const OrbOut O{hf_x_ + bl * nk * nk * nao2, nk * nao2, nao2, 0, nao, 1, 0};
+        OrbArgs oa{(int)nao, (int)NQ, (int)nk, 4, kplus_tab_, kminus_tab_, 1.0};
+        oa.kmap_st = nk;
+        zero(hf_x_ + bl * nk * nk * nao2, nk * nk * nao2);
+        launch_reduce<true>(3, dim3((unsigned)nk, (unsigned)nk), stream_, oa, A, M, C, O);
+      } else {
+        HfExchangeArgs a{};
+        a.nao = (int)nao; a.nso = (int)nso; a.nk = (int)nk; a.NQ = (int)NQ;
+        a.dm = dm + s * nk * nso2 + ro * nso + co;
+        a.V = Vq_; a.X = hf_x_ + bl * nk * nk * nao2;
+        a.kplus = kplus_tab_; a.adj = adj_x_dev_;
+        a.herm = bl == 2 ? nullptr : hf_herm_;
+        orb_dispatch([&](auto nb) {
+          constexpr int NB4 = decltype(nb)::value;
+          if constexpr (4 * NB4 <= kHfMaxNao) {
+            const dim3 g((unsigned)nk, 1, (unsigned)nk * HfReduce<NB4>::GROUPS);
+            launch_orb(hf_exchange_kernel<NB4>, a, g, HfReduce<NB4>::NT, HfReduce<NB4>::lds_bytes(), stream_);
+          }
+        });
+      }
       GWHIP_CHECK(hipEventRecord(ex1, stream_));
       GWHIP_CHECK(hipEventSynchronize(ex1));
       float m = 0.f;

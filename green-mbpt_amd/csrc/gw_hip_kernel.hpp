@@ -347,6 +347,16 @@ private:
   // kernel, whose fourteen or sixteen blocks leave one wave per SIMD, 1.96 and 15.8.
   bool orb_gemm() const { return d_.nao > kOrbMaxNao || tune_.orb_gemm != 0; }
   bool hf_gemm() const { return d_.nao > kHfMaxNao || tune_.orb_gemm != 0; }
+  // The exchange of nao 41 to 48 as one work-group of four waves per pair on 16x16x4 products (launch_reduce), or
+  // as six single waves per pair (hf_exchange_kernel).  A wave of either has a SIMD to itself, and a round of the
+  // first takes 1.5 times a round of the second (2.05 against 1.33 ms at nao = 44, naux = 200), so the one with the
+  // fewer rounds so weighted: nk = 14, 16, 27, 48 the first, others to 64 the second.  nao = 44, first and second:
+  // nk = 27, naux = 200 6.2 and 6.7 ms; nk = 16, naux = 300 3.2 and 4.2; nk = 18 4.1 and 2.8; nk = 36, naux = 150
+  // 9.3 and 8.2.
+  bool hf_16() const {
+    const int64_t pairs = d_.nk * d_.nk;
+    return d_.nao > 40 && 3 * ceil_div(pairs, 256) < 2 * ceil_div(6 * pairs, 1024);
+  }
   bool vjp_gemm() const { return d_.nao > kVjpMaxNao || tune_.orb_gemm != 0; }
   void p0_prep_gemm(int64_t q, const double2* G, int64_t t0, int64_t tc);
   void sigma_epi_gemm(const double2* G, double2* Sigma, const SigmaRows& r, int64_t t0, int64_t tc, double scale);

@@ -132,3 +132,23 @@ def test_exchange_above_48_is_the_gemm_form(nao):
     finally:
         k.close()
     assert np.array_equal(F, F_gemm)
+
+
+@pytest.mark.parametrize("c", [
+    dict(nk=13, nao=45, nso=45, ns=1), dict(nk=14, nao=41, nso=41, ns=2), dict(nk=14, nao=48, nso=48, ns=1),
+    dict(nk=14, nao=45, nso=90, ns=1), dict(nk=17, nao=44, nso=44, ns=1),
+])
+@pytest.mark.parametrize("hermitian", [True, False])
+def test_exchange_of_three_blocks(c, hermitian):
+    """nao of 41 to 48, where the number of pairs decides between the two exchange kernels."""
+    dm, Vp, S, mad = random_system(c["nk"], c["nao"], c["nso"], c["ns"], 3, 800 + c["nk"])
+    if not hermitian:
+        rng = np.random.default_rng(c["nk"])
+        dm = dm + 0.1 * (rng.standard_normal(dm.shape) + 1j * rng.standard_normal(dm.shape))
+    k = _kernel(c["nk"], c["nao"], c["nso"], c["ns"], 3, mesh=(c["nk"], 1, 1))
+    try:
+        k.upload_V(Vp)
+        F = k.hf(dm, S, mad)
+    finally:
+        k.close()
+    assert rel_err(F, ho.hf_fock(dm, Vp, S, mad, c["nk"], c["nao"], c["nso"], c["ns"], 3)) < 1e-10
