@@ -153,15 +153,22 @@ void gw_hip_kernel::hf_device(const double2* dm, const double2* S, double madelu
   hipLaunchKernelGGL(hf_direct_add_kernel, dim3((unsigned)ceil_div(nmat * nao2, 256)), dim3(256), 0, stream_, hf_work_, Vd,
                      F, (int)nk, (int)NQ, (int)nao, (int)nso, (int)nspin, x2c ? 1 : 0);
   GWHIP_CHECK(hipGetLastError());
-  // a density matrix that is Hermitian to rounding makes the aa and bb exchange blocks Hermitian
-  hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(64), 0, stream_, reinterpret_cast<int*>(hcheck_), (int64_t)4);
-  hipLaunchKernelGGL(herm_check_kernel, dim3(herm_check_blocks(nmat * nso2)), dim3(256), 0, stream_, dm, nmat, (int)nso,
-                     hcheck_);
-  hipLaunchKernelGGL(herm_flag_kernel, dim3(1), dim3(1), 0, stream_, hcheck_, 1e-15, hf_herm_);
-  GWHIP_CHECK(hipGetLastError());
+  const int nblk = x2c ? 3 : 1;
+  // A density matrix that is Hermitian to rounding makes the aa and bb exchange blocks Hermitian, which saves the
+  // exchange kernel about a third of its time.  To find out takes three launches, 13 us of a Fock build, so only
+  // from about 70 us of exchange on, at 0.1 TFLOP/s for the work-groups of one CU.  Without and with the check:
+  // nk = 1, nao = 4, naux = 20 66 and 80 us; nk = 1, nao = 16, naux = 100 (66 us by this estimate) 119 and 128.
+  const bool check = !hf_gemm() && !hf_16() &&
+                     16.0 * NQ * nao2 * nao * nspin * (x2c ? 2 : 1) * ceil_div(nk * nk, 256) > 7e6;
+  if (check) {
+    hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(64), 0, stream_, reinterpret_cast<int*>(hcheck_), (int64_t)4);
+    hipLaunchKernelGGL(herm_check_kernel, dim3(herm_check_blocks(nmat * nso2)), dim3(256), 0, stream_, dm, nmat, (int)nso,
+                       hcheck_);
+    hipLaunchKernelGGL(herm_flag_kernel, dim3(1), dim3(1), 0, stream_, hcheck_, 1e-15, hf_herm_);
+    GWHIP_CHECK(hipGetLastError());
+  }
   // exchange: X[blk][q][k] = sum_Q V(k, k+q)_Q dm(k+q)_blk V(k, k+q)_Q^H for all (k, q) in one
   // launch per spin block, then F(k)_blk -= pref/nk sum_q X[blk][q][k] (fixed order in q)
-  const int nblk = x2c ? 3 : 1;
   if (!hf_x_) hf_x_ = dalloc<double2>((size_t)nblk * nk * nk * nao2);
   Event ex0, ex1;
   float ex_ms = 0.f;
@@ -193,7 +200,7 @@ void gw_hip_kernel::hf_device(const double2* dm, const double2* S, double madelu
         a.dm = dm + s * nk * nso2 + ro * nso + co;
         a.V = Vq_; a.X = hf_x_ + bl * nk * nk * nao2;
         a.kplus = kplus_tab_; a.adj = adj_x_dev_;
-        a.herm = bl == 2 ? nullptr : hf_herm_;
+        a.herm = check && bl != 2 ? hf_herm_ : nullptr;
         orb_dispatch([&](auto nb) {
           constexpr int NB4 = decltype(nb)::value;
           if constexpr (4 * NB4 <= kHfMaxNao) {

@@ -152,3 +152,20 @@ def test_exchange_of_three_blocks(c, hermitian):
     finally:
         k.close()
     assert rel_err(F, ho.hf_fock(dm, Vp, S, mad, c["nk"], c["nao"], c["nso"], c["ns"], 3)) < 1e-10
+
+
+@pytest.mark.parametrize("nao", [3, 5, 9, 13, 17, 21, 28, 29, 33, 37, 40, 41, 48])
+@pytest.mark.parametrize("work", [6e6, 8e6])
+def test_hermitian_density_matrix(nao, work):
+    """On both sides of the work from which on a Hermitian density matrix is looked for, at the block counts of the
+    exchange kernel."""
+    NQ = int(work / (16.0 * nao ** 3)) + 1
+    dm, Vp, S, mad = random_system(2, nao, nao, 1, NQ, 900 + nao)
+    dm = 0.5 * (dm + np.conj(np.swapaxes(dm, -1, -2)))
+    k = _kernel(2, nao, nao, 1, NQ, mesh=(2, 1, 1))
+    try:
+        k.upload_V(Vp)
+        F = k.hf(dm, S, mad)
+    finally:
+        k.close()
+    assert rel_err(F, ho.hf_fock(dm, Vp, S, mad, 2, nao, nao, 1, NQ)) < 1e-10
