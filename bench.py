@@ -28,27 +28,56 @@ WORKLOAD = dict(nk=64, mesh=(4, 4, 4), nao=26, NQ=300, ns=1, beta=100.0, lam=1e4
 
 # HBM bytes per launch of the main kernels on this workload, from two rocprofv3 --pmc runs
 # (FETCH_SIZE, WRITE_SIZE in KiB per dispatch) of `bench.py --steps 1 --warmup 0 --no-cpu
-# [--no-check | --precision fp64] --no-autotune` with the same build; each scaled by what the
+# [--no-check | --precision fp64] --no-autotune`; each scaled by what the
 # counter reads for a plain 2 GiB device copy (bench.py --copy-calibration): FETCH_SIZE reads 0.5x
 # the bytes the copy reads, WRITE_SIZE 1.0x the bytes it writes.
 # Source: profiles/gw_sigma_nk64_nao26_naux300_hbm_traffic.md
 PMC_PER_LAUNCH_KIB = {
-    "split": {"Sigma GEMM": (3.5381e6, 1.0229e7), "Sigma epilogue": (5.5368e6, 5.1620e4),
-              "P0 GEMM": (7.7133e6, 6.8067e5), "P0 prep": (6.9709e5, 5.3279e6),  # P0 GEMM: 16 launches per q
-              "Dyson inverse": (5.7157e7, 6.7429e7)},  # every kernel of the inverse, one evaluation
-    "fp64": {"Sigma GEMM": (2.9702e7, 1.0307e7), "Sigma epilogue": (5.5368e6, 5.1620e4),
-             "P0 GEMM": (2.2308e7, 4.2419e4), "P0 prep": (7.4680e5, 1.0163e7),
-             "Dyson inverse": (5.7126e7, 6.7429e7)},
+    "split": {"Sigma GEMM": (3.5562e6, 1.0177e7), "Sigma epilogue": (1.0584e7, 3.8872e4),
+              "P0 GEMM": (1.1288e7, 1.2693e6), "P0 prep": (6.9734e5, 5.3100e6),  # P0 GEMM with its partial sums
+              "Dyson inverse": (5.3400e7, 6.7701e7)},  # every kernel of the inverse, one evaluation
+    "fp64": {"Sigma GEMM": (1.5028e7, 1.0210e7), "Sigma epilogue": (1.0703e7, 6.8068e4),
+             "P0 GEMM": (1.7954e7, 4.2527e4), "P0 prep": (7.4748e5, 1.0187e7),
+             "Dyson inverse": (5.3410e7, 6.7695e7)},
 }
 PMC_CALIBRATION = (0.5, 1.0)
 PMC_SOURCE = "profiles/gw_sigma_nk64_nao26_naux300_hbm_traffic.md"
+# the parameters that those runs had, per family: other values, no traffic figure
+PMC_TUNING = {"Sigma GEMM": dict(sigma_tile=0, sigma_group=4, sigma_split_tile=4),
+              "P0 GEMM": dict(p0_tile=0, p0_group=1, p0_split_tile=4, p0_kchunks=0),
+              "P0 prep": dict(aux_per_wave=4, p0_fused_slices=1)}
 # the int8 GEMM kernel of each block tile (tuning keys p0_split_tile / sigma_split_tile)
 OZAKI_KERNEL = {2: "zgemm_ozaki_pipe_kernel", 4: "zgemm_ozaki32_kernel"}
-# the register Sigma epilogue of each form (tuning key epi_form) at nao = 26; the profiled traffic
-# figures belong to form 1
+F64_TILE = {0: (64, 64), 1: (128, 64), 2: (64, 128)}
+# the Sigma epilogue by the value of the tuning key epi_form while that chose among three kernels; kernel_labels
+# has the one that is left
 EPI_KERNEL = {1: "sigma_epi4_kernel<7> (Sigma += (V G) R, FP64 4x4x4 MFMA)",
               2: "sigma_epi4w_kernel<7,2,4> (Sigma += (V G) R, FP64 4x4x4 MFMA, one i group per wave)",
               3: "sigma_epi_mfma_kernel<2,double> (Sigma += (V G) R, FP64 16x16x4 MFMA)"}
+
+
+def kernel_labels(split, w, slices, tuning):
+    """The kernel that each family launches for the workload (nao <= 40) with these parameters."""
+    nb4 = -(-w["nao"] // 4)
+    prep = slices if split and tuning["p0_fused_slices"] else 0
+    if split:
+        one = "true" if tuning["p0_kchunks"] == 1 else "false"  # k chunks of a launch
+        sigma = f"{OZAKI_KERNEL[tuning['sigma_split_tile']]}<{slices}, true> (R = P-tilde conj(V), int8 slices)"
+        p0 = f"{OZAKI_KERNEL[tuning['p0_split_tile']]}<{slices}, {one}> (P0 = Z conj(V)^T, int8 slices)"
+    else:
+        f64 = {t: "zgemm_f64_kernel<%d, %d>" % mn for t, mn in F64_TILE.items()}
+        # the product of one triangle has 64-row tiles whatever the tile asked for
+        sigma = f64[tuning["sigma_tile"] if tuning["sigma_tile"] != 1 else 0] + \
+            " (R = P-tilde conj(V) of one triangle, FP64 MFMA)"
+        p0 = f64[tuning["p0_tile"]] + " (P0 = Z conj(V)^T, FP64 MFMA)"
+    return {"Sigma GEMM": sigma, "P0 GEMM": p0,
+            "Sigma epilogue": f"sigma_epi_kernel<{nb4}> (Sigma += (V G) R, FP64 4x4x4 MFMA)",
+            "P0 prep": f"z_prep_kernel<{nb4}, {prep}> (Z = Gb V Gq, FP64 4x4x4 MFMA)"}
+
+
+def upper_tiles(n, bm, bn):
+    """Elements of the bm x bn block tiles of an n x n product that do not lie wholly below the diagonal."""
+    return bm * bn * sum(m < c + bn for m in range(0, n, bm) for c in range(0, n, bn))
 
 
 def algorithmic_flops(nk, nao, NQ, nts, nw_b, pseudo_ns=1):
@@ -61,12 +90,13 @@ def algorithmic_flops(nk, nao, NQ, nts, nw_b, pseudo_ns=1):
     return dict(P0=f_p0, Sigma=f_s, Dyson=f_dys, IR=f_ir, total=f_p0 + f_s + f_dys + f_ir)
 
 
-def stage_work(w, T, slices):
+def stage_work(w, T, slices, oz_tile=None, f64_tile=None):
     """Work of each kernel family over one Sigma evaluation of the full mesh (nq = nk):
     algorithmic flops (the reference's GEMM count, 8 flops per complex MAC; for the two big GEMMs on
     the half tau grid, which is all the reference computes for P0 and all that R = P-tilde conj(V)
-    needs), int8 operations issued by the split-precision GEMMs, and algorithmic bytes (each operand
-    read once and each result written once, in the representation the kernel reads and writes)."""
+    needs), operations issued by those GEMMs (int8 in split precision; oz_tile, f64_tile: P0's block tile), and
+    algorithmic bytes (each operand read once and each result written once, in the representation the kernel reads
+    and writes)."""
     nk, nao, NQ, nts, nwb = w["nk"], w["nao"], w["NQ"], T.nts, T.nw_b
     half, nao2, B = nts // 2, nao * nao, 16.0
     pairs = slices * (slices + 1) // 2
@@ -74,13 +104,17 @@ def stage_work(w, T, slices):
     kc_p = -(-nao2 // 64) * 64
     sl = 2 * slices                                   # int8 bytes per element and K step: planes x slices
     V = nk * NQ * nao2 * B                            # V(k, k +- q) of one q
+    # G is Hermitian: the FP64 Sigma product sums K from each 64-row tile's first row on, P0 takes the upper tiles
+    half_k = sum(64 * (-(-(NQ - m) // 8) * 8) for m in range(0, NQ, 64))
     out = {
         "Sigma GEMM": dict(flops=8.0 * NQ * NQ * nk * nao2 * half * nk,
                            issued=2.0 * 4 * pairs * NQ * kc_s * nk * nao2 * half * nk,
+                           issued_fp64=8.0 * half_k * nk * nao2 * half * nk,
                            bytes_fp64=nk * (half * NQ * NQ * B + V + half * nk * NQ * nao2 * B),
                            bytes_split=nk * (half * NQ * sl * kc_s + nk * nao2 * sl * kc_s + half * nk * NQ * nao2 * B)),
         "P0 GEMM": dict(flops=8.0 * NQ * NQ * nk * nao2 * half * nk,
-                        issued=2.0 * 4 * pairs * NQ * NQ * nk * kc_p * half * nk,
+                        issued=2.0 * 4 * pairs * upper_tiles(NQ, *(oz_tile or (32, 64))) * nk * kc_p * half * nk,
+                        issued_fp64=8.0 * upper_tiles(NQ, *(f64_tile or (64, 64))) * nk * nao2 * half * nk,
                         bytes_fp64=nk * (half * nk * NQ * nao2 * B + V + half * NQ * NQ * B),
                         bytes_split=nk * (half * NQ * nk * sl * kc_p + NQ * nk * sl * kc_p + half * NQ * NQ * B)),
         "Sigma epilogue": dict(flops=16.0 * NQ * nao ** 3 * nk * nts * nk, issued=None,
@@ -94,28 +128,27 @@ def stage_work(w, T, slices):
     return out
 
 
-def roofline(stats, precision, w, T, slices, tuning, steps=1):
+def roofline(stats, precision, w, T, slices, tuning, steps=1, labels=None):
     """Roofline of the kernel family with the largest share of the step, from the per-launch times
     measured with HIP events on the library's stream: achieved = algorithmic flops per launch / mean
     launch time, frac = achieved / the published peak of the arithmetic the kernel uses (int8 5.0 POP/s
-    for the split GEMMs, FP64 78.6 TFLOP/s otherwise); issued_frac = int8 operations issued / time /
-    peak; traffic = the rocprofv3 counter bytes per launch of this build, traffic_ratio = traffic /
+    for the split GEMMs, FP64 78.6 TFLOP/s otherwise), from the operations issued where a product of a
+    Hermitian matrix issues fewer than the algorithm counts; issued_frac = operations issued / time /
+    peak; traffic = the rocprofv3 counter bytes per launch, traffic_ratio = traffic /
     algorithmic bytes.  Every family's figures are listed under all_stages.  stats holds launch counts
-    and times summed over `steps` evaluations; the work figures are per evaluation."""
-    work = stage_work(w, T, slices)
+    and times summed over `steps` evaluations; the work figures are per evaluation.  labels: the kernels' names
+    (kernel_labels)."""
     split = precision == "split"
+    p0_oz = {2: (32, 64), 4: (64, 64)}[tuning.get("p0_split_tile", 2)]
+    work = stage_work(w, T, slices, p0_oz, F64_TILE[tuning.get("p0_tile", 0)])
     int8 = {"Sigma GEMM", "P0 GEMM"} if split else set()
-    s_kernel = OZAKI_KERNEL.get(tuning.get("sigma_split_tile", 2), "?")
-    p_kernel = OZAKI_KERNEL.get(tuning.get("p0_split_tile", 2), "?")
-    names = {"Sigma GEMM": (f"{s_kernel}<{slices}> (R = P-tilde conj(V), int8 slices)"
-                            if split else "zgemm_f64_kernel<64,64,true,false> (R = P-tilde conj(V), FP64 MFMA)"),
-             "P0 GEMM": (f"{p_kernel}<{slices}> (P0 = Z conj(V)^T, int8 slices)"
-                         if split else "zgemm_f64_kernel<64,64,true,true> (P0 = Z conj(V)^T, FP64 MFMA)"),
-             "Sigma epilogue": EPI_KERNEL.get(tuning.get("epi_form", 1) or 1, "?"),
-             "P0 prep": (f"z_prep_slice_kernel<2,{slices},1>" if split else "z_prep_mfma_kernel<2,double>") +
-                        " (Z = Gb V Gq, FP64 MFMA)",
+    names = {"Sigma GEMM": f"{OZAKI_KERNEL.get(tuning.get('sigma_split_tile', 2), '?')}<{slices}>"
+                           if split else "zgemm_f64_kernel",
+             "P0 GEMM": f"{OZAKI_KERNEL.get(tuning.get('p0_split_tile', 2), '?')}<{slices}>" if split else "zgemm_f64_kernel",
+             "Sigma epilogue": EPI_KERNEL.get(tuning.get("epi_form", 1) or 1, "?"), "P0 prep": "z_prep_kernel",
              "Dyson inverse": "block_inverse: Hermitian block Gauss-Jordan, gj_inverse_kernel pivots + "
                               "zgemm_f64_kernel upper-tile updates ((I - P0)^-1 per (q, Omega), FP64)"}
+    names.update(labels or {})
     rows = {}
     for name, (n, ms) in stats.items():
         if not n or name not in work:
@@ -131,12 +164,16 @@ def roofline(stats, precision, w, T, slices, tuning, steps=1):
              "peak_unit": "TOPS (int8)" if name in int8 else "TFLOP/s (FP64)",
              "frac": flops / t / 1e12 / peak, "algorithmic_flops_per_launch": flops,
              "algorithmic_bytes": alg_bytes}
-        if name in int8 and wk["issued"]:
-            r["issued_tops"] = wk["issued"] * per / t / 1e12
-            r["issued_frac"] = r["issued_tops"] / peak
+        issued = wk["issued"] if name in int8 else wk.get("issued_fp64")
+        if issued:
+            r["issued_tops" if name in int8 else "issued_tflops"] = issued * per / t / 1e12
+            r["issued_frac"] = issued * per / t / 1e12 / peak
+            r["frac"] = min(r["frac"], r["issued_frac"])
         pmc = PMC_PER_LAUNCH_KIB.get(precision, {}).get(name)
-        if name == "Sigma epilogue" and (tuning.get("epi_form", 1) or 1) != 1:
-            pmc = None  # profiled for the 4x4x4 all-groups form only
+        if any(tuning.get(k_, v_) != v_ for k_, v_ in PMC_TUNING.get(name, {}).items()):
+            pmc = None
+        if not labels and name == "Sigma epilogue" and (tuning.get("epi_form", 1) or 1) != 1:
+            pmc = None
         if pmc is not None:
             tr = 1024.0 * (pmc[0] / PMC_CALIBRATION[0] + pmc[1] / PMC_CALIBRATION[1])
             r.update({"traffic": tr, "traffic_ratio": tr / alg_bytes, "traffic_source": PMC_SOURCE})
@@ -275,7 +312,7 @@ def main():
     ap.add_argument("--no-autotune", action="store_true",
                     help="keep the default launch parameters (the autotuner's choice for this workload)")
     ap.add_argument("--tuning", default="",
-                    help="launch parameters to set after autotuning, e.g. p0_split_tile=3,sigma_split_tile=3")
+                    help="launch parameters to set after autotuning, e.g. p0_split_tile=2,sigma_split_tile=2")
     ap.add_argument("--capacity", action="store_true",
                     help="one split-precision evaluation at nk=64, nao=64, naux=300 (device memory held, time)")
     ap.add_argument("--copy-calibration", action="store_true",
@@ -347,7 +384,9 @@ def main():
     regions = k.timings()
     fl = algorithmic_flops(w["nk"], w["nao"], w["NQ"], T.nts, T.nw_b)
     S_host = S_d.cpu().numpy().view(np.complex128).copy()
-    roof = roofline(stats, args.precision, w, T, args.slices, k.tuning(), args.steps)
+    tuning = k.tuning()
+    roof = roofline(stats, args.precision, w, T, args.slices, tuning, args.steps,
+                    kernel_labels(args.precision == "split", w, args.slices, tuning))
 
     check = {}
     if prec == gl.PREC_SPLIT and not args.no_check:
@@ -534,7 +573,7 @@ def bench_hf(args):
     flops = 8.0 * 2 * nk * nk * NQ * nao ** 3         # per launch: two nao^3 complex products per (k, k', Q)
     vbytes = 16.0 * nk * nk * NQ * nao * nao           # V(k, k') read once per launch
     roof = {"bound": "mfma", "achieved": flops / avg_s / 1e12, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
-            "kernel": "orb_reduce_kernel<2,true> (exchange sum_Q V dm V^H over all (k, q), FP64 MFMA)",
+            "kernel": "hf_exchange_kernel<7> (exchange sum_Q V dm V^H over all (k, q), FP64 MFMA)",
             "launches": ex_n, "avg_launch_ms": avg_s * 1e3, "algorithmic_bytes": vbytes,
             "hbm_GBps_algorithmic": vbytes / avg_s / 1e9, "traffic": None}
     roof["frac"] = roof["achieved"] / roof["peak"]

@@ -65,3 +65,43 @@ def test_epilogue_label_and_traffic_follow_the_tuned_form():
     assert r1["kernel"].startswith("sigma_epi4_kernel<7>") and r1["traffic"] > 0
     assert r3["kernel"].startswith("sigma_epi_mfma_kernel<2,double>") and r3["traffic"] is None
     assert r1["achieved"] == pytest.approx(r3["achieved"])
+
+
+DEFAULTS = dict(p0_tile=0, sigma_tile=0, aux_per_wave=4, p0_group=1, sigma_group=4, p0_split_tile=4, sigma_split_tile=4,
+                p0_fused_slices=1, orbital_gemm=0, p0_kchunks=0, epi_form=0)
+
+
+@pytest.mark.parametrize("precision", ["split", "fp64"])
+@pytest.mark.parametrize("change", [dict(), dict(p0_split_tile=2, sigma_split_tile=2, p0_tile=1, sigma_tile=2),
+                                    dict(p0_fused_slices=0, p0_tile=2, sigma_tile=1, epi_form=3)])
+def test_printed_kernels_are_in_the_source(precision, change):
+    import re
+
+    b = _bench()
+    tuning = dict(DEFAULTS, **change)
+    src = ""
+    csrc = os.path.join(ROOT, "green-mbpt_amd", "csrc")
+    for f in os.listdir(csrc):
+        with open(os.path.join(csrc, f)) as fh:
+            src += fh.read()
+    kernels = set(re.findall(r"__global__[^;{]*?\b(\w+_kernel)\(", src))
+    assert len(kernels) > 20
+    labels = b.kernel_labels(precision == "split", b.WORKLOAD, 4, tuning)
+    r = b.roofline(_stats(1), precision, b.WORKLOAD, T, 4, tuning, 1, labels)["all_stages"]
+    for name, row in r.items():
+        found = re.findall(r"\w+_kernel\b", row["kernel"])
+        assert found and set(found) <= kernels, (name, row["kernel"])
+    assert r["Sigma epilogue"]["traffic"] > 0
+    assert (r["Sigma GEMM"]["traffic"] is None) == (change.get("sigma_split_tile", 4) != 4 or change.get("sigma_tile", 0) != 0)
+
+
+def test_fp64_fraction_is_of_the_work_issued():
+    """Half of P-tilde and the upper tiles of P0: NQ = 300 in tiles of 64 issues 880/300 x 64/300 and 15/25 x
+    (320/300)^2 of the algorithm's products; at 16.5 and 24.0 ms per launch neither exceeds the peak."""
+    b = _bench()
+    st = _stats(1)
+    st["Sigma GEMM"], st["P0 GEMM"] = [64, 64 * 16.5], [64, 64 * 24.0]
+    r = b.roofline(st, "fp64", b.WORKLOAD, T, 4, DEFAULTS, 1)["all_stages"]
+    for name, ratio in (("Sigma GEMM", 880 / 300 * 64 / 300), ("P0 GEMM", 15 / 25 * (320 / 300) ** 2)):
+        assert r[name]["issued_tflops"] == pytest.approx(r[name]["achieved"] * ratio)
+        assert r[name]["frac"] == pytest.approx(r[name]["issued_frac"]) and 0.5 < r[name]["frac"] < 1
