@@ -535,6 +535,16 @@ void gw_hip_kernel::orb_dispatch(F&& f) const {
   }
 }
 
+// f(std::integral_constant<int, NB>) for the 16-wide blocks of the P0 operand.
+template <typename F>
+void gw_hip_kernel::prep16_dispatch(F&& f) const {
+  switch (z_prep16_blocks(d_.nao, d_.pseudo_ns)) {
+    case 1: return f(std::integral_constant<int, 1>{});
+    case 2: return f(std::integral_constant<int, 2>{});
+    default: return f(std::integral_constant<int, 3>{});
+  }
+}
+
 namespace {
 template <typename K, typename A>
 void launch_orb(K kern, A& args, dim3 grid, int threads, size_t lds, hipStream_t st) {
@@ -566,15 +576,19 @@ void gw_hip_kernel::p0_prep(int64_t q, const double2* G, int64_t t0, int64_t tc,
   ZPrepArgs a = prep_args(q, G, t0, qpw);
   a.kn = (int)(nq * d_.nk);
   const dim3 grid((unsigned)ceil_div(d_.NQ, 4 * a.qpb), (unsigned)a.kn, (unsigned)tc);
-  if (z_prep16_takes(d_.nao)) {
+  if (z_prep16_blocks(d_.nao, d_.pseudo_ns)) {
     const int sb = d_.pseudo_ns > 1 ? 2 : 1;
-    for (a.s0 = 0; a.s0 < d_.pseudo_ns; a.s0 += sb)
-      launch_orb(sb == 2 ? z_prep16_kernel<0, 2> : z_prep16_kernel<0, 1>, a, grid, 256, z_prep16_lds_bytes(sb), stream_);
+    prep16_dispatch([&](auto nb) {
+      constexpr int NB = decltype(nb)::value;
+      for (a.s0 = 0; a.s0 < d_.pseudo_ns; a.s0 += sb)
+        launch_orb(sb == 2 ? z_prep16_kernel<NB, 0, 2> : z_prep16_kernel<NB, 0, 1>, a, grid, 256,
+                   z_prep16_lds_bytes(NB, sb), stream_);
+    });
     return;
   }
   orb_dispatch([&](auto nb) {
     constexpr int NB4 = decltype(nb)::value;
-    if constexpr (!z_prep16_takes(4 * NB4)) {
+    if constexpr (!z_prep16_blocks(4 * NB4, 4)) {
       const int sb = prep_spin_blocks(NB4, (int)d_.pseudo_ns);
       for (int s0 = 0; s0 < d_.pseudo_ns; s0 += sb) {
         a.s0 = s0;
@@ -613,17 +627,20 @@ void gw_hip_kernel::p0_prep_slice(int64_t q, const double2* G, int64_t t0, int64
   a.sb = (int)d_.pseudo_ns;
   const dim3 grid((unsigned)ceil_div(d_.NQ, 4 * a.qpb), (unsigned)d_.nk, (unsigned)tc);
   const int ns = split_ns_;
-  if (z_prep16_takes(d_.nao)) {
-    auto go = [&](auto k3, auto k4, auto k5) {
-      launch_orb(ns == 5 ? k5 : ns == 4 ? k4 : k3, a, grid, 256, z_prep16_lds_bytes(a.sb), stream_);
-    };
-    if (a.sb == 2) go(z_prep16_kernel<3, 2>, z_prep16_kernel<4, 2>, z_prep16_kernel<5, 2>);
-    else go(z_prep16_kernel<3, 1>, z_prep16_kernel<4, 1>, z_prep16_kernel<5, 1>);
+  if (z_prep16_blocks(d_.nao, d_.pseudo_ns)) {
+    prep16_dispatch([&](auto nb) {
+      constexpr int NB = decltype(nb)::value;
+      auto go = [&](auto k3, auto k4, auto k5) {
+        launch_orb(ns == 5 ? k5 : ns == 4 ? k4 : k3, a, grid, 256, z_prep16_lds_bytes(NB, a.sb), stream_);
+      };
+      if (a.sb == 2) go(z_prep16_kernel<NB, 3, 2>, z_prep16_kernel<NB, 4, 2>, z_prep16_kernel<NB, 5, 2>);
+      else go(z_prep16_kernel<NB, 3, 1>, z_prep16_kernel<NB, 4, 1>, z_prep16_kernel<NB, 5, 1>);
+    });
     return;
   }
   orb_dispatch([&](auto nb) {
     constexpr int NB4 = decltype(nb)::value;
-    if constexpr (NB4 <= kFusedMaxNao / 4 && !z_prep16_takes(4 * NB4)) {
+    if constexpr (NB4 <= kFusedMaxNao / 4 && !z_prep16_blocks(4 * NB4, 2)) {
       const size_t lds = z_prep_lds_bytes(NB4, a.sb, ns, (int)kc_p0_);
       if (ns == 5) launch_orb(z_prep_kernel<NB4, 5>, a, grid, OrbCfg<NB4>::NT, lds, stream_);
       else if (ns == 4) launch_orb(z_prep_kernel<NB4, 4>, a, grid, OrbCfg<NB4>::NT, lds, stream_);
@@ -1067,7 +1084,7 @@ bool gw_hip_kernel::sigma_upper(bool split) const {
 // evaluation, 228 with the 16-wide fused kernel and epilogue that this size had before.
 bool gw_hip_kernel::fused_p0() const {
   if (d_.pns != 1 || d_.pseudo_ns > 2 || d_.nao > kFusedMaxNao || orb_gemm()) return false;
-  if (z_prep16_takes(d_.nao)) return true;
+  if (z_prep16_blocks(d_.nao, d_.pseudo_ns)) return true;
   const int nb4 = (int)ceil_div(d_.nao, 4), kc = (int)ceil_div(d_.nao * d_.nao, 64) * 64;
   return z_prep_fits(nb4, (int)d_.pseudo_ns, split_ns_, kc);
 }

@@ -400,6 +400,8 @@ private:
   void finish_sigma(double2* Sigma, int64_t nkS, bool split);
   template <typename F>
   void orb_dispatch(F&& f) const;
+  template <typename F>
+  void prep16_dispatch(F&& f) const;
   void star_tables();
   const double2* star_rotate(int64_t iq, int64_t q);
   void solve_star_device(const double2* G_ibz, double2* Sigma_ibz, int precision);

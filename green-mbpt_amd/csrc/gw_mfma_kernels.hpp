@@ -18,8 +18,9 @@
 // point paired with itself is read in place, as its stored block need not be Hermitian to the last bit.
 // Measured (one MI355X, nk = 27, nao = 26, naux = 250, 100 tau, per launch): Sigma epilogue 4.5 ms in full
 // and 3.95 ms on the upper triangle (4.9 and 4.4 ms with the four products as one 16-wide group of i,
-// padded to 28 x 28 x 32); P0 prep 2.45 ms, 3.2 ms with the slicing (2.7 ms with 16x16x4 MFMAs, padded to 32).
-// Both wait for their per-Q operands: with those loads taken out 3.4, 2.75 and 1.6 ms.
+// padded to 28 x 28 x 32).  It waits for its per-Q operands: 3.4 and 2.75 ms with those loads taken out.
+// The P0 operand is the exception where nao nearly fills 16-wide blocks (z_prep16_kernel): there 2.6 ms on
+// v_mfma_f64_16x16x4 and 2.9 with the slicing, against 2.6 and 3.3 on the 4-wide blocks.
 //
 // Layouts (complex = double2):
 //   V [k][Q][p][m]  = V^Q_pm(k, k + q)     the resident integrals of one q
@@ -115,8 +116,8 @@ __device__ __forceinline__ void lds_fence() {
 // V_Q of the P0 prep, which all waves of a work-group need, is brought to LDS once, one slab of NB4 tiles
 // (4 m x 4 p x 4 Q, 1 KB in fragment order) at a time, the loads of a slab under the products of the one
 // before.  Loaded by each wave into registers instead, the slabs of nao above 36 spill (nao = 38, naux = 250,
-// nk = 27, 50 tau: 25 against 8.9 ms); below, 1.20 against 0.99 ms at nao = 18, 2.45 both ways at 26, 3.5
-// against 3.2 at 30.  The reductions have the registers, and are slower by 7 to 10 % from LDS.
+// nk = 27, 50 tau: 25 against 8.9 ms); below, 1.20 against 0.99 ms at nao = 18.  The reductions have the registers,
+// and are slower by 7 to 10 % from LDS.
 
 // Waves of a work-group for NB4 blocks: WS share the column blocks (two each), QW take different
 // quads.  Two waves per SIMD.
@@ -389,21 +390,29 @@ void z_prep_kernel(ZPrepArgs p) {
   }
 }
 
-// The same for nao of 41 to 48 on v_mfma_f64_16x16x4f64, three 16-wide blocks a side.  In column blocks those
-// sizes make six waves for four SIMDs, and G leaves no room for a second slab of V_Q: the kernel above waits.
-// Here each of four waves has a SIMD and its whole register file to itself, holds Z_Q and W, loads V_Q a slab
-// ahead and meets no barrier.  Bound: FP64 matrix cores (two thirds of their 16x16x4 rate) and the first slab.
+// The same on v_mfma_f64_16x16x4f64, NB 16-wide blocks a side, for the nao that fill them (z_prep16_blocks).  Each of
+// four waves takes a Q of its own, holds Z_Q and W in registers, loads V_Q a slab ahead and meets no barrier; two waves
+// per SIMD, at NB = 3 one with the whole register file.  In column blocks (the kernel above) a quad's digits and the
+// slabs of V_Q leave room for one work-group on a CU from nao = 25 on, with two spin blocks or at nao = 31 and 32 of one
+// or two waves per SIMD, and twelve blocks make six waves for four SIMDs.
+// Bound: FP64 matrix cores (two thirds of their 16x16x4 rate at nao = 48) and the first slab of a Q.
 // Register r of a 16x16 result holds row lane/16 + 4 r, column lane%16: the operand layout of the next product.
-// Per launch (nk = 8, naux = 300, 50 tau), and in column blocks: FP64 4.2 ms at nao 41 (5.5), 4.7 at 48 (5.8); four
-// slices 4.5 (6.5) and 4.8 (7.0); two spin blocks at nao 44 7.7 (10.5), four at nk = 4, nao 41 6.2 (7.9).
-// LDS: SB spin blocks of Gb and Gq as zero-padded planes [48][49].  A work-group takes 4 qpb consecutive Q.
-constexpr int ZP16_N = 48, ZP16_LD = ZP16_N + 1, ZP16_PL = ZP16_N * ZP16_LD;
-inline size_t z_prep16_lds_bytes(int sb) { return (size_t)sb * 4 * ZP16_PL * sizeof(double); }
-constexpr bool z_prep16_takes(int64_t nao) { return nao > 40 && nao <= ZP16_N; }
+// LDS: SB spin blocks of Gb and Gq as zero-padded planes [16 NB][16 NB + 1].  A work-group takes 4 qpb consecutive Q.
+inline size_t z_prep16_lds_bytes(int nb, int sb) { return (size_t)sb * 4 * 16 * nb * (16 * nb + 1) * sizeof(double); }
+// 16-wide blocks where they are the faster ones, else 0.  Per launch, 16-wide and in column blocks, nk = 27, naux =
+// 8 nao, 50 tau, four slices: nao 12 0.19 and 0.17 ms, 13 0.24 and 0.31, 16 0.27 and 0.37, 17 1.2 and 0.75, 24 1.86
+// and 1.91 (two spin blocks 3.3 and 3.1), 25 2.3 and 2.6, 32 3.3 and 6.0 (5.7 and 10.2); FP64 24 1.65 and 1.19, 26 2.07
+// and 2.14, 32 3.1 and 3.5.  nk = 8, naux = 300: nao 41 4.5 and 6.5, 48 4.8 and 7.0.  Four spin blocks at nao 14: an
+// evaluation of 9.2 and 9.0 ms.
+constexpr int z_prep16_blocks(int64_t nao, int64_t pseudo_ns) {
+  if (nao > 12 && nao <= 16 && pseudo_ns <= 2) return 1;
+  if (nao > 24 && nao <= 32) return 2;
+  return nao > 40 && nao <= 48 ? 3 : 0;
+}
 
-template <int NS, int SB>
-__global__ __launch_bounds__(256, 1) void z_prep16_kernel(ZPrepArgs p) {
-  constexpr int NB = 3, LD = ZP16_LD, PL = ZP16_PL;
+template <int NB, int NS, int SB>
+__global__ __launch_bounds__(256, NB < 3 ? 2 : 1) void z_prep16_kernel(ZPrepArgs p) {
+  constexpr int N16 = 16 * NB, LD = N16 + 1, PL = N16 * LD;
   extern __shared__ double zp16_lds[];  // [SB][Gb re | Gb im | Gq re | Gq im]
   const DevDims& d = p.d;
   const int nao = d.nao, nao2 = nao * nao;
@@ -419,8 +428,8 @@ __global__ __launch_bounds__(256, 1) void z_prep16_kernel(ZPrepArgs p) {
     const double2* Gbar = p.G + g_index(d, tt, is, k);
     const double2* Gk = p.G + g_index(d, tau, is, kq);
     double* g = zp16_lds + (size_t)s * 4 * PL;
-    for (int e = tid; e < ZP16_N * ZP16_N; e += 256) {
-      const int r = e / ZP16_N, c = e - (e / ZP16_N) * ZP16_N;
+    for (int e = tid; e < N16 * N16; e += 256) {
+      const int r = e / N16, c = e - (e / N16) * N16;
       double2 vb = make_double2(0.0, 0.0), vq = make_double2(0.0, 0.0);
       if (r < nao && c < nao) {
         vb = Gbar[(int64_t)(b * nao + r) * d.nso + a * nao + c];  // Gb[t = r][p = c]

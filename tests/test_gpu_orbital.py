@@ -60,9 +60,14 @@ def test_spin_blocks(case):
     _check(*_system(2, case["nao"], 5, ns=case.get("ns", 1), nso=case.get("nso")))
 
 
-@pytest.mark.parametrize("case", [dict(nao=41), dict(nao=48), dict(nao=45, ns=2), dict(nao=44, nso=88), dict(nao=48, nso=96)])
-def test_three_wide_blocks(case):
-    """nao of 41 to 48, more auxiliary indices than a work-group of the P0 prep takes, and several q per launch."""
+@pytest.mark.parametrize("case", [
+    dict(nao=12), dict(nao=13), dict(nao=16), dict(nao=17), dict(nao=16, ns=2), dict(nao=14, nso=28), dict(nao=24),
+    dict(nao=25), dict(nao=32), dict(nao=33), dict(nao=31, ns=2), dict(nao=26, nso=52), dict(nao=41), dict(nao=48),
+    dict(nao=45, ns=2), dict(nao=44, nso=88), dict(nao=48, nso=96),
+])
+def test_wide_blocks(case):
+    """The P0 operand on 16-wide blocks at the edges of its sizes, with more auxiliary indices than a work-group takes
+    and several q per launch."""
     _check(*_system(2, case["nao"], 19, ns=case.get("ns", 1), nso=case.get("nso")))
 
 

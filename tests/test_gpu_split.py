@@ -324,10 +324,10 @@ def test_int8_defaults_survive_other_tuning():
 
 @pytest.mark.parametrize("slices", [3, 4, 5])
 @pytest.mark.parametrize("spins", [1, 2])
-@pytest.mark.parametrize("nao", [41, 47, 48])
-def test_fused_slicing_of_three_blocks(nao, spins, slices):
-    """nao of 41 to 48, with a last work-group that is not full: the fused kernel, also with both spin blocks, against
-    the separate pass (the same sums with one spin block, hence the same bits; with two they are added in another
+@pytest.mark.parametrize("nao", [13, 16, 25, 31, 32, 41, 47, 48])
+def test_fused_slicing_of_wide_blocks(nao, spins, slices):
+    """The sizes of one, two and three 16-wide blocks, with a last work-group that is not full: the fused kernel, also
+    with both spin blocks, against the separate pass (the same sums with one spin block, hence the same bits; with two they are added in another
     order, up to the last digit's rounding) and against the oracle."""
     G, V, T, d = synthetic(2, nao, 21, ns=spins, beta=20.0, lam=1e3, mesh=(2, 1, 1), seed=29, sigma=0.5 / nao)
     out = []
