@@ -58,8 +58,11 @@ EPI_KERNEL = {1: "sigma_epi4_kernel<7> (Sigma += (V G) R, FP64 4x4x4 MFMA)",
 
 def kernel_labels(split, w, slices, tuning):
     """The kernel that each family launches for the workload (nao <= 40) with these parameters."""
-    nb4 = -(-w["nao"] // 4)
+    nao, nb4 = w["nao"], -(-w["nao"] // 4)
     prep = slices if split and tuning["p0_fused_slices"] else 0
+    wide = 1 if 12 < nao <= 16 else 2 if 24 < nao <= 32 else 0  # 16-wide blocks of the P0 operand
+    prep = f"z_prep16_kernel<{wide}, {prep}, {w['ns']}> (Z = Gb V Gq, FP64 16x16x4 MFMA)" if wide else \
+        f"z_prep_kernel<{nb4}, {prep}> (Z = Gb V Gq, FP64 4x4x4 MFMA)"
     if split:
         one = "true" if tuning["p0_kchunks"] == 1 else "false"  # k chunks of a launch
         sigma = f"{OZAKI_KERNEL[tuning['sigma_split_tile']]}<{slices}, true> (R = P-tilde conj(V), int8 slices)"
@@ -72,7 +75,7 @@ def kernel_labels(split, w, slices, tuning):
         p0 = f64[tuning["p0_tile"]] + " (P0 = Z conj(V)^T, FP64 MFMA)"
     return {"Sigma GEMM": sigma, "P0 GEMM": p0,
             "Sigma epilogue": f"sigma_epi_kernel<{nb4}> (Sigma += (V G) R, FP64 4x4x4 MFMA)",
-            "P0 prep": f"z_prep_kernel<{nb4}, {prep}> (Z = Gb V Gq, FP64 4x4x4 MFMA)"}
+            "P0 prep": prep}
 
 
 def upper_tiles(n, bm, bn):

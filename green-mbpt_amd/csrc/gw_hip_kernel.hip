@@ -433,7 +433,7 @@ void gw_hip_kernel::ensure_slices() {
 
 // tune_ with the keys that are left to the sizes filled in.  Row-tile group of the Sigma product: 256 rows of A
 // whichever the tile (64 x 64, nk = 27, nao = 26, naux = 250: 57.6 ms an evaluation with four row tiles, 65.8 with
-// eight, 69.4 with sixteen).
+// eight, 69.4 with sixteen; within 3 % of the best of two to sixteen at nk 2 to 64, nao 8 to 60, naux 60 to 400).
 Tuning gw_hip_kernel::tuning() const {
   Tuning t = tune_;
   if (!t.p0_oz_tile) t.p0_oz_tile = ozaki_default_tile(split_ns_, d_.nk, ceil_div(d_.nao * d_.nao, 64) * 64);
@@ -553,7 +553,7 @@ void launch_orb(K kern, A& args, dim3 grid, int threads, size_t lds, hipStream_t
   hipLaunchKernelGGL(kern, xcd_launch_grid(args.xg), dim3(threads), lds, st, args);
   GWHIP_CHECK(hipGetLastError());
 }
-// Spin blocks of G that fit the LDS of one work-group (at most 150 KB)
+// Spin blocks of G that fit the LDS of one work-group with z_prep_kernel's slabs
 int prep_spin_blocks(int nb4, int pseudo_ns) {
   int sb = pseudo_ns;
   while (sb > 1 && !z_prep_fits(nb4, sb, 0, 0)) sb /= 2;
@@ -1133,7 +1133,7 @@ void gw_hip_kernel::gather_mats(const double2* base, const int* map, int64_t n) 
 // The P0 orbital product as two batched FP64 GEMMs over k per (tau, spin block), for any nao:
 //   W[k][Q][p][n] = sum_m V(k, k+q)_Q[p][m] Gq(k)[m][n],     Gq = G(tau, is, k + q) block (a, b)
 //   Z[k][Q][t][n] (+)= sum_p Gb(k)[t][p] W[k][Q][p][n],      Gb = G(beta - tau, is, k) block (b, a)
-// (the same Z_Q = Gb V_Q Gq as z_prep_mfma_kernel, src/gw_cpu_kernel.cpp:200-215).
+// (the same Z_Q = Gb V_Q Gq as z_prep_kernel, src/gw_cpu_kernel.cpp:200-215).
 void gw_hip_kernel::p0_prep_gemm(int64_t q, const double2* G, int64_t t0, int64_t tc) {
   const int64_t nk = d_.nk, NQ = d_.NQ, nao = d_.nao, nao2 = nao * nao, nso = d_.nso, nso2 = nso * nso;
   const int64_t vq = NQ * nao2;
@@ -1167,7 +1167,7 @@ void gw_hip_kernel::p0_prep_gemm(int64_t q, const double2* G, int64_t t0, int64_
 // any nao; R(tz) in scratch_ [tz][nkb][Q][n][j] serves tau = t0 + tz and beta - tau:
 //   XT[k][Q][n][i] = sum_m G(k)[m][n] V_Q[i][m],   G = G(tau, is, km[k]) block (a, b), i.e. X = V_Q G
 //   Sigma(tau, is, k)[a,b](i, j) += scale sum_{Q, n} X[i][Q, n] R[k][Q][n][j]
-// (sigma_epi_mfma_kernel's products, src/gw_cpu_kernel.cpp:359-373).
+// (sigma_epi_kernel's products, src/gw_cpu_kernel.cpp:359-373).
 void gw_hip_kernel::sigma_epi_gemm(const double2* G, double2* Sigma, const SigmaRows& r, int64_t t0, int64_t tc,
                                    double scale) {
   const int64_t NQ = d_.NQ, nao = d_.nao, nao2 = nao * nao, nso = d_.nso, nso2 = nso * nso, vq = NQ * nao2, nkb = r.n;
@@ -1331,10 +1331,11 @@ void gw_hip_kernel::autotune(const double2* G, int precision) {
   const int qpws[4] = {1, 2, 4, 8};
   tune_.qpw = best_of(4, qpws, [&](int c) { p0_prep(0, G, 0, tcp, c); });
   if (!split) {
-    const int shapes[3] = {0, 1, 2};
+    const int shapes[3] = {0, 2, 1};
     p0_prep(0, G, 0, tcp, tune_.qpw);
     tune_.p0_shape = best_of(3, shapes, [&](int c) { p0_gemm(0, tcp, P_, c); });
-    tune_.s_shape = best_of(3, shapes, [&](int c) { sigma_gemm(P_, sigma_rows(d_.nk - 1), tcs, c); });
+    // the half product has no 128-row tile (sigma_gemm)
+    tune_.s_shape = best_of(sigma_half(false) ? 2 : 3, shapes, [&](int c) { sigma_gemm(P_, sigma_rows(d_.nk - 1), tcs, c); });
   } else {
     if (fused_p0()) {  // fused prep + slicing vs the two kernels
       const int fz[2] = {0, 1};

@@ -350,9 +350,9 @@ private:
   // The exchange of nao 41 to 48 as one work-group of four waves per pair on 16x16x4 products (launch_reduce), or
   // as six single waves per pair (hf_exchange_kernel).  A wave of either has a SIMD to itself, and a round of the
   // first takes 1.5 times a round of the second (2.05 against 1.33 ms at nao = 44, naux = 200), so the one with the
-  // fewer rounds so weighted: nk = 14, 16, 27, 48 the first, others to 64 the second.  nao = 44, first and second:
-  // nk = 27, naux = 200 6.2 and 6.7 ms; nk = 16, naux = 300 3.2 and 4.2; nk = 18 4.1 and 2.8; nk = 36, naux = 150
-  // 9.3 and 8.2.
+  // fewer rounds so weighted: nk = 14 to 16, 27, 35, 42, 48, 53 and 57 the first, others to 64 the second.  nao = 44,
+  // first and second: nk = 27, naux = 200 6.2 and 6.7 ms; nk = 16, naux = 300 3.2 and 4.2; nk = 18 4.1 and 2.8;
+  // nk = 36, naux = 150 9.3 and 8.2.
   bool hf_16() const {
     const int64_t pairs = d_.nk * d_.nk;
     return d_.nao > 40 && 3 * ceil_div(pairs, 256) < 2 * ceil_div(6 * pairs, 1024);
@@ -363,7 +363,7 @@ private:
   void gather_g(const double2* G, int64_t tau, int64_t is, const int* map, int64_t n);
   void gather_mats(const double2* base, const int* map, int64_t n);
   void hf_exchange_gemm(const double2* dm_s, int nblk);
-  // the VJP's orbital products: register-chained kernels, or batched GEMMs (orb_gemm())
+  // the VJP's orbital products: register-chained kernels, or batched GEMMs (vjp_gemm())
   void vjp_sandwich(bool has_l, bool has_r, int NB, dim3 grid, const OrbArgs& a, const OrbOp& L, const OrbOp& V,
                     const OrbOp& R, const OrbOut& X);
   void vjp_reduce(bool has_m, int NB, dim3 grid, const OrbArgs& a, const OrbOp& A, const OrbOp& M, const OrbOp& C,

@@ -135,8 +135,7 @@ struct OrbCfg {
 //   Z[t][n] = sum_p Gb[t][p] W[p][n]       A = Gb (the same), B = W
 // grid: (ceil(NQ / (4 QPB)), rows, tcount), QPB quads per work-group.  LDS: SB spin blocks of Gb
 // (transposed) and Gq, zero-padded [N4][N4]; a launch covers the spin blocks s0 .. s0 + SB and adds to Z
-// when s0 > 0.  V_Q is streamed once per wave and spin block (the waves of a work-group and the tau
-// neighbours find it in L1 and L2).
+// when s0 > 0.  V_Q is brought to LDS once per work-group and spin block (the tau neighbours find it in L2).
 // NS = 0: Z in FP64.  NS > 0: straight into the NS int8 slices of the split-precision contraction, with
 // the arithmetic of slice_rows_kernel: the work-group that forms Z_Q(tau, k) owns the whole slice
 // row-chunk (row (tau, Q), chunk k, nao^2 elements), so the chunk exponent is a maximum over its lanes

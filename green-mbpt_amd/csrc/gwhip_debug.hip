@@ -256,7 +256,6 @@ double debug_gemm_bench(int which, int NQ, int nk, int nao, int batch, int shape
   const int64_t nao2 = (int64_t)nao * nao, NQ2 = (int64_t)NQ * NQ, vsz = (int64_t)nk * NQ * nao2;
   ZGemmArgs a{};
   int64_t na, nb, nc;
-  bool akc = true, bkc = false;
   if (which == 0) {  // Sigma: R[tau] = P[tau] conj(V)
     na = batch * NQ2; nb = vsz; nc = batch * vsz;
     a.M = NQ; a.N = (int)(nk * nao2); a.K = NQ; a.batch = batch; a.kin = NQ; a.nin = (int)nao2;
@@ -269,7 +268,6 @@ double debug_gemm_bench(int which, int NQ, int nk, int nao, int batch, int shape
     a.sAb = vsz; a.sAm = nao2; a.sAko = NQ * nao2; a.sAki = 1;
     a.sBb = 0; a.sBko = NQ * nao2; a.sBki = 1; a.sBno = 0; a.sBni = nao2;
     a.sCb = NQ2; a.sCm = NQ; a.sCno = 0; a.sCni = 1;
-    bkc = true;
   }
   double2 *dA = nullptr, *dB = nullptr, *dC = nullptr;
   GWHIP_CHECK(hipMalloc(&dA, na * sizeof(double2)));

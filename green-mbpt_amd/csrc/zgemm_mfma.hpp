@@ -1,4 +1,4 @@
-// Complex FP64 GEMM on CDNA4 matrix cores (v_mfma_f64_16x16x4f64).
+// Complex FP64 GEMM on CDNA4 matrix cores (v_mfma_f64_4x4x4_4b).
 //
 // C[b](m, n) (+)= alpha * sum_k opA(A[b](m, k)) * opB(B[b](k, n))
 //

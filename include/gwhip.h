@@ -147,7 +147,7 @@ int gwhip_eval_sigma_device(gwhip_handle* h, const void* G_dev, void* Sigma_dev,
  * grid and V (gwhip_set_grid, gwhip_upload_V / gwhip_generate_V) and, for the split modes, V's int8
  * slice stores, which the first gwhip_eval_sigma_device or gwhip_autotune in a split mode builds.
  * GWHIP_ERR_UNSUPPORTED when one tau point and one q do not fit the workspace (nk = 64, nao = 26,
- * naux = 300 needs about 0.64 GB in FP64 and does not), for nao > 48 (the orbital GEMM form) and
+ * naux = 300 needs about 0.64 GB in FP64 and does not), for nao > 48, for the orbital GEMM form and
  * with the q -> 0 correction on.  Results are bit-identical to gwhip_eval_sigma_device.  All calls on one
  * GPU share its array: calls that overlap on one GPU (several host threads, several handles) race
  * and must be serialised by the caller.
