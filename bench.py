@@ -33,11 +33,11 @@ WORKLOAD = dict(nk=64, mesh=(4, 4, 4), nao=26, NQ=300, ns=1, beta=100.0, lam=1e4
 # the bytes the copy reads, WRITE_SIZE 1.0x the bytes it writes.
 # Source: profiles/gw_sigma_nk64_nao26_naux300_hbm_traffic.md
 PMC_PER_LAUNCH_KIB = {
-    "split": {"Sigma GEMM": (3.5562e6, 1.0177e7), "Sigma epilogue": (1.0584e7, 3.8872e4),
-              "P0 GEMM": (1.1288e7, 1.2693e6), "P0 prep": (6.9734e5, 5.3100e6),  # P0 GEMM with its partial sums
+    "split": {"Sigma GEMM": (3.5764e6, 1.0179e7), "Sigma epilogue": (1.0594e7, 3.8867e4),
+              "P0 GEMM": (1.1323e7, 1.2693e6), "P0 prep": (6.7506e5, 5.3391e6),  # P0 GEMM with its partial sums
               "Dyson inverse": (5.3400e7, 6.7701e7)},  # every kernel of the inverse, one evaluation
-    "fp64": {"Sigma GEMM": (1.5028e7, 1.0210e7), "Sigma epilogue": (1.0703e7, 6.8068e4),
-             "P0 GEMM": (1.7954e7, 4.2527e4), "P0 prep": (7.4748e5, 1.0187e7),
+    "fp64": {"Sigma GEMM": (1.5028e7, 1.0210e7), "Sigma epilogue": (1.0692e7, 6.8110e4),
+             "P0 GEMM": (1.7864e7, 4.2532e4), "P0 prep": (7.5572e5, 1.0162e7),
              "Dyson inverse": (5.3410e7, 6.7695e7)},
 }
 PMC_CALIBRATION = (0.5, 1.0)
